@@ -24,6 +24,7 @@
 
 #include "vrt_g3_errors.hpp"
 #include "vrt_g3_internal.hpp"
+#include "vrt_gemm.hpp"
 #include "vrt_internal.hpp"
 #include "vrt_q8_device.hpp"
 
@@ -51,8 +52,7 @@ struct BdAttn {
     const float* sin_t;
     float eps, attn_scale;
     float* part;              // [n][G][2 H + H hd]: m and l per head, then acc per head
-    _Float16* ohi;            // [n][H hd] attention output, f16 high part
-    _Float16* olo;            //   ... and low part
+    _Float16* o;              // attention output, an activation buffer of H hd columns
     G3State* st;
     uint32_t block;
 };
@@ -365,10 +365,8 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
         const double den = static_cast<double>(static_cast<float>(s_l));
         if (tid == 0u && (!(den > 0.0) || !__builtin_isfinite(den))) atomicMin(&A.st->nonfinite, g3_code_softmax(A.block));
         const float v = static_cast<float>(static_cast<double>(acc) / den);
-        const uint64_t o = static_cast<uint64_t>(b) * H * hd + h * hd + tid;
-        const _Float16 hi = static_cast<_Float16>(v);
-        A.ohi[o] = hi;
-        A.olo[o] = static_cast<_Float16>(v - static_cast<float>(hi));
+        const uint64_t o = gm_off(b, h * hd + tid, H * hd / 32u);
+        gm_split(v, A.o[o], A.o[o + kGmLo]);
     }
 }
 
@@ -403,10 +401,8 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_merge(BdAttn A) {
         double num = 0.0;
         for (uint32_t c = 0; c < n_act; ++c) num += s_w[c] * static_cast<double>(part[c * stride + 2u * H + h * hd + i]);
         const float v = static_cast<float>(num / den);
-        const uint64_t o = static_cast<uint64_t>(b) * H * hd + h * hd + i;
-        const _Float16 hi = static_cast<_Float16>(v);
-        A.ohi[o] = hi;
-        A.olo[o] = static_cast<_Float16>(v - static_cast<float>(hi));
+        const uint64_t o = gm_off(b, h * hd + i, H * hd / 32u);
+        gm_split(v, A.o[o], A.o[o + kGmLo]);
     }
 }
 
@@ -502,10 +498,8 @@ struct vrt_g3_batch {
     float* h = nullptr;             // [rows][d] residual stream
     float* x = nullptr;             // [kBdMaxSplits][rows][d] O / down projection partials
     float* qkv = nullptr;           // [kBdMaxSplits][rows][(H + 2) hd] q|k|v partials
-    _Float16* ahi = nullptr;        // [rows][max(d, H hd)] GEMM input, f16 high part
-    _Float16* alo = nullptr;
-    _Float16* ghi = nullptr;        // [rows][F] gelu(gate) * up, f16 high part
-    _Float16* glo = nullptr;
+    _Float16* a = nullptr;          // activation buffer of max(d, H hd) columns: GEMM input
+    _Float16* gg = nullptr;         // activation buffer of F columns: gelu(gate) * up
     float* part = nullptr;          // [rows][max G][2 H + H hd] attention chunk partials
     float* logits = nullptr;        // [rows][V]
     LmPartial* amx = nullptr;       // [rows][kBdArgParts]
@@ -588,15 +582,10 @@ extern "C" int vrt_g3_batch_create(vrt_g3* g, uint32_t max_seqs, uint32_t max_ct
     B->x = static_cast<float*>(p);
     if (int rc = bd_alloc(B, kBdMaxSplits * R * nqkv * 4u, &p)) return fail(rc);
     B->qkv = static_cast<float*>(p);
-    const size_t aw = std::max(d, qw);
-    if (int rc = bd_alloc(B, R * aw * 2u, &p)) return fail(rc);
-    B->ahi = static_cast<_Float16*>(p);
-    if (int rc = bd_alloc(B, R * aw * 2u, &p)) return fail(rc);
-    B->alo = static_cast<_Float16*>(p);
-    if (int rc = bd_alloc(B, R * F * 2u, &p)) return fail(rc);
-    B->ghi = static_cast<_Float16*>(p);
-    if (int rc = bd_alloc(B, R * F * 2u, &p)) return fail(rc);
-    B->glo = static_cast<_Float16*>(p);
+    if (int rc = bd_alloc(B, gm_size(R, std::max(d, qw)) * 2u, &p)) return fail(rc);
+    B->a = static_cast<_Float16*>(p);
+    if (int rc = bd_alloc(B, gm_size(R, F) * 2u, &p)) return fail(rc);
+    B->gg = static_cast<_Float16*>(p);
     if (int rc = bd_alloc(B, R * gmax * (2u * H + qw) * 4u, &p)) return fail(rc);
     B->part = static_cast<float*>(p);
     if (int rc = bd_alloc(B, R * c.vocab_size * 4u, &p)) return fail(rc);
@@ -655,11 +644,10 @@ static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
         const BdLayer& BL = B->layers[l];
         // previous block's FFN output into the residual, then the attention norm
         if (int rc = pf_norm(B->h, l ? B->x : nullptr, s_down, xs, l ? g->layers[l - 1].post_ffw : nullptr, Ly.attn_norm,
-                             d, eps, B->ahi, B->alo, B->st, l ? l - 1u : 0u, n, s, true))
+                             d, eps, B->a, B->st, l ? l - 1u : 0u, n, s, true))
             return rc;
         uint32_t s_qkv = 1;
-        if (int rc = pf_project(g, l, kProjQkv, B->ahi, B->alo, n, B->qkv,
-                                std::min(kBdMaxSplits, pf_splits(n, nqkv)), &s_qkv, s))
+        if (int rc = pf_project(g, l, kProjQkv, B->a, n, B->qkv, &s_qkv, s))
             return rc;
         BdAttn A{};
         A.qkv = B->qkv;
@@ -681,8 +669,7 @@ static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
         A.eps = eps;
         A.attn_scale = g->P.attn_scale;
         A.part = B->part;
-        A.ohi = B->ahi;
-        A.olo = B->alo;
+        A.o = B->a;
         A.st = B->st;
         A.block = l;
         {
@@ -701,20 +688,19 @@ static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
             }
         }
         uint32_t s_o = 1;
-        if (int rc = pf_project(g, l, kProjO, B->ahi, B->alo, n, B->x, std::min(kBdMaxSplits, pf_splits(n, d)), &s_o, s))
+        if (int rc = pf_project(g, l, kProjO, B->a, n, B->x, &s_o, s))
             return rc;
-        if (int rc = pf_norm(B->h, B->x, s_o, xs, Ly.post_attn, Ly.ffn_norm, d, eps, B->ahi, B->alo, B->st, l, n, s, true))
+        if (int rc = pf_norm(B->h, B->x, s_o, xs, Ly.post_attn, Ly.ffn_norm, d, eps, B->a, B->st, l, n, s, true))
             return rc;
-        if (int rc = pf_ffn_glu(g, l, B->ahi, B->alo, n, B->ghi, B->glo, s)) return rc;
-        if (int rc = pf_project(g, l, kProjDown, B->ghi, B->glo, n, B->x, std::min(kBdMaxSplits, pf_splits(n, d)),
-                                &s_down, s))
+        if (int rc = pf_ffn_glu(g, l, B->a, n, B->gg, s)) return rc;
+        if (int rc = pf_project(g, l, kProjDown, B->gg, n, B->x, &s_down, s))
             return rc;
     }
     // final residual (:1849-1855) and output norm (rms_norm_inplace, :1866-1868) as the LM input
-    if (int rc = pf_norm(B->h, B->x, s_down, xs, g->layers[L - 1u].post_ffw, g->out_norm_dev, d, eps, B->ahi, B->alo, B->st,
+    if (int rc = pf_norm(B->h, B->x, s_down, xs, g->layers[L - 1u].post_ffw, g->out_norm_dev, d, eps, B->a, B->st,
                          L - 1u, n, s, false))
         return rc;
-    if (int rc = pf_lm_logits(g, B->ahi, B->alo, n, B->logits, s)) return rc;
+    if (int rc = pf_lm_logits(g, B->a, n, B->logits, s)) return rc;
     {
         const float* lg = B->logits;
         uint32_t V = c.vocab_size;

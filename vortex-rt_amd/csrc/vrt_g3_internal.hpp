@@ -95,9 +95,9 @@ struct CoopSlot {
 constexpr int kMaxCoopDevices = 64;
 CoopSlot& coop_slot(int device);   // vrt_decode.hip
 
-// A block's weight matrices expanded once for the prefill GEMMs: the quants as f16 [N][K] and
-// the block scales as fp32 [N][K / 32]. qkv: the q, k, v rows concatenated; gu: the gate and up
-// rows interleaved in groups of 64 (32 gate rows, then the same 32 up rows).
+// A block's weight matrices expanded once for the row-batch GEMMs (the layout of vrt_gemm.hpp: the
+// quants as f16, the block scales as fp32). qkv: the q, k, v rows concatenated; gu: the gate and
+// up rows interleaved in groups of 32 (16 gate rows, then the same 16 up rows).
 struct PfMatrix {
     const void* h = nullptr;
     const float* s = nullptr;
@@ -111,9 +111,11 @@ struct PfState {
     uint32_t max_t = 0;     // prompt positions per call
     float* h = nullptr;     // [max_t][d] residual stream
     float* x = nullptr;     // [max_t][d] sublayer outputs (O projection, down projection)
-    void* ahi = nullptr;    // [max_t][max(d, H*hd, F)] GEMM input, f16 high part
-    void* alo = nullptr;    //   ... and low part
-    float* big = nullptr;   // [max_t][max(H*hd + 2*hd, 2F)] q|k|v rows, then gate|up rows
+    _Float16* a = nullptr;  // activation buffer (vrt_gemm.hpp) of max(d, H*hd) columns: normed rows, attention output
+    _Float16* g = nullptr;  // activation buffer of F columns: gelu(gate) * up
+    float* qkv = nullptr;   // [splits][max_t][H*hd + 2*hd] q|k|v rows
+    _Float16* qhi = nullptr;   // [max_t][H*hd] queries after QK-norm and RoPE, f16 high part
+    _Float16* qlo = nullptr;   //   ... and low part
     void* khi = nullptr;    // attention keys (tkv x hd), f16 high part: a segment's history, then its rows
     void* klo = nullptr;    //   ... and low part
     void* vhi = nullptr;    // attention values (Tp x hd), f16 high part
@@ -187,16 +189,12 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0 = 0, bool final = true);
 // block l's projections over M rows as (split-K) GEMMs, its gate/up product, the residual
 // norms over rows, embedding rows, and the logits of M rows against the tied embedding table.
 enum PfProj : uint32_t { kProjQkv = 0, kProjO = 1, kProjDown = 2 };
-int pf_project(vrt_g3* g, uint32_t l, uint32_t which, const _Float16* ahi, const _Float16* alo, uint32_t M, float* c,
-               uint32_t splits, uint32_t* used, hipStream_t s);
-int pf_ffn_glu(vrt_g3* g, uint32_t l, const _Float16* ahi, const _Float16* alo, uint32_t M, _Float16* ghi,
-               _Float16* glo, hipStream_t s);
+int pf_project(vrt_g3* g, uint32_t l, uint32_t which, const _Float16* a, uint32_t M, float* c, uint32_t* used, hipStream_t s);
+int pf_ffn_glu(vrt_g3* g, uint32_t l, const _Float16* a, uint32_t M, _Float16* o, hipStream_t s);
 int pf_norm(float* h, const float* f, uint32_t nsplit, uint64_t sstride, const float* w_post, const float* w_next,
-            uint32_t n, float eps, _Float16* xhi, _Float16* xlo, G3State* st, uint32_t block, uint32_t rows, hipStream_t s,
-            bool into);
+            uint32_t n, float eps, _Float16* x, G3State* st, uint32_t block, uint32_t rows, hipStream_t s, bool into);
 int pf_embed_rows(vrt_g3* g, const uint32_t* tokens, uint32_t rows, float* h, hipStream_t s);
-int pf_lm_logits(vrt_g3* g, const _Float16* xhi, const _Float16* xlo, uint32_t M, float* logits, hipStream_t s);
-uint32_t pf_splits(uint32_t M, uint32_t N);
+int pf_lm_logits(vrt_g3* g, const _Float16* x, uint32_t M, float* logits, hipStream_t s);
 // Final residual + output norm + LM head + argmax of the current step (vrt_gemma3.hip).
 int g3_enqueue_lm(vrt_g3* g, hipStream_t s);
 int mk_read_trace(vrt_g3* g, uint64_t* out, uint64_t cap, uint32_t* nwg, uint32_t* slots);

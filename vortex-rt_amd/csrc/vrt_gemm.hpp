@@ -1,0 +1,64 @@
+// vrt_gemm.hpp -- the row-batch projections of the prefill and the batched decode on MFMA
+// (vrt_gemm.hip): operand layouts and launches.
+//
+// Operand order. Both operands of v_mfma_f32_16x16x32_f16 hold 16 rows x 32 consecutive k: lane l
+// gives row l % 16, k = 8 (l / 16) + j, j < 8. Activations and weights are kept in memory as
+// such units, 512 halves each, in lane order, so a wave's operand load is one contiguous 1 KB, from
+// memory straight to registers or to LDS, and an LDS read of it is conflict-free without padding.
+//   activations [row tile of 16][K / 32][hi, lo][512]   (f16 high and low parts, A = hi + lo)
+//   weights     [row tile of 16][K / 32][512]           (the Q8_0 quants as f16, exact)
+//   scales      [K / 32][npad]                          (fp32), npad = N rounded up to 128
+// One unit of K is one Q8_0 block, so a block's scale multiplies whole MFMA results.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace vrt {
+
+constexpr uint32_t kGmRowPad = 128;   // rows of an activation buffer and of a weight matrix: whole tiles
+
+// Offset (halves) of element (row, k) of an activation buffer with nkb = K / 32: its high part;
+// the low part is kGmLo further.
+constexpr uint32_t kGmLo = 512;
+__host__ __device__ __forceinline__ uint64_t gm_off(uint32_t row, uint32_t k, uint32_t nkb) {
+    return (static_cast<uint64_t>(row >> 4) * nkb + (k >> 5)) * 1024u + ((k >> 3) & 3u) * 128u + (row & 15u) * 8u + (k & 7u);
+}
+// Halves of an activation buffer of `rows` rows (padded to whole tiles) and K columns.
+__host__ __device__ __forceinline__ uint64_t gm_size(uint64_t rows, uint32_t K) {
+    return (rows + kGmRowPad - 1u) / kGmRowPad * kGmRowPad * K * 2u;
+}
+
+// x = hi + lo. The product that x often is must be rounded to fp32 before it is rounded to f16: left to
+// itself the compiler rounds it to f16 in one step (v_fma_mixlo_f16) for the subtraction and in two
+// for the stored hi, and where the two differ (about one value in 2^13) the pair is one f16 ulp off.
+__device__ __forceinline__ void gm_split(float x, _Float16& hi, _Float16& lo) {
+    asm("" : "+v"(x));
+    hi = static_cast<_Float16>(x);
+    lo = static_cast<_Float16>(x - static_cast<float>(hi));
+}
+
+struct GmArgs {
+    const _Float16* a;     // activations, M rows
+    const _Float16* w;     // weights, N rows
+    const float* ws;       // their block scales [nkb][npad]
+    float* c;              // C [M][N] fp32 (row stride ldc), split z at c + z * c_bs; or, gate/up:
+    _Float16* o;           // gelu_tanh(gate) * up as an activation buffer of N / 2 columns
+    uint64_t c_bs;
+    uint32_t ldc;
+    uint32_t M, N, nkb, npad;
+};
+
+// C = A x W^T, or with glu (w: gate and up rows interleaved in groups of 16, 16 gate rows first)
+// gelu_tanh(gate) * up. gm_splits: the K splits that suit this shape (1: none);
+// the consumer adds the partials in split order.
+uint32_t gm_splits(uint32_t M, uint32_t N, uint32_t nkb);
+int gm_run(const GmArgs& G, uint32_t splits, bool glu, hipStream_t s);
+// One-time expansion of Q8_0 rows into a weight matrix: up to three matrices concatenated
+// (rows0, rows1, the rest), or with glu the gate (w0) and up (w1) rows interleaved. Rows N..npad-1
+// are zero with scale 0.
+int gm_expand(const uint8_t* w0, const uint8_t* w1, const uint8_t* w2, uint32_t rows0, uint32_t rows1, uint32_t N,
+              uint32_t nkb, bool glu, _Float16* wh, float* ws, hipStream_t s);
+
+}  // namespace vrt

@@ -19,6 +19,7 @@
 
 #include "vrt_g3_errors.hpp"
 #include "vrt_g3_internal.hpp"
+#include "vrt_gemm.hpp"
 #include "vrt_q8_device.hpp"
 
 namespace vrt {
@@ -36,9 +37,10 @@ constexpr uint32_t kPfTile = 64;     // attention score rows are padded to a mul
 // ---- row kernels ---------------------------------------------------------------------------
 
 __device__ __forceinline__ void pf_split(float x, _Float16* hi, _Float16* lo) {
-    const _Float16 h = static_cast<_Float16>(x);
+    _Float16 h, l;
+    gm_split(x, h, l);
     *hi = h;
-    *lo = static_cast<_Float16>(x - static_cast<float>(h));
+    *lo = l;
 }
 
 // pf_split of four consecutive values (8-byte aligned destinations).
@@ -47,8 +49,10 @@ __device__ __forceinline__ void pf_split4(f4 x, _Float16* hi, _Float16* lo) {
     half4 h, l;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        h[k] = static_cast<_Float16>(x[k]);
-        l[k] = static_cast<_Float16>(x[k] - static_cast<float>(h[k]));
+        _Float16 a, b;
+        gm_split(x[k], a, b);
+        h[k] = a;
+        l[k] = b;
     }
     *reinterpret_cast<half4*>(hi) = h;
     *reinterpret_cast<half4*>(lo) = l;
@@ -73,19 +77,19 @@ __global__ void __launch_bounds__(kPfThreads) k_pf_embed(const uint8_t* tok_embd
     }
 }
 
-// One wave per row t (four rows per workgroup, `rows` rows in all; n <= 64 NE elements, NE per
-// lane; the sums are wave reductions, with no barrier). With f (the previous sublayer's output,
-// the sum of nsplit partial rows f + s * sstride added in order s = 0, 1, ...):
-// h = f * (scale(f) * w_post) + h (rms_norm_inplace then add_inplace, src/gemma3.cpp:1036-1042,
-// :1703-1711, :1849-1855). Then, with w_next:
-// the GEMM input (h * scale(h)) * w_next as f16 hi/lo (rms_norm_into, :991-996), or with
+// One wave per row t (four rows per workgroup, `rows` rows in all; n <= 256 NQ elements, a multiple
+// of 32; lane l owns the runs of four from 4 l + 256 k; the sums are wave reductions, with no
+// barrier). With f (the previous sublayer's output, the sum of nsplit partial rows f + s * sstride
+// added in order s = 0, 1, ...): h = f * (scale(f) * w_post) + h (rms_norm_inplace then
+// add_inplace, src/gemma3.cpp:1036-1042, :1703-1711, :1849-1855). Then, with w_next: the GEMM
+// input (h * scale(h)) * w_next into the activation buffer x (rms_norm_into, :991-996), or with
 // `into` 0 h * (scale(h) * w_next) (rms_norm_inplace, the output norm :1866-1868). nonfinite:
 // lowest block whose residual went non-finite (:1857-1863), reported through st->nonfinite.
-template <uint32_t NE>
+template <uint32_t NQ>
 __global__ void __launch_bounds__(kPfThreads) k_pf_norm_w(float* h, const float* f, uint32_t nsplit, uint64_t sstride,
                                                           const float* w_post, const float* w_next, uint32_t n, float eps,
-                                                          _Float16* xhi, _Float16* xlo, G3State* st, uint32_t block,
-                                                          uint32_t rows, uint32_t into) {
+                                                          _Float16* x, G3State* st, uint32_t block, uint32_t rows,
+                                                          uint32_t into) {
 #pragma clang fp contract(off)
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t t = blockIdx.x * (kPfThreads / 64u) + (threadIdx.x >> 6);
@@ -93,49 +97,62 @@ __global__ void __launch_bounds__(kPfThreads) k_pf_norm_w(float* h, const float*
     float* hr = h + static_cast<uint64_t>(t) * n;
     // Every load is issued at a clamped, in-bounds index and masked afterwards, so the loads of
     // a row are in flight together (no branch, hence no wait, between them).
-    uint32_t ic[NE];
-    bool live[NE];
+    uint32_t ic[NQ];
+    bool live[NQ];
 #pragma unroll
-    for (uint32_t k = 0; k < NE; ++k) {
-        live[k] = lane + 64u * k < n;
-        ic[k] = min(lane + 64u * k, n - 1u);
+    for (uint32_t k = 0; k < NQ; ++k) {
+        live[k] = 4u * lane + 256u * k < n;
+        ic[k] = min(4u * lane + 256u * k, n - 4u);
     }
-    float hv[NE], wp[NE], wn[NE];
+    f4 hv[NQ], wp[NQ], wn[NQ];
 #pragma unroll
-    for (uint32_t k = 0; k < NE; ++k) {
-        hv[k] = hr[ic[k]];
-        wp[k] = w_post ? w_post[ic[k]] : 0.0f;
-        wn[k] = w_next ? w_next[ic[k]] : 0.0f;
+    for (uint32_t k = 0; k < NQ; ++k) {
+        hv[k] = *reinterpret_cast<const f4*>(hr + ic[k]);
+        wp[k] = w_post ? *reinterpret_cast<const f4*>(w_post + ic[k]) : f4{0.0f, 0.0f, 0.0f, 0.0f};
+        wn[k] = w_next ? *reinterpret_cast<const f4*>(w_next + ic[k]) : f4{0.0f, 0.0f, 0.0f, 0.0f};
     }
     if (f) {
         const float* fr = f + static_cast<uint64_t>(t) * n;
-        // every partial is loaded before the first add, then the partials are added in split order
-        float fp[NE][kPfMaxSplits];
+        f4 fv[NQ];
+        if (nsplit == 1u) {
 #pragma unroll
-        for (uint32_t q = 0; q < kPfMaxSplits; ++q) {
-            const float* fq = fr + min(q, nsplit - 1u) * sstride;
+            for (uint32_t k = 0; k < NQ; ++k) fv[k] = *reinterpret_cast<const f4*>(fr + ic[k]);
+        } else {   // every partial is loaded before the first add, then the partials are added in split order
+            f4 fp[NQ][kPfMaxSplits];
 #pragma unroll
-            for (uint32_t k = 0; k < NE; ++k) fp[k][q] = fq[ic[k]];
+            for (uint32_t q = 0; q < kPfMaxSplits; ++q) {
+                const float* fq = fr + min(q, nsplit - 1u) * sstride;
+#pragma unroll
+                for (uint32_t k = 0; k < NQ; ++k) fp[k][q] = *reinterpret_cast<const f4*>(fq + ic[k]);
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < NQ; ++k) {
+                fv[k] = fp[k][0];
+#pragma unroll
+                for (uint32_t q = 1; q < kPfMaxSplits; ++q)
+                    if (q < nsplit)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) fv[k][e] += fp[k][q][e];
+            }
         }
-        float fv[NE];
         double ss = 0.0;
 #pragma unroll
-        for (uint32_t k = 0; k < NE; ++k) {
-            fv[k] = 0.0f;
+        for (uint32_t k = 0; k < NQ; ++k)
 #pragma unroll
-            for (uint32_t q = 0; q < kPfMaxSplits; ++q)
-                if (q < nsplit) fv[k] += fp[k][q];
-            if (!live[k]) fv[k] = 0.0f;
-            ss += static_cast<double>(fv[k]) * static_cast<double>(fv[k]);
-        }
+            for (int e = 0; e < 4; ++e) {
+                if (!live[k]) fv[k][e] = 0.0f;
+                ss += static_cast<double>(fv[k][e]) * static_cast<double>(fv[k][e]);
+            }
         const float sc = pf_rms_scale(wave_red_sum_d(ss), n, eps);
         int bad = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < NE; ++k) {
-            hv[k] = fv[k] * (sc * wp[k]) + hv[k];
+        for (uint32_t k = 0; k < NQ; ++k) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) hv[k][e] = fv[k][e] * (sc * wp[k][e]) + hv[k][e];
             if (live[k]) {
-                hr[ic[k]] = hv[k];
-                bad |= !__builtin_isfinite(hv[k]);
+                *reinterpret_cast<f4*>(hr + ic[k]) = hv[k];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bad |= !__builtin_isfinite(hv[k][e]);
             }
         }
         if (bad) atomicMin(&st->nonfinite, g3_code_nonfinite(block));
@@ -143,15 +160,22 @@ __global__ void __launch_bounds__(kPfThreads) k_pf_norm_w(float* h, const float*
     if (!w_next) return;
     double ss = 0.0;
 #pragma unroll
-    for (uint32_t k = 0; k < NE; ++k) {
-        const float v = live[k] ? hv[k] : 0.0f;
-        ss += static_cast<double>(v) * static_cast<double>(v);
-    }
+    for (uint32_t k = 0; k < NQ; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v = live[k] ? hv[k][e] : 0.0f;
+            ss += static_cast<double>(v) * static_cast<double>(v);
+        }
     const float sc = pf_rms_scale(wave_red_sum_d(ss), n, eps);
 #pragma unroll
-    for (uint32_t k = 0; k < NE; ++k) {
-        const float y = into ? (hv[k] * sc) * wn[k] : hv[k] * (sc * wn[k]);
-        if (live[k]) pf_split(y, xhi + static_cast<uint64_t>(t) * n + ic[k], xlo + static_cast<uint64_t>(t) * n + ic[k]);
+    for (uint32_t k = 0; k < NQ; ++k) {
+        f4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = into ? (hv[k][e] * sc) * wn[k][e] : hv[k][e] * (sc * wn[k][e]);
+        if (live[k]) {
+            const uint64_t o = gm_off(t, ic[k], n / 32u);
+            pf_split4(y, x + o, x + o + kGmLo);
+        }
     }
 }
 
@@ -177,22 +201,15 @@ __device__ __forceinline__ float pf_gelu_mul(float x, float up) {
 // ---- GEMM on MFMA: Q8_0 weights ---------------------------------------------------------------
 
 struct PfGemm {
-    const _Float16* ahi;     // A [M][K] (row stride lda), f16 high and low parts
-    const _Float16* alo;
-    uint32_t lda;
+    const _Float16* a;       // A [M][K], an activation buffer (vrt_gemm.hpp)
     const uint8_t* w[3];     // W as Q8_0 matrices concatenated along N (rows[i] rows each)
     uint32_t rows[3];
     uint32_t nseg;
-    const uint8_t* w_end;    //   one past the arena
-    float* c;                // C [M][N] fp32 (row stride ldc; split z at c + z * c_bs), or
-    _Float16* chi;           //   C as f16 high and low parts
-    _Float16* clo;
-    uint32_t ldc;
+    float* c;                // C [M][N] fp32 (row stride N; split z at c + z * c_bs), or with glu
+    _Float16* o;             //   gelu_tanh(gate) * up as an activation buffer of N / 2 columns
     uint64_t c_bs;
     uint32_t M, N, K;
-    uint32_t glu;            // Q8_0 GEMM: w[0] = gate, w[1] = up (N = 2F), output gelu_tanh(gate) * up
-    const _Float16* wh;      // expanded weights: the quants of N rows as f16 [N][K] (nullptr: Q8_0 w)
-    const float* ws;         //   and their block scales [N][K / 32]
+    uint32_t glu;            // w[0] = gate, w[1] = up (N = 2F)
 };
 
 // C[M][N] = A[M][K] (f16 hi/lo) x W^T with W the Q8_0 rows (segments concatenated along N).
@@ -216,24 +233,23 @@ constexpr uint32_t kQgChunk = 12;  // K steps per straight-line chunk of the mai
 // Epilogue of the Q8_0 GEMMs: with G.glu the wave holding a 64-column group's up columns hands
 // them to the wave holding its gate columns through `xch` (LDS of at least NWN / 2 x 16 x 64
 // floats per 32-row band, free once the K loop is done), which writes gelu_tanh(gate) * up as
-// f16 hi/lo; otherwise the fp32 tile goes to split z's slice of C. Waves with `active` false
-// hold no tile but still pass the barriers.
+// f16 hi/lo; otherwise the fp32 tile goes to split z's slice of C.
 template <int WN, int NWN>
 __device__ __forceinline__ void pf_gemm_epilogue(const PfGemm& G, const float16v (&acc)[WN], uint32_t z, uint32_t m0,
                                                  uint32_t n0, uint32_t wm, uint32_t wn, uint32_t kh, uint32_t l32,
-                                                 uint32_t lane, float* xch, bool active = true) {
+                                                 uint32_t lane, float* xch) {
     if (G.glu) {
         // the wave holding a group's up columns hands them to the wave holding its gate columns
         // (gelu_tanh(gate) * up, shaders/gelu_mul.comp:23-31)
         static_assert(WN == 1, "one 32-column MFMA tile per wave");
         __syncthreads();   // every wave is done reading the LDS stages
         const uint32_t pair = wm * (NWN / 2u) + (wn >> 1);
-        if (active && (wn & 1u)) {
+        if (wn & 1u) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) xch[(pair * 16u + r) * 64u + lane] = acc[0][r];
         }
         __syncthreads();
-        if (!active || (wn & 1u)) return;
+        if (wn & 1u) return;
         const uint32_t F = G.N / 2u;
         const uint32_t col = n0 / 2u + 32u * (wn >> 1) + l32;
         if (col >= F) return;
@@ -241,13 +257,12 @@ __device__ __forceinline__ void pf_gemm_epilogue(const PfGemm& G, const float16v
         for (int r = 0; r < 16; ++r) {
             const uint32_t row = m0 + 32u * wm + 8u * (r / 4) + 4u * kh + (r % 4);
             if (row < G.M) {
-                const uint64_t o = static_cast<uint64_t>(row) * G.ldc + col;
-                pf_split(pf_gelu_mul(acc[0][r], xch[(pair * 16u + r) * 64u + lane]), G.chi + o, G.clo + o);
+                const uint64_t o = gm_off(row, col, F / 32u);
+                pf_split(pf_gelu_mul(acc[0][r], xch[(pair * 16u + r) * 64u + lane]), G.o + o, G.o + o + kGmLo);
             }
         }
         return;
     }
-    if (!active) return;
     float* c = G.c + static_cast<uint64_t>(z) * G.c_bs;
 #pragma unroll
     for (int j = 0; j < WN; ++j) {
@@ -256,7 +271,7 @@ __device__ __forceinline__ void pf_gemm_epilogue(const PfGemm& G, const float16v
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const uint32_t row = m0 + 32u * wm + 8u * (r / 4) + 4u * kh + (r % 4);
-            if (row < G.M) c[static_cast<uint64_t>(row) * G.ldc + col] = acc[j][r];
+            if (row < G.M) c[static_cast<uint64_t>(row) * G.N + col] = acc[j][r];
         }
     }
 }
@@ -320,9 +335,9 @@ __global__ void __launch_bounds__(128 * NWN) k_pf_gemm_q8(PfGemm G) {
             const uint32_t u = AU * tid + j, r = u >> 3, c = u & 7u;
             const uint32_t k = 32u * kb + 8u * c;
             const uint32_t rr = min(m0 + r, G.M - 1u), kk = min(k, 32u * kb_hi - 8u);
-            const uint64_t o = (static_cast<uint64_t>(rr) * G.lda + kk) * 2u;
-            R.a[0][j] = *reinterpret_cast<gv4>(reinterpret_cast<uintptr_t>(G.ahi) + o);
-            R.a[1][j] = *reinterpret_cast<gv4>(reinterpret_cast<uintptr_t>(G.alo) + o);
+            const uintptr_t o = reinterpret_cast<uintptr_t>(G.a + gm_off(rr, kk, nkb));
+            R.a[0][j] = *reinterpret_cast<gv4>(o);
+            R.a[1][j] = *reinterpret_cast<gv4>(o + 2u * kGmLo);
         }
         const uint32_t b = kb + wb;
         R.wl = wlive_t && b < kb_hi;
@@ -452,9 +467,8 @@ __device__ __forceinline__ uint64_t pf_vswz(uint32_t t, uint32_t d, uint32_t hd)
 
 // ---- QK-norm, RoPE, KV cache ------------------------------------------------------------
 
-// Row t of qkv = [q (H heads x hd) | k (hd) | v (hd)]: QK-norm per head (src/gemma3.cpp:
-// 1045-1104), NeoX RoPE at position t (:1371-1424), in place (q also as f16 hi/lo rows of
-// qhi/qlo); then k and v go to the KV cache slot t % slots when position t is still in the
+// Row t of qkv = [q (H heads x hd) | k (hd) | v (hd)], the sum of nsplit partials: QK-norm per head (src/gemma3.cpp:
+// 1045-1104), NeoX RoPE at position t (:1371-1424), q as f16 hi/lo rows of qhi/qlo; then k and v go to the KV cache slot t % slots when position t is still in the
 // window after the prompt (the serial loop's eviction leaves exactly those, :1590-1600); with
 // kv16 (1 fp16, 2 bf16) the cache holds 16-bit entries and k and v are rounded to them first
 // (the attention below then sees the cached values, as the serial loop does). The attention operands as f16 hi/lo: k and
@@ -464,7 +478,8 @@ __device__ __forceinline__ uint64_t pf_vswz(uint32_t t, uint32_t d, uint32_t hd)
 // One wave per head (lane l: dims l + 64 e): the sum of squares is a wave reduction and the
 // RoPE partners come through the wave's own LDS row, so the kernel has no barrier.
 constexpr uint32_t kPfQkMaxWaves = 8;
-__global__ void __launch_bounds__(kPfQkMaxWaves * 64) k_pf_qk(float* qkv, uint32_t T, uint32_t H, uint32_t hd,
+__global__ void __launch_bounds__(kPfQkMaxWaves * 64) k_pf_qk(const float* qkv, uint32_t nsplit,
+                                                            uint64_t sstride, uint32_t T, uint32_t H, uint32_t hd,
                                                             const float* q_norm, const float* k_norm,
                                                             const float* cos_t, const float* sin_t, float eps,
                                                             float* kc, float* vc, uint32_t slots, _Float16* qhi,
@@ -484,7 +499,7 @@ __global__ void __launch_bounds__(kPfQkMaxWaves * 64) k_pf_qk(float* qkv, uint32
     const uint32_t pos = p0 + t;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const uint32_t nqkv = (H + 2u) * hd, half = hd >> 1;
-    float* row = qkv + static_cast<uint64_t>(t) * nqkv;
+    const float* row = qkv + static_cast<uint64_t>(t) * nqkv;
     float* xw = xs[wave];
     const bool keep = t + slots >= T;   // the last `slots` positions of the segment reach the ring
     const uint64_t slot = static_cast<uint64_t>(pos % slots) * hd;
@@ -492,7 +507,13 @@ __global__ void __launch_bounds__(kPfQkMaxWaves * 64) k_pf_qk(float* qkv, uint32
     // them is in flight together (no branch, hence no wait, between them). v first: it is only
     // stored, after the heads.
     const uint32_t vi = min(threadIdx.x, hd - 1u);
-    const float vr = row[(H + 1u) * hd + vi];
+    // element i of the row, the split partials added in order
+    auto at = [&](uint32_t i) {
+        float v = row[i];
+        for (uint32_t z = 1; z < nsplit; ++z) v += row[z * sstride + i];
+        return v;
+    };
+    const float vr = at((H + 1u) * hd + vi);
     uint32_t ic[4], ei[4];
     bool live[4];
 #pragma unroll
@@ -508,12 +529,11 @@ __global__ void __launch_bounds__(kPfQkMaxWaves * 64) k_pf_qk(float* qkv, uint32
         sn[e] = sin_t[static_cast<uint64_t>(pos) * half + ei[e]];
     }
     for (uint32_t hh = wave; hh <= H; hh += nw) {   // H query heads, then the key head
-        const float* x = row + hh * hd;
         const float* w = hh < H ? q_norm : k_norm;
         float v[4], wv[4];
 #pragma unroll
         for (uint32_t e = 0; e < 4u; ++e) {
-            v[e] = x[ic[e]];
+            v[e] = at(hh * hd + ic[e]);
             wv[e] = w[ic[e]];
         }
         double sq = 0.0;
@@ -550,7 +570,7 @@ __global__ void __launch_bounds__(kPfQkMaxWaves * 64) k_pf_qk(float* qkv, uint32
         __builtin_amdgcn_wave_barrier();   // this head's reads of xw come before the next head's writes
     }
     for (uint32_t i = threadIdx.x; i < hd; i += blockDim.x) {   // v is not normed
-        const float vv0 = i == vi ? vr : row[(H + 1u) * hd + i];
+        const float vv0 = i == vi ? vr : at((H + 1u) * hd + i);
         const float vv = kv16 ? kv16_float(kv16_bits(vv0, kv16), kv16) : vv0;
         if (keep) {
             if (kv16) reinterpret_cast<uint16_t*>(vc)[slot + i] = kv16_bits(vv, kv16);
@@ -604,14 +624,14 @@ __global__ void __launch_bounds__(kPfThreads) k_pf_kv_hist(const float* kc, cons
 // r % 4][l % 32].
 constexpr uint32_t kPfAttKC = 128;   // keys per attention chunk (a multiple of 32)
 struct PfAttn {
-    const _Float16* qhi;   // [T][H * hd] queries, normed and rotated (overwritten by the output)
+    const _Float16* qhi;   // [T][H * hd] queries, normed and rotated
     const _Float16* qlo;
     const _Float16* khi;   // keys in pf_kswz order, by key coordinate (32-key tiles)
     const _Float16* klo;
     const _Float16* vhi;   // values in pf_vswz order
     const _Float16* vlo;
-    _Float16* ohi;         // [T][H * hd] output
-    _Float16* olo;
+    _Float16* o;           // output, an activation buffer of H * hd columns: row q - o_row of query row q
+    uint32_t o_row;        //   (earlier query rows of the first tile are not written)
     float* opart;          // [H][qtmax][maxc][32][hd] chunk partials, sum_j e_j v_j
     float* mpart;          // [H][qtmax][maxc][32] their maxima (base 2)
     double* lpart;         // [H][qtmax][maxc][32] their sums of e_j
@@ -802,20 +822,19 @@ __global__ void __launch_bounds__(256) k_pf_attn(PfAttn A) {
     lsum += __shfl_xor(lsum, 32);   // both lane halves now hold query q's sum
     const uint64_t unit = (static_cast<uint64_t>(h) * A.qtmax + i) * A.maxc + c;
     if (nch == 1u) {   // the whole key range: normalise and write the output rows
-        if (q >= T) return;
+        if (q >= T || q < A.o_row) return;
         const double den = lsum;
         if (wave == 0u && hf == 0u && (!(den > 0.0) || !__builtin_isfinite(den)))   // :1666-1670
             atomicMin(&A.st->nonfinite, g3_code_softmax(A.block));
         const float inv = static_cast<float>(1.0 / den);
-        const uint64_t oo = static_cast<uint64_t>(q) * qw + h * HD;
 #pragma unroll
         for (uint32_t j = 0; j < DW; ++j) {
             if (wave + 4u * j >= DT) continue;
 #pragma unroll
             for (uint32_t rq = 0; rq < 4u; ++rq) {
-                const uint32_t d = 32u * (wave + 4u * j) + 8u * rq + 4u * hf;
+                const uint64_t oo = gm_off(q - A.o_row, h * HD + 32u * (wave + 4u * j) + 8u * rq + 4u * hf, qw / 32u);
                 pf_split4(f4{o[j][4 * rq] * inv, o[j][4 * rq + 1] * inv, o[j][4 * rq + 2] * inv, o[j][4 * rq + 3] * inv},
-                          A.ohi + oo + d, A.olo + oo + d);
+                          A.o + oo, A.o + oo + kGmLo);
             }
         }
         return;
@@ -856,7 +875,7 @@ __global__ void __launch_bounds__(256) k_pf_attn_merge(PfAttn A) {
     pf_att_range(A.qo + q0, A.qo + T, A.window, ks, ke);
     const uint32_t nch = (ke - ks + A.kc - 1u) / A.kc;
     const uint32_t r = threadIdx.x >> 3, g = blockIdx.z * 8u + (threadIdx.x & 7u);
-    if (nch == 1u || q0 + r >= T) return;
+    if (nch == 1u || q0 + r >= T || q0 + r < A.o_row) return;
     const uint64_t unit0 = (static_cast<uint64_t>(h) * A.qtmax + i) * A.maxc;
     // chunks in groups of kG, every load of a group issued together (indices clamped to the last
     // chunk; the clamped duplicates are not used): one round of loads for up to kG chunks
@@ -906,200 +925,11 @@ __global__ void __launch_bounds__(256) k_pf_attn_merge(PfAttn A) {
     if (g == 0u && (!(den > 0.0) || !__builtin_isfinite(den)))   // :1666-1670
         atomicMin(&A.st->nonfinite, g3_code_softmax(A.block));
     const float inv = static_cast<float>(1.0 / den);
-    const uint64_t oo = static_cast<uint64_t>(q0 + r) * (A.H * HD) + h * HD + g * (4u * NF);
 #pragma unroll
-    for (uint32_t k = 0; k < NF; ++k)
-        pf_split4(f4{acc[k][0] * inv, acc[k][1] * inv, acc[k][2] * inv, acc[k][3] * inv}, A.ohi + oo + 4u * k,
-                  A.olo + oo + 4u * k);
-}
-
-// ---- expanded weights ------------------------------------------------------------------------
-
-// One-time expansion of a Q8_0 matrix for the prefill GEMMs: row n of the expanded matrix gets
-// the quants of source row src(n) as f16 (exact: |q| <= 127) and its block scales as fp32. With
-// `glu`, the rows are the gate/up matrices interleaved in groups of 64 (32 gate rows, then the
-// same 32 up rows: the column order of the gate/up GEMM's epilogue); otherwise up to three
-// matrices are concatenated. One thread per (row, block).
-__global__ void __launch_bounds__(kPfThreads) k_pf_expand(const uint8_t* w0, const uint8_t* w1, const uint8_t* w2,
-                                                          uint32_t rows0, uint32_t rows1, uint32_t N, uint32_t nkb,
-                                                          uint32_t glu, _Float16* wh, float* ws) {
-    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kPfThreads + threadIdx.x;
-    if (i >= static_cast<uint64_t>(N) * nkb) return;
-    const uint32_t n = static_cast<uint32_t>(i / nkb), b = static_cast<uint32_t>(i % nkb);
-    const uint8_t* src;
-    if (glu) {
-        const uint32_t grp = n >> 6, wi = n & 63u;
-        src = (wi < 32u ? w0 : w1) + static_cast<uint64_t>(32u * grp + (wi & 31u)) * nkb * 34u;
-    } else if (n < rows0) {
-        src = w0 + static_cast<uint64_t>(n) * nkb * 34u;
-    } else if (n < rows0 + rows1) {
-        src = w1 + static_cast<uint64_t>(n - rows0) * nkb * 34u;
-    } else {
-        src = w2 + static_cast<uint64_t>(n - rows0 - rows1) * nkb * 34u;
+    for (uint32_t k = 0; k < NF; ++k) {
+        const uint64_t oo = gm_off(q0 + r - A.o_row, h * HD + g * (4u * NF) + 4u * k, A.H * HD / 32u);
+        pf_split4(f4{acc[k][0] * inv, acc[k][1] * inv, acc[k][2] * inv, acc[k][3] * inv}, A.o + oo, A.o + oo + kGmLo);
     }
-    const uint8_t* blk = src + 34u * b;
-    ws[i] = half_bits_to_float(static_cast<uint32_t>(blk[0]) | (static_cast<uint32_t>(blk[1]) << 8));
-    _Float16* dst = wh + static_cast<uint64_t>(n) * nkb * 32u + 32u * b;
-#pragma unroll
-    for (uint32_t k = 0; k < 32u; ++k) dst[k] = static_cast<_Float16>(static_cast<float>(static_cast<int8_t>(blk[2 + k])));
-}
-
-// The Q8_0 GEMM of k_pf_gemm_q8 on expanded weights (G.wh, G.ws): a K step of SB Q8_0 blocks
-// (32 SB wide) stages the f16 rows of the tile's W blocks with plain 16-byte copies (no int8
-// conversion on the K loop's critical path) and the SB block scales per row. Same tiles,
-// splits and epilogues as k_pf_gemm_q8, with KW times the waves: wave group kw (of 2 NWN
-// waves) computes the step's Q8_0 blocks kw, kw + KW, ... for every tile, so a SIMD runs KW
-// waves whose LDS reads, MFMA chains and scale-and-add work overlap; before the epilogue the
-// partial tiles of groups 1..KW-1 are added, in group order, to those of group 0 through LDS.
-// The register ring holds 8 / SB steps in flight (the same bytes for every SB).
-template <int WN, int NWN, int SB, int KW>
-__global__ void __launch_bounds__(128 * NWN * KW) k_pf_gemm_h(PfGemm G) {
-    constexpr uint32_t NT = 128u * NWN * KW;
-    constexpr uint32_t BN = 32u * WN * NWN;
-    constexpr uint32_t UR = 4u * SB;                   // 16-byte units per staged row
-    constexpr uint32_t PITCH = 16u * UR + 16u;         // LDS row pitch in bytes (padded)
-    constexpr uint32_t AU = 2u * kQgBM * UR / NT;      // A units per thread (hi units, then lo)
-    constexpr uint32_t WU = BN * UR / NT;              // W units per thread
-    constexpr uint32_t AHEAD = 8u / SB;                // steps in flight ahead of the one computed
-    constexpr uint32_t CHUNK = 24u / SB;               // steps per straight-line chunk
-    static_assert((SB == 2 || SB == 4) && (KW == 2 || KW == 4) && SB % KW == 0, "blocks per step, wave groups");
-    static_assert(AU >= 1u && 2u * kQgBM * UR % NT == 0u, "whole A units per thread");
-    static_assert(WU >= 1u && BN * UR % NT == 0u, "whole W units per thread");
-    static_assert(BN <= NT, "one row of scales per thread");
-    __shared__ __align__(16) unsigned char s_a[2][2][kQgBM * PITCH];
-    __shared__ __align__(16) unsigned char s_w[2][BN * PITCH];
-    __shared__ float s_sc[2][BN][SB];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t kh = lane >> 5, l32 = lane & 31u;
-    const uint32_t m0 = blockIdx.y * kQgBM, n0 = blockIdx.x * BN;
-    const uint32_t nkb = G.K >> 5;
-    const uint32_t S = gridDim.z, z = blockIdx.z;
-    const uint32_t kb_lo = nkb * z / S, kb_hi = nkb * (z + 1u) / S;
-    const uint32_t nsteps = (kb_hi - kb_lo + SB - 1u) / SB;
-    typedef const __attribute__((address_space(1))) v4u* gv4;
-    struct Stage {
-        v4u a[AU];   // unit u = AU tid + j: array u / (UR kQgBM), row (u % (UR kQgBM)) / UR, column u % UR
-        v4u w[WU];
-        float sc[SB];
-    };
-    // Every load is issued at a clamped, in-bounds address (dead data is zeroed when stored).
-    auto load = [&](uint32_t step, Stage& R) {
-        const uint32_t kb = kb_lo + SB * step;
-#pragma unroll
-        for (uint32_t j = 0; j < AU; ++j) {
-            const uint32_t u = AU * tid + j, ui = u % (UR * kQgBM), r = ui / UR, c = ui % UR;
-            const uint32_t k = 32u * kb + 8u * c;
-            const uint32_t rr = min(m0 + r, G.M - 1u), kk = min(k, 32u * kb_hi - 8u);
-            const uint64_t o = (static_cast<uint64_t>(rr) * G.lda + kk) * 2u;
-            R.a[j] = *reinterpret_cast<gv4>(reinterpret_cast<uintptr_t>(u < UR * kQgBM ? G.ahi : G.alo) + o);
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < WU; ++j) {
-            const uint32_t u = WU * tid + j, r = u / UR, c = u % UR;
-            const uint32_t rr = min(n0 + r, G.N - 1u), kk = min(32u * kb + 8u * c, 32u * kb_hi - 8u);
-            R.w[j] = *reinterpret_cast<gv4>(reinterpret_cast<uintptr_t>(G.wh) + (static_cast<uint64_t>(rr) * G.K + kk) * 2u);
-        }
-        {   // the step's block scales of row tid (clamped to the split's last block)
-            typedef const __attribute__((address_space(1))) float* gf;
-            const uint32_t rr = min(n0 + (tid < BN ? tid : 0u), G.N - 1u);
-            const gf row = reinterpret_cast<gf>(reinterpret_cast<uintptr_t>(G.ws + static_cast<uint64_t>(rr) * nkb));
-#pragma unroll
-            for (uint32_t q = 0; q < SB; ++q) R.sc[q] = row[min(kb + q, kb_hi - 1u)];
-        }
-    };
-    auto store = [&](const Stage& R, uint32_t st, uint32_t step) {
-        const uint32_t kb = kb_lo + SB * step;
-#pragma unroll
-        for (uint32_t j = 0; j < AU; ++j) {
-            const uint32_t u = AU * tid + j, ui = u % (UR * kQgBM), r = ui / UR, c = ui % UR;
-            const bool live = m0 + r < G.M && 32u * kb + 8u * c < 32u * kb_hi;
-            *reinterpret_cast<v4u*>(&s_a[st][u / (UR * kQgBM)][r * PITCH + c * 16u]) = live ? R.a[j] : v4u{0u, 0u, 0u, 0u};
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < WU; ++j) {
-            const uint32_t u = WU * tid + j, r = u / UR, c = u % UR;
-            const bool live = n0 + r < G.N && 32u * kb + 8u * c < 32u * kb_hi;
-            *reinterpret_cast<v4u*>(&s_w[st][r * PITCH + c * 16u]) = live ? R.w[j] : v4u{0u, 0u, 0u, 0u};
-        }
-        if (tid < BN) {
-            const bool rl = n0 + tid < G.N;
-#pragma unroll
-            for (uint32_t q = 0; q < SB; ++q) s_sc[st][tid][q] = rl && kb + q < kb_hi ? R.sc[q] : 0.0f;
-        }
-    };
-    const uint32_t kw = wave / (2u * NWN), wv = wave % (2u * NWN);   // block group of the step, tile
-    const uint32_t wm = wv / NWN, wn = wv % NWN;
-    float16v acc[WN];
-#pragma unroll
-    for (int j = 0; j < WN; ++j) acc[j] = float16v{};
-    auto compute = [&](uint32_t st) {
-        const unsigned char* pa_hi = &s_a[st][0][(32u * wm + l32) * PITCH + 16u * kh];
-        const unsigned char* pa_lo = &s_a[st][1][(32u * wm + l32) * PITCH + 16u * kh];
-#pragma unroll
-        for (uint32_t bq = 0; bq < SB / KW; ++bq) {
-            const uint32_t b = kw + KW * bq;
-            half8 ah[2], al[2];
-#pragma unroll
-            for (uint32_t ks = 0; ks < 2; ++ks) {
-                ah[ks] = *reinterpret_cast<const half8*>(pa_hi + 64u * b + 32u * ks);
-                al[ks] = *reinterpret_cast<const half8*>(pa_lo + 64u * b + 32u * ks);
-            }
-#pragma unroll
-            for (int j = 0; j < WN; ++j) {
-                const uint32_t nl = 32u * (WN * wn + j) + l32;
-                const unsigned char* pw = &s_w[st][nl * PITCH + 64u * b + 16u * kh];
-                const half8 w0 = *reinterpret_cast<const half8*>(pw), w1 = *reinterpret_cast<const half8*>(pw + 32u);
-                float16v p = {};
-                p = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[0], w0, p, 0, 0, 0);
-                p = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[0], w0, p, 0, 0, 0);
-                p = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[1], w1, p, 0, 0, 0);
-                p = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[1], w1, p, 0, 0, 0);
-                const float sc = s_sc[st][nl][b];
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[j][r] += sc * p[r];
-            }
-        }
-    };
-    static_assert(AHEAD <= CHUNK, "ring inside a chunk");
-    for (uint32_t i = 0; i < nsteps; i += CHUNK) {
-        Stage R[AHEAD];
-        auto clamp = [&](uint32_t j) { return min(i + j, nsteps - 1u); };
-#pragma unroll
-        for (uint32_t u = 0; u < AHEAD; ++u) load(clamp(u), R[u]);
-#pragma unroll
-        for (uint32_t u = 0; u < CHUNK; ++u) {
-            const uint32_t j = i + u;
-            if (j < nsteps) {
-                store(R[u % AHEAD], j & 1u, j);
-                __syncthreads();
-            }
-            if (u + AHEAD < CHUNK) load(clamp(u + AHEAD), R[u % AHEAD]);
-            if (j < nsteps) compute(j & 1u);
-        }
-    }
-    {   // the other groups' partials into group 0 (s_a: (KW - 1) 2 NWN WN 16 x 64 floats fit)
-        constexpr uint32_t RS = 2u * NWN * WN * 16u * 64u;   // floats per group
-        static_assert((KW - 1u) * RS * 4u <= sizeof(s_a), "reduction area");
-        __syncthreads();   // every wave is done reading the LDS stages
-        float* red = reinterpret_cast<float*>(&s_a[0][0][0]);
-        if (kw != 0u) {
-#pragma unroll
-            for (int j = 0; j < WN; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) red[(kw - 1u) * RS + ((wv * WN + j) * 16u + r) * 64u + lane] = acc[j][r];
-        }
-        __syncthreads();
-        if (kw == 0u) {
-#pragma unroll
-            for (uint32_t q = 1; q < KW; ++q)
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[j][r] += red[(q - 1u) * RS + ((wv * WN + j) * 16u + r) * 64u + lane];
-        }
-    }   // (the GLU epilogue's exchange reuses s_a after a barrier of its own)
-    pf_gemm_epilogue<WN, NWN>(G, acc, z, m0, n0, wm, wn, kh, l32, lane, reinterpret_cast<float*>(&s_a[0][0][0]),
-                              kw == 0u);
 }
 
 // ---- host side --------------------------------------------------------------------------
@@ -1115,139 +945,102 @@ static int pf_launch_q8(const PfGemm& G, uint32_t splits, hipStream_t s) {
     return VRT_OK;
 }
 
-constexpr int kPfStepBlocks = 4;   // Q8_0 blocks per K step of the 64 x 64 tiles
-constexpr int kPfWaveGroups = 4;   // their wave groups (the 64 x 128 tiles: 2 blocks, 2 groups)
-
-template <int WN, int NWN, int SB, int KW>
-static int pf_launch_h(const PfGemm& G, uint32_t splits, hipStream_t s) {
-    constexpr uint32_t BN = 32u * WN * NWN;
-    const dim3 grid((G.N + BN - 1u) / BN, (G.M + kQgBM - 1u) / kQgBM, splits);
-    PfGemm arg = G;
-    void* args[] = {&arg};
-    VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_gemm_h<WN, NWN, SB, KW>), grid,
-                                  dim3(128u * NWN * KW), args, 0, s));
-    return VRT_OK;
+// K splits of the GEMMs on the Q8_0 rows: enough workgroups to cover the CUs.
+static uint32_t pf_splits_q8(uint32_t M, uint32_t N, uint32_t K) {
+    const uint32_t tiles = ((M + kQgBM - 1u) / kQgBM) * ((N + 63u) / 64u);
+    const uint32_t s = std::min(kPfMaxSplits, std::max(1u, 256u / std::max(1u, tiles)));
+    return std::max(1u, std::min(s, (K / 32u) / 2u));
 }
 
-// The Q8_0 GEMM's launch: on the expanded weights when `ex` holds them, else on the arena.
-static int pf_launch_w(PfGemm& G, const PfMatrix* ex, uint32_t splits, hipStream_t s) {
-    const uint32_t mt = (G.M + kQgBM - 1u) / kQgBM;
-    const bool wide = G.N % 128u == 0u && (G.N / 128u) * mt >= 128u;
-    if (ex && ex->h) {
-        G.wh = static_cast<const _Float16*>(ex->h);
-        G.ws = ex->s;
-        // one row tile (the batched decode's rows): 32-column tiles, twice the workgroups (1.256 ->
-        // 1.211 ms per step of 64 sequences); the GLU epilogue pairs gate and up inside 64 columns
-        if (!G.glu && G.M <= kQgBM) return pf_launch_h<1, 1, kPfStepBlocks, kPfWaveGroups>(G, splits, s);
-        return wide ? pf_launch_h<1, 4, 2, 2>(G, splits, s) : pf_launch_h<1, 2, kPfStepBlocks, kPfWaveGroups>(G, splits, s);
-    }
-    return wide ? pf_launch_q8<1, 4>(G, splits, s) : pf_launch_q8<1, 2>(G, splits, s);
-}
-
-// C[M][N] = A[M][K] (f16 hi/lo) x W^T, W = Q8_0 matrices concatenated along N (or their
-// expansion `ex`). With splits > 1 the K blocks are split and C holds the partial products
-// C + z * M * N, z < splits.
-static int pf_gemm(vrt_g3* g, const _Float16* ahi, const _Float16* alo, uint32_t M, uint32_t K,
+// C[M][N] = A[M][K] (an activation buffer) x W^T, W = Q8_0 matrices concatenated along N, or
+// their expansion `ex` where there is one (vrt_gemm.hip). With `used`, the K blocks may be split over
+// *used workgroups; C then holds the partial products C + z * M * N, z < *used. With glu (segs: gate, up):
+// gelu_tanh(A Wg^T) * (A Wu^T) into the activation buffer o (src/gemma3.cpp:1720-1801 up to the
+// down projection).
+static int pf_gemm(const _Float16* a, uint32_t M, uint32_t K,
                    std::initializer_list<std::pair<const uint8_t*, uint32_t>> segs, const PfMatrix* ex, float* c,
-                   uint32_t splits, hipStream_t s) {
+                   _Float16* o, bool glu, uint32_t* used, hipStream_t s) {
+    uint32_t N = 0;
+    for (const auto& sg : segs) N += sg.second;
+    // any N: rows past N load clamped, in-bounds rows, are zeroed in LDS and never stored
+    if (K % 32u != 0u || N == 0u || (glu && N % 64u != 0u))
+        return set_error(VRT_ERR_INVALID, "prefill GEMM shape not supported");
+    if (ex && ex->h) {
+        GmArgs G{};
+        G.a = a;
+        G.w = static_cast<const _Float16*>(ex->h);
+        G.ws = ex->s;
+        G.c = c;
+        G.o = o;
+        G.c_bs = static_cast<uint64_t>(M) * N;
+        G.ldc = G.N = N;
+        G.M = M;
+        G.nkb = K / 32u;
+        G.npad = (N + kGmRowPad - 1u) / kGmRowPad * kGmRowPad;
+        const uint32_t splits = used ? gm_splits(M, N, G.nkb) : 1u;
+        if (used) *used = splits;
+        return gm_run(G, splits, glu, s);
+    }
     PfGemm G{};
-    G.ahi = ahi;
-    G.alo = alo;
-    G.lda = K;
+    G.a = a;
     for (const auto& sg : segs) {
         G.w[G.nseg] = sg.first;
         G.rows[G.nseg++] = sg.second;
-        G.N += sg.second;
     }
-    G.w_end = g->P.arena_end;
+    G.N = N;
     G.c = c;
-    G.ldc = G.N;
+    G.o = o;
+    G.c_bs = static_cast<uint64_t>(M) * N;
     G.M = M;
     G.K = K;
-    // any N: rows past N load clamped, in-bounds rows, are zeroed in LDS and never stored
-    if (K % 32u != 0u || G.N == 0u) return set_error(VRT_ERR_INVALID, "prefill GEMM shape not supported");
-    G.c_bs = static_cast<uint64_t>(M) * G.N;
-    splits = std::max(1u, std::min(splits, (K / 32u) / 2u));
-    return pf_launch_w(G, ex, splits, s);
+    G.glu = glu ? 1u : 0u;
+    const uint32_t splits = used ? pf_splits_q8(M, N, K) : 1u;
+    if (used) *used = splits;
+    const uint32_t mt = (M + kQgBM - 1u) / kQgBM;
+    return N % 128u == 0u && (N / 128u) * mt >= 128u ? pf_launch_q8<1, 4>(G, splits, s) : pf_launch_q8<1, 2>(G, splits, s);
 }
 
-// gelu_tanh(A Wg^T) * (A Wu^T) as f16 hi/lo [M][F] (row stride F): the gate/up GEMM with the
-// product in its epilogue (src/gemma3.cpp:1720-1801 up to the down projection), one K split.
-static int pf_gemm_glu(vrt_g3* g, const _Float16* ahi, const _Float16* alo, uint32_t M, uint32_t K, const uint8_t* wg,
-                       const uint8_t* wu, uint32_t F, const PfMatrix* ex, _Float16* ohi, _Float16* olo, hipStream_t s) {
-    PfGemm G{};
-    G.ahi = ahi;
-    G.alo = alo;
-    G.lda = K;
-    G.w[0] = wg;
-    G.w[1] = wu;
-    G.rows[0] = G.rows[1] = F;
-    G.nseg = 2u;
-    G.N = 2u * F;
-    G.w_end = g->P.arena_end;
-    G.chi = ohi;
-    G.clo = olo;
-    G.ldc = F;
-    G.M = M;
-    G.K = K;
-    G.glu = 1u;
-    if (K % 32u != 0u || F % 32u != 0u) return set_error(VRT_ERR_INVALID, "prefill GEMM shape not supported");
-    return pf_launch_w(G, ex, 1u, s);
-}
-
-// K splits of the 640-row projections (O and down): enough workgroups to cover the CUs.
-uint32_t pf_splits(uint32_t M, uint32_t N) {
-    const uint32_t tiles = ((M + kQgBM - 1u) / kQgBM) * ((N + 63u) / 64u);
-    return std::min(kPfMaxSplits, std::max(1u, 256u / std::max(1u, tiles)));
-}
-
-// k_pf_norm_w over `rows` rows of n <= 2048 elements (elements per lane: the smallest of 4, 8,
-// 12, 16, 24, 32 that covers n).
+// k_pf_norm_w over `rows` rows of n <= 2048 elements (runs of four per lane: the smallest of 1, 2, 3,
+// 4, 6, 8 that covers n).
 int pf_norm(float* h, const float* f, uint32_t nsplit, uint64_t sstride, const float* w_post, const float* w_next,
-            uint32_t n, float eps, _Float16* xhi, _Float16* xlo, G3State* st, uint32_t block, uint32_t rows, hipStream_t s,
-            bool into) {
+            uint32_t n, float eps, _Float16* x, G3State* st, uint32_t block, uint32_t rows, hipStream_t s, bool into) {
     uint32_t in = into ? 1u : 0u;
-    void* args[] = {&h, &f, &nsplit, &sstride, &w_post, &w_next, &n, &eps, &xhi, &xlo, &st, &block, &rows, &in};
-    const uint32_t ne = (n + 63u) / 64u;
-    const void* fn = ne <= 4u    ? reinterpret_cast<const void*>(&k_pf_norm_w<4>)
-                     : ne <= 8u  ? reinterpret_cast<const void*>(&k_pf_norm_w<8>)
-                     : ne <= 12u ? reinterpret_cast<const void*>(&k_pf_norm_w<12>)
-                     : ne <= 16u ? reinterpret_cast<const void*>(&k_pf_norm_w<16>)
-                     : ne <= 24u ? reinterpret_cast<const void*>(&k_pf_norm_w<24>)
-                     : ne <= 32u ? reinterpret_cast<const void*>(&k_pf_norm_w<32>)
-                                 : nullptr;
-    if (!fn || nsplit > kPfMaxSplits) return set_error(VRT_ERR_INVALID, "prefill norm shape not supported");
+    void* args[] = {&h, &f, &nsplit, &sstride, &w_post, &w_next, &n, &eps, &x, &st, &block, &rows, &in};
+    const uint32_t nq = (n + 255u) / 256u;
+    const void* fn = nq <= 1u   ? reinterpret_cast<const void*>(&k_pf_norm_w<1>)
+                     : nq <= 2u ? reinterpret_cast<const void*>(&k_pf_norm_w<2>)
+                     : nq <= 3u ? reinterpret_cast<const void*>(&k_pf_norm_w<3>)
+                     : nq <= 4u ? reinterpret_cast<const void*>(&k_pf_norm_w<4>)
+                     : nq <= 6u ? reinterpret_cast<const void*>(&k_pf_norm_w<6>)
+                     : nq <= 8u ? reinterpret_cast<const void*>(&k_pf_norm_w<8>)
+                                : nullptr;
+    if (!fn || n % 32u != 0u || nsplit > kPfMaxSplits) return set_error(VRT_ERR_INVALID, "prefill norm shape not supported");
     const uint32_t per = kPfThreads / 64u;
     VRT_HIP_CHECK(hipLaunchKernel(fn, dim3((rows + per - 1u) / per), dim3(kPfThreads), args, 0, s));
     return VRT_OK;
 }
 
-// Block l's projection `which` over M rows (the building blocks of the batched decode): C =
-// A x W^T with K split over `splits` workgroups (clamped to the K blocks; the count used goes to
-// *used), partial z at c + z * M * N.
-int pf_project(vrt_g3* g, uint32_t l, uint32_t which, const _Float16* ahi, const _Float16* alo, uint32_t M, float* c,
-               uint32_t splits, uint32_t* used, hipStream_t s) {
+// Block l's projection `which` over the M rows of the activation buffer a: C = A x W^T, or partial
+// z of *used K splits at c + z * M * N.
+int pf_project(vrt_g3* g, uint32_t l, uint32_t which, const _Float16* a, uint32_t M, float* c, uint32_t* used, hipStream_t s) {
     const LayerParams& Ly = g->layers[l];
     const PfLayerW* lw = g->pf.lw.empty() ? nullptr : &g->pf.lw[l];
     const uint32_t d = g->cfg.embedding_length, hd = g->cfg.head_dim, qw = g->cfg.head_count * hd;
     const uint32_t F = g->cfg.feed_forward_length;
-    const uint32_t K = which == kProjQkv ? d : (which == kProjO ? qw : F);
-    *used = std::max(1u, std::min(splits, (K / 32u) / 2u));
     switch (which) {
-    case kProjQkv: return pf_gemm(g, ahi, alo, M, d, {{Ly.wq, qw}, {Ly.wk, hd}, {Ly.wv, hd}}, lw ? &lw->qkv : nullptr, c, splits, s);
-    case kProjO: return pf_gemm(g, ahi, alo, M, qw, {{Ly.wo, d}}, lw ? &lw->o : nullptr, c, splits, s);
-    case kProjDown: return pf_gemm(g, ahi, alo, M, F, {{Ly.wd, d}}, lw ? &lw->down : nullptr, c, splits, s);
+    case kProjQkv: return pf_gemm(a, M, d, {{Ly.wq, qw}, {Ly.wk, hd}, {Ly.wv, hd}}, lw ? &lw->qkv : nullptr, c, nullptr, false, used, s);
+    case kProjO: return pf_gemm(a, M, qw, {{Ly.wo, d}}, lw ? &lw->o : nullptr, c, nullptr, false, used, s);
+    case kProjDown: return pf_gemm(a, M, F, {{Ly.wd, d}}, lw ? &lw->down : nullptr, c, nullptr, false, used, s);
     default: return set_error(VRT_ERR_INVALID, "unknown projection %u", which);
     }
 }
 
-// Block l's gelu_tanh(gate) * up over M rows, as f16 hi/lo [M][F].
-int pf_ffn_glu(vrt_g3* g, uint32_t l, const _Float16* ahi, const _Float16* alo, uint32_t M, _Float16* ghi,
-               _Float16* glo, hipStream_t s) {
+// Block l's gelu_tanh(gate) * up over the M rows of a, into the activation buffer o of F columns.
+int pf_ffn_glu(vrt_g3* g, uint32_t l, const _Float16* a, uint32_t M, _Float16* o, hipStream_t s) {
     const LayerParams& Ly = g->layers[l];
     const PfLayerW* lw = g->pf.lw.empty() ? nullptr : &g->pf.lw[l];
-    return pf_gemm_glu(g, ahi, alo, M, g->cfg.embedding_length, Ly.wg, Ly.wu, g->cfg.feed_forward_length,
-                       lw ? &lw->gu : nullptr, ghi, glo, s);
+    const uint32_t F = g->cfg.feed_forward_length;
+    return pf_gemm(a, M, g->cfg.embedding_length, {{Ly.wg, F}, {Ly.wu, F}}, lw ? &lw->gu : nullptr, nullptr, o, true, nullptr, s);
 }
 
 // Embedding rows of `rows` tokens (device array) into h [rows][d].
@@ -1260,10 +1053,10 @@ int pf_embed_rows(vrt_g3* g, const uint32_t* tokens, uint32_t rows, float* h, hi
     return VRT_OK;
 }
 
-// Logits of M rows against the tied Q8_0 embedding table: logits [M][vocab] = x W_embd^T, x as
-// f16 hi/lo [M][d] (MFMA on the Q8_0 rows of the arena, one K split).
-int pf_lm_logits(vrt_g3* g, const _Float16* xhi, const _Float16* xlo, uint32_t M, float* logits, hipStream_t s) {
-    return pf_gemm(g, xhi, xlo, M, g->cfg.embedding_length, {{g->P.tok_embd, g->cfg.vocab_size}}, nullptr, logits, 1u, s);
+// Logits of M rows against the tied Q8_0 embedding table: logits [M][vocab] = x W_embd^T, x an
+// activation buffer (MFMA on the Q8_0 rows of the arena, one K split).
+int pf_lm_logits(vrt_g3* g, const _Float16* x, uint32_t M, float* logits, hipStream_t s) {
+    return pf_gemm(x, M, g->cfg.embedding_length, {{g->P.tok_embd, g->cfg.vocab_size}}, nullptr, logits, nullptr, false, nullptr, s);
 }
 
 static uint32_t pf_pad(uint32_t T) { return (T + kPfTile - 1u) / kPfTile * kPfTile; }
@@ -1271,7 +1064,6 @@ static uint32_t pf_pad(uint32_t T) { return (T + kPfTile - 1u) / kPfTile * kPfTi
 int pf_setup(vrt_g3* g, uint32_t max_t) {
     const uint32_t d = g->cfg.embedding_length, H = g->cfg.head_count, hd = g->cfg.head_dim;
     const uint32_t F = g->cfg.feed_forward_length, qw = H * hd, nqkv = qw + 2u * hd;
-    const uint32_t kmax = std::max(std::max(d, qw), F);
     PfState& p = g->pf;
     p.max_t = 0;
     if (d > 8u * kPfThreads || hd > 256u || hd % 32u || d % 32u || qw % 32u || F % 32u || nqkv % 32u) return VRT_OK;
@@ -1286,12 +1078,16 @@ int pf_setup(vrt_g3* g, uint32_t max_t) {
     p.h = static_cast<float*>(q);
     if (int rc = take(static_cast<size_t>(max_t) * d * 4u * kPfMaxSplits, &q)) return rc;
     p.x = static_cast<float*>(q);
-    if (int rc = take(static_cast<size_t>(max_t) * kmax * 2u, &q)) return rc;
-    p.ahi = q;
-    if (int rc = take(static_cast<size_t>(max_t) * kmax * 2u, &q)) return rc;
-    p.alo = q;
-    if (int rc = take(static_cast<size_t>(max_t) * std::max(nqkv, 2u * F) * 4u, &q)) return rc;
-    p.big = static_cast<float*>(q);
+    if (int rc = take(gm_size(max_t, std::max(d, qw)) * 2u, &q)) return rc;
+    p.a = static_cast<_Float16*>(q);
+    if (int rc = take(gm_size(max_t, F) * 2u, &q)) return rc;
+    p.g = static_cast<_Float16*>(q);
+    if (int rc = take(static_cast<size_t>(max_t) * nqkv * 4u * kPfMaxSplits, &q)) return rc;
+    p.qkv = static_cast<float*>(q);
+    if (int rc = take(static_cast<size_t>(max_t) * qw * 2u, &q)) return rc;
+    p.qhi = static_cast<_Float16*>(q);
+    if (int rc = take(static_cast<size_t>(max_t) * qw * 2u, &q)) return rc;
+    p.qlo = static_cast<_Float16*>(q);
     // keys and values of a segment's history and rows (f16 each): prompts longer than max_t run
     // in segments whose keys reach back to position 0 in a global block
     p.tkv = static_cast<uint32_t>(std::max<uint64_t>(tp, pf_pad(g->cfg.context_length)));
@@ -1317,30 +1113,23 @@ int pf_setup(vrt_g3* g, uint32_t max_t) {
         p.lw.resize(g->layers.size());
         const hipStream_t s = g->ctx->stream;
         auto expand = [&](const uint8_t* w0, const uint8_t* w1, const uint8_t* w2, uint32_t r0, uint32_t r1, uint32_t N,
-                          uint32_t K, uint32_t glu, PfMatrix* m) -> int {
+                          uint32_t K, bool glu, PfMatrix* m) -> int {
             void* hq;
             void* sq;
-            if (int rc = take(static_cast<size_t>(N) * K * 2u, &hq)) return rc;
-            if (int rc = take(static_cast<size_t>(N) * (K / 32u) * 4u, &sq)) return rc;
-            uint32_t nkb = K / 32u;
-            _Float16* wh = static_cast<_Float16*>(hq);
-            float* ws = static_cast<float*>(sq);
-            void* args[] = {&w0, &w1, &w2, &r0, &r1, &N, &nkb, &glu, &wh, &ws};
-            const uint64_t n = static_cast<uint64_t>(N) * nkb;
-            VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_expand),
-                                          dim3(static_cast<uint32_t>((n + kPfThreads - 1u) / kPfThreads)),
-                                          dim3(kPfThreads), args, 0, s));
+            const size_t np = (N + kGmRowPad - 1u) / kGmRowPad * kGmRowPad;
+            if (int rc = take(np * K * 2u, &hq)) return rc;
+            if (int rc = take(np * (K / 32u) * 4u, &sq)) return rc;
             m->h = hq;
-            m->s = ws;
-            return VRT_OK;
+            m->s = static_cast<const float*>(sq);
+            return gm_expand(w0, w1, w2, r0, r1, N, K / 32u, glu, static_cast<_Float16*>(hq), static_cast<float*>(sq), s);
         };
         for (size_t l = 0; l < g->layers.size(); ++l) {
             const LayerParams& Ly = g->layers[l];
             PfLayerW& w = p.lw[l];
-            if (int rc = expand(Ly.wq, Ly.wk, Ly.wv, qw, hd, nqkv, d, 0u, &w.qkv)) return rc;
-            if (int rc = expand(Ly.wo, Ly.wo, Ly.wo, d, 0u, d, qw, 0u, &w.o)) return rc;
-            if (int rc = expand(Ly.wg, Ly.wu, Ly.wu, F, F, 2u * F, d, 1u, &w.gu)) return rc;
-            if (int rc = expand(Ly.wd, Ly.wd, Ly.wd, d, 0u, d, F, 0u, &w.down)) return rc;
+            if (int rc = expand(Ly.wq, Ly.wk, Ly.wv, qw, hd, nqkv, d, false, &w.qkv)) return rc;
+            if (int rc = expand(Ly.wo, Ly.wo, Ly.wo, d, 0u, d, qw, false, &w.o)) return rc;
+            if (int rc = expand(Ly.wg, Ly.wu, Ly.wu, F, F, 2u * F, d, true, &w.gu)) return rc;
+            if (int rc = expand(Ly.wd, Ly.wd, Ly.wd, d, 0u, d, F, false, &w.down)) return rc;
         }
     }
     p.max_t = max_t;
@@ -1358,15 +1147,17 @@ static int pf_attn_launch(const PfAttn& A, dim3 grid, hipStream_t s) {
     return VRT_OK;
 }
 
-// Causal local/global attention of one block (k_pf_attn) over the queries in qhi/qlo [T][H hd],
-// written back in place as the attention output, for the query tiles from qt0 on.
-static int pf_attention(vrt_g3* g, const LayerParams& Ly, uint32_t T, uint32_t qt0, _Float16* qhi, _Float16* qlo,
-                        hipStream_t s, uint32_t qo = 0) {
+// Causal local/global attention of one block (k_pf_attn) over the queries of p.qhi/p.qlo [T][H hd],
+// for the query rows from o_row on; row q goes to row q - o_row of the activation buffer p.a.
+static int pf_attention(vrt_g3* g, const LayerParams& Ly, uint32_t T, uint32_t o_row, hipStream_t s, uint32_t qo) {
     const PfState& p = g->pf;
     const uint32_t H = g->cfg.head_count, hd = g->cfg.head_dim;
     PfAttn A{};
-    A.qhi = A.ohi = qhi;
-    A.qlo = A.olo = qlo;
+    A.qhi = p.qhi;
+    A.qlo = p.qlo;
+    A.o = p.a;
+    A.o_row = o_row;
+    const uint32_t qt0 = o_row / 32u;
     A.khi = static_cast<const _Float16*>(p.khi);
     A.klo = static_cast<const _Float16*>(p.klo);
     A.vhi = static_cast<const _Float16*>(p.vhi);
@@ -1419,14 +1210,12 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0, bool final) {
     const PfState& p = g->pf;
     hipStream_t s = g->ctx->stream;
     uint32_t d = g->cfg.embedding_length, H = g->cfg.head_count, hd = g->cfg.head_dim;
-    uint32_t F = g->cfg.feed_forward_length;
-    const uint32_t qw = H * hd, L = g->cfg.block_count;
+    const uint32_t nqkv = (H + 2u) * hd, L = g->cfg.block_count;
     const G3Params& P = g->P;
-    _Float16* ahi = static_cast<_Float16*>(p.ahi);
-    _Float16* alo = static_cast<_Float16*>(p.alo);
+    _Float16* a = p.a;
     float* h = p.h;
     float* x = p.x;
-    float* big = p.big;
+    float* qkv = p.qkv;
     float eps = P.eps;
     G3State* st = P.st;
     if (T == 0u || T > p.max_t || static_cast<uint64_t>(p0) + T > g->cfg.context_length)
@@ -1442,19 +1231,18 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0, bool final) {
         void* args[] = {&te, &tok, &d, &es, &h};
         if (int rc = launch(reinterpret_cast<const void*>(&k_pf_embed), dim3(T), args)) return rc;
     }
-    const PfLayerW* lw = p.lw.empty() ? nullptr : p.lw.data();
-    const uint32_t s_o = pf_splits(T, d);        // split partials of the O and down projections
-    uint64_t xs = static_cast<uint64_t>(T) * d;  // one partial [T][d]
+    uint64_t xs = static_cast<uint64_t>(T) * d;  // one O / down partial [T][d]
     uint32_t s_down = 1;                         // splits of the previous block's down projection
     for (uint32_t l = 0; l < L; ++l) {
         const LayerParams& Ly = g->layers[l];
         {   // previous block's FFN output into the residual, then the attention norm
             const float* f = l ? x : nullptr;
             const float* wpost = l ? g->layers[l - 1].post_ffw : nullptr;
-            if (int rc = pf_norm(h, f, s_down, xs, wpost, Ly.attn_norm, d, eps, ahi, alo, st, l ? l - 1u : 0u, T, s, true))
+            if (int rc = pf_norm(h, f, s_down, xs, wpost, Ly.attn_norm, d, eps, a, st, l ? l - 1u : 0u, T, s, true))
                 return rc;
         }
-        if (int rc = pf_gemm(g, ahi, alo, T, d, {{Ly.wq, qw}, {Ly.wk, hd}, {Ly.wv, hd}}, lw ? &lw[l].qkv : nullptr, big, 1, s)) return rc;
+        uint32_t s_qkv = 1;
+        if (int rc = pf_project(g, l, kProjQkv, a, T, qkv, &s_qkv, s)) return rc;
         // key coordinates: the history this segment's queries can see (from kb: position 0 in a
         // global block, the window's start rounded down to 32 in a local one), then its rows
         const uint32_t window = Ly.slots >= g->cfg.context_length ? 0u : Ly.slots;
@@ -1486,7 +1274,9 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0, bool final) {
             _Float16* vhi = static_cast<_Float16*>(p.vhi);
             _Float16* vlo = static_cast<_Float16*>(p.vlo);
             uint32_t kvf = P.kv16, p0_ = p0, qo_ = qo;
-            void* args[] = {&big, &T, &H, &hd, &qn, &kn, &ct, &sn, &eps, &kc, &vc, &slots, &ahi, &alo, &khi, &klo, &vhi, &vlo,
+            uint64_t qs = static_cast<uint64_t>(T) * nqkv;
+            _Float16 *qhi = p.qhi, *qlo = p.qlo;
+            void* args[] = {&qkv, &s_qkv, &qs, &T, &H, &hd, &qn, &kn, &ct, &sn, &eps, &kc, &vc, &slots, &qhi, &qlo, &khi, &klo, &vhi, &vlo,
                             &kvf, &p0_, &qo_};
             const uint32_t waves = std::min(H + 1u, kPfQkMaxWaves);
             VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_qk), dim3(tp), dim3(64u * waves), args, 0, s));
@@ -1497,26 +1287,16 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0, bool final) {
         const bool last = l + 1u == L;
         if (last && !final) break;   // an earlier segment: the last block's keys and values are all it leaves
         const uint32_t fr = last ? 1u : T;
-        const uint64_t a0 = last ? static_cast<uint64_t>(T - 1u) * d : 0u;
-        const uint64_t aq = last ? static_cast<uint64_t>(T - 1u) * qw : 0u;
-        // the attention output replaces q (hi/lo in ahi/alo)
-        if (int rc = pf_attention(g, Ly, T, last ? (T - 1u) / 32u : 0u, ahi, alo, s, qo)) return rc;
-        uint32_t so = last ? pf_splits(1u, d) : s_o;
-        if (int rc = pf_gemm(g, ahi + aq, alo + aq, fr, qw, {{Ly.wo, d}}, lw ? &lw[l].o : nullptr, x, so, s)) return rc;
-        so = std::max(1u, std::min(so, (qw / 32u) / 2u));
-        {   // attention output into the residual, then the FFN norm (the O partials of fr rows)
-            const uint64_t xo = static_cast<uint64_t>(fr) * d;
-            if (int rc = pf_norm(h + a0, x, so, xo, Ly.post_attn, Ly.ffn_norm, d, eps, ahi + a0, alo + a0, st, Ly.index,
-                                 fr, s, true))
-                return rc;
-        }
-        // gelu(gate) * up as f16 hi/lo in `big` (the gate/up GEMM still reads ahi/alo).
-        _Float16* ghi = reinterpret_cast<_Float16*>(big);
-        _Float16* glo = ghi + static_cast<uint64_t>(fr) * F;
-        if (int rc = pf_gemm_glu(g, ahi + a0, alo + a0, fr, d, Ly.wg, Ly.wu, F, lw ? &lw[l].gu : nullptr, ghi, glo, s))
+        float* hr = last ? h + static_cast<uint64_t>(T - 1u) * d : h;
+        if (int rc = pf_attention(g, Ly, T, last ? T - 1u : 0u, s, qo)) return rc;
+        uint32_t so = 1;
+        if (int rc = pf_project(g, l, kProjO, a, fr, x, &so, s)) return rc;
+        // attention output into the residual, then the FFN norm (the O partials of fr rows)
+        if (int rc = pf_norm(hr, x, so, static_cast<uint64_t>(fr) * d, Ly.post_attn, Ly.ffn_norm, d, eps, a, st, Ly.index,
+                             fr, s, true))
             return rc;
-        s_down = std::max(1u, std::min(last ? pf_splits(1u, d) : s_o, (F / 32u) / 2u));
-        if (int rc = pf_gemm(g, ghi, glo, fr, F, {{Ly.wd, d}}, lw ? &lw[l].down : nullptr, x, s_down, s)) return rc;
+        if (int rc = pf_ffn_glu(g, l, a, fr, p.g, s)) return rc;
+        if (int rc = pf_project(g, l, kProjDown, p.g, fr, x, &s_down, s)) return rc;
     }
     if (!final) return VRT_OK;
     {   // last position: its FFN output (the split partials summed in order) and its residual
