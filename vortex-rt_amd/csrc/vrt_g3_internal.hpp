@@ -121,11 +121,10 @@ struct PfState {
     void* vhi = nullptr;    // attention values (Tp x hd), f16 high part
     void* vlo = nullptr;    //   ... and low part
     uint32_t tkv = 0;       // key coordinates of khi..vlo: max(max_t, context_length), padded
-    uint32_t qtmax = 0;     // 32-query tiles of max_t
-    uint32_t maxc = 0;      // key chunks per query tile, at most
-    float* opart = nullptr;     // [H][qtmax][maxc][32][hd] attention unit partials
-    float* mpart = nullptr;     // [H][qtmax][maxc][32] their maxima
-    double* lpart = nullptr;    // [H][qtmax][maxc][32] their exp sums
+    uint32_t parts = 0;         // attention partials: (32-query tile, head, key chunk)s
+    float* opart = nullptr;     // [parts][32 hd] their weighted values
+    float* mpart = nullptr;     // [parts][32] their maxima
+    double* lpart = nullptr;    // [parts][32] their exp sums
     std::vector<PfLayerW> lw;   // expanded weights per block (empty: the GEMMs read the Q8_0 arena)
 };
 

@@ -57,18 +57,6 @@ __device__ __forceinline__ void gm_store_c(float* c, uint32_t ldc, uint32_t N, u
         if (n + k < N) p[k] = x[k];
 }
 
-// 64 lanes x 16 (or 4) bytes from base + voff straight into LDS at lds + lane * 16 (or 4). In
-// assembly so that the waits are placed by hand: the compiler would wait for every such load in
-// flight before any LDS read.
-__device__ __forceinline__ void gm_lds16(const void* base, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :: "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void gm_lds4(const void* base, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-                 :: "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
-}
-
 // Tiles of 32 MT rows x 32 NT columns, four waves of 16 MT x 16 NT each (2 x 2). K advances one
 // Q8_0 block per step through NS LDS stages filled by direct global-to-LDS loads, NS - 1 steps
 // ahead; one barrier per step both hands over the stage that has arrived and frees the one read
@@ -326,7 +314,7 @@ static GmTile gm_tile_shape(uint32_t M, uint32_t N, uint32_t nkb, bool glu) {
     GmTile t{2u, 2u, 1u};
     if (wgs(4u, 4u) >= 512u) t = {4u, 4u, 1u};
     else if (wgs(2u, 4u) >= 256u) t = {2u, 4u, 1u};
-    if (!glu && wgs(t.mt, t.nt) <= 160u) t.splits = std::min(4u, std::max(1u, nkb / 8u));
+    if (!glu && t.nt == 2u && wgs(2u, 2u) <= kGmSplitWgs) t.splits = std::min(4u, std::max(1u, nkb / 8u));
     return t;
 }
 

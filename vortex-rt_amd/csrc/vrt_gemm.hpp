@@ -39,6 +39,18 @@ __device__ __forceinline__ void gm_split(float x, _Float16& hi, _Float16& lo) {
     lo = static_cast<_Float16>(x - static_cast<float>(hi));
 }
 
+// 64 lanes x 16 (or 4) bytes from base + voff straight into LDS at lds + lane * 16 (or 4). In
+// assembly so that the waits are placed by hand: the compiler would wait for every such load in
+// flight before any LDS read.
+__device__ __forceinline__ void gm_lds16(const void* base, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void gm_lds4(const void* base, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                 :: "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
+}
+
 struct GmArgs {
     const _Float16* a;     // activations, M rows
     const _Float16* w;     // weights, N rows
@@ -53,6 +65,8 @@ struct GmArgs {
 // C = A x W^T, or with glu (w: gate and up rows interleaved in groups of 16, 16 gate rows first)
 // gelu_tanh(gate) * up. gm_splits: the K splits that suit this shape (1: none);
 // the consumer adds the partials in split order.
+constexpr uint32_t kGmSplitWgs = 160;   // K is split up to this many 64 x 64 tiles, in four at most:
+constexpr uint64_t kGmSplitFloats = 4ull * kGmSplitWgs * 64u * 64u;   //   so many partial sums
 uint32_t gm_splits(uint32_t M, uint32_t N, uint32_t nkb);
 int gm_run(const GmArgs& G, uint32_t splits, bool glu, hipStream_t s);
 // One-time expansion of Q8_0 rows into a weight matrix: up to three matrices concatenated

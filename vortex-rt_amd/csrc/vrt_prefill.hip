@@ -16,6 +16,7 @@
 #include <cstdint>
 #include <initializer_list>
 #include <utility>
+#include <vector>
 
 #include "vrt_g3_errors.hpp"
 #include "vrt_g3_internal.hpp"
@@ -467,117 +468,127 @@ __device__ __forceinline__ uint64_t pf_vswz(uint32_t t, uint32_t d, uint32_t hd)
 
 // ---- QK-norm, RoPE, KV cache ------------------------------------------------------------
 
-// Row t of qkv = [q (H heads x hd) | k (hd) | v (hd)], the sum of nsplit partials: QK-norm per head (src/gemma3.cpp:
-// 1045-1104), NeoX RoPE at position t (:1371-1424), q as f16 hi/lo rows of qhi/qlo; then k and v go to the KV cache slot t % slots when position t is still in the
-// window after the prompt (the serial loop's eviction leaves exactly those, :1590-1600); with
-// kv16 (1 fp16, 2 bf16) the cache holds 16-bit entries and k and v are rounded to them first
-// (the attention below then sees the cached values, as the serial loop does). The attention operands as f16 hi/lo: k and
-// v in the pf_kswz / pf_vswz tile layouts. One
-// workgroup per position t < Tp: those with t >= T write the zero padding keys and values
-// (keys past the prompt are masked, and zero values keep the masked products zero).
-// One wave per head (lane l: dims l + 64 e): the sum of squares is a wave reduction and the
-// RoPE partners come through the wave's own LDS row, so the kernel has no barrier.
-constexpr uint32_t kPfQkMaxWaves = 8;
-__global__ void __launch_bounds__(kPfQkMaxWaves * 64) k_pf_qk(const float* qkv, uint32_t nsplit,
-                                                            uint64_t sstride, uint32_t T, uint32_t H, uint32_t hd,
-                                                            const float* q_norm, const float* k_norm,
-                                                            const float* cos_t, const float* sin_t, float eps,
-                                                            float* kc, float* vc, uint32_t slots, _Float16* qhi,
-                                                            _Float16* qlo, _Float16* khi, _Float16* klo, _Float16* vhi,
-                                                            _Float16* vlo, uint32_t kv16, uint32_t p0, uint32_t qo) {
-#pragma clang fp contract(off)
-    __shared__ float xs[kPfQkMaxWaves][256];
-    const uint32_t t = blockIdx.x;           // row of the segment; position p0 + t, key coordinate qo + t
-    const uint32_t kt = qo + t;
-    if (t >= T) {   // whole workgroup
-        for (uint32_t i = threadIdx.x; i < hd; i += blockDim.x) {
-            const uint64_t ko = pf_kswz(kt, i, hd), vo = pf_vswz(kt, i, hd);
-            khi[ko] = klo[ko] = vhi[vo] = vlo[vo] = static_cast<_Float16>(0.0f);
-        }
+// Four consecutive cache entries from entry i on (fp32, or 16-bit in the first half of the buffer).
+__device__ __forceinline__ void kv_store4(float* c, uint64_t i, f4 x, uint32_t kv16) {
+    if (!kv16) {
+        *reinterpret_cast<f4*>(c + i) = x;
         return;
     }
-    const uint32_t pos = p0 + t;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+    u16x4 b;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = kv16_bits(x[e], kv16);
+    *reinterpret_cast<u16x4*>(reinterpret_cast<uint16_t*>(c) + i) = b;
+}
+
+// Row t of qkv = [q (H heads x hd) | k (hd) | v (hd)], the sum of nsplit partials: QK-norm per head
+// (src/gemma3.cpp:1045-1104), NeoX RoPE at position p0 + t (:1371-1424), q as f16 hi/lo rows of
+// qhi/qlo; then k and v go to the KV cache slot of the position when it is still in the window
+// after the segment (the serial loop's eviction leaves exactly those, :1590-1600); with kv16 (1 fp16,
+// 2 bf16) the cache holds 16-bit entries and k and v are rounded to them first (the attention below
+// then sees the cached values, as the serial loop does). The attention operands as f16 hi/lo: k and
+// v in the pf_kswz / pf_vswz tile layouts. Rows t >= T write the zero padding keys and values
+// (keys past the prompt are masked, and zero values keep the masked products zero).
+// One workgroup per eight rows, one wave per row. Lane l holds the dims 4 l .. 4 l + 3 of every head
+// (hd <= 256), so loads, cache stores and operand stores are 8 to 16 bytes per lane, the sums of
+// squares are wave reductions and a RoPE partner sits hd / 8 lanes away. The values of the eight
+// rows, consecutive in the value operand, meet in LDS and leave as 16-byte stores (one row per
+// workgroup and two-byte stores: 14.4 us at 2048 rows).
+constexpr uint32_t kPfQkRows = 8;
+constexpr uint32_t kPfQkHeads = 4;   // heads in flight per wave
+__global__ void __launch_bounds__(64 * kPfQkRows) k_pf_qk(const float* qkv, uint32_t nsplit, uint64_t sstride, uint32_t T,
+                                                          uint32_t H, uint32_t hd, const float* q_norm,
+                                                          const float* k_norm, const float* cos_t, const float* sin_t,
+                                                          float eps, float* kc, float* vc, uint32_t slots, _Float16* qhi,
+                                                          _Float16* qlo, _Float16* khi, _Float16* klo, _Float16* vhi,
+                                                          _Float16* vlo, uint32_t kv16, uint32_t p0, uint32_t qo) {
+#pragma clang fp contract(off)
+    __shared__ __align__(16) float s_v[kPfQkRows][256];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t t = blockIdx.x * kPfQkRows + wave, kt = qo + t, pos = p0 + t;
     const uint32_t nqkv = (H + 2u) * hd, half = hd >> 1;
-    const float* row = qkv + static_cast<uint64_t>(t) * nqkv;
-    float* xw = xs[wave];
-    const bool keep = t + slots >= T;   // the last `slots` positions of the segment reach the ring
-    const uint64_t slot = static_cast<uint64_t>(pos % slots) * hd;
-    // Loads are issued at clamped, in-bounds indices and masked afterwards, so each group of
-    // them is in flight together (no branch, hence no wait, between them). v first: it is only
-    // stored, after the heads.
-    const uint32_t vi = min(threadIdx.x, hd - 1u);
-    // element i of the row, the split partials added in order
-    auto at = [&](uint32_t i) {
-        float v = row[i];
-        for (uint32_t z = 1; z < nsplit; ++z) v += row[z * sstride + i];
-        return v;
-    };
-    const float vr = at((H + 1u) * hd + vi);
-    uint32_t ic[4], ei[4];
-    bool live[4];
+    const uint32_t i = min(4u * lane, hd - 4u);   // this lane's dims (clamped: lanes past hd store nothing)
+    const bool live = 4u * lane < hd;
+    f4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (t < T) {   // whole wave
+        const float* row = qkv + static_cast<uint64_t>(t) * nqkv + i;
+        // four elements of the row, the split partials added in order
+        auto at = [&](uint32_t o) {
+            f4 x = *reinterpret_cast<const f4*>(row + o);
+            for (uint32_t z = 1; z < nsplit; ++z) {
+                const f4 y = *reinterpret_cast<const f4*>(row + z * sstride + o);
 #pragma unroll
-    for (uint32_t e = 0; e < 4u; ++e) {
-        live[e] = lane + 64u * e < hd;
-        ic[e] = min(lane + 64u * e, hd - 1u);
-        ei[e] = ic[e] < half ? ic[e] : ic[e] - half;
-    }
-    float cs[4], sn[4];
+                for (int e = 0; e < 4; ++e) x[e] += y[e];
+            }
+            return x;
+        };
+        const bool keep = t + slots >= T;   // the last `slots` positions of the segment reach the ring
+        const uint64_t slot = static_cast<uint64_t>(pos % slots) * hd + i;
+        const bool lower = i < half;
+        const uint32_t ri = lower ? i : i - half;
+        const f4 cs = *reinterpret_cast<const f4*>(cos_t + static_cast<uint64_t>(pos) * half + ri);
+        const f4 sn = *reinterpret_cast<const f4*>(sin_t + static_cast<uint64_t>(pos) * half + ri);
+        const f4 wq = *reinterpret_cast<const f4*>(q_norm + i), wk = *reinterpret_cast<const f4*>(k_norm + i);
+        v = at((H + 1u) * hd);
+        const uint32_t partner = lower ? lane + (hd >> 3) : lane - (hd >> 3);
+        for (uint32_t h0 = 0; h0 <= H; h0 += kPfQkHeads) {   // H query heads, then the key head
+            f4 x[kPfQkHeads];
 #pragma unroll
-    for (uint32_t e = 0; e < 4u; ++e) {
-        cs[e] = cos_t[static_cast<uint64_t>(pos) * half + ei[e]];
-        sn[e] = sin_t[static_cast<uint64_t>(pos) * half + ei[e]];
-    }
-    for (uint32_t hh = wave; hh <= H; hh += nw) {   // H query heads, then the key head
-        const float* w = hh < H ? q_norm : k_norm;
-        float v[4], wv[4];
+            for (uint32_t k = 0; k < kPfQkHeads; ++k) x[k] = at(min(h0 + k, H) * hd);
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) {
-            v[e] = at(hh * hd + ic[e]);
-            wv[e] = w[ic[e]];
-        }
-        double sq = 0.0;
+            for (uint32_t k = 0; k < kPfQkHeads; ++k) {
+                const uint32_t hh = h0 + k;
+                if (hh > H) break;
+                double sq = 0.0;
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) {
-            if (!live[e]) v[e] = 0.0f;
-            sq += static_cast<double>(v[e]) * static_cast<double>(v[e]);
-        }
-        const float sc = pf_rms_scale(wave_red_sum_d(sq), hd, eps);
+                for (int e = 0; e < 4; ++e) sq += live ? static_cast<double>(x[k][e]) * static_cast<double>(x[k][e]) : 0.0;
+                const float sc = pf_rms_scale(wave_red_sum_d(sq), hd, eps);
+                f4 y;
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e)
-            if (live[e]) xw[ic[e]] = v[e] * (sc * wv[e]);   // values *= scale * weights (src/gemma3.cpp:1097-1102)
-        // the partners are other lanes' values: a wave's LDS accesses complete in order
-        __builtin_amdgcn_wave_barrier();
+                for (int e = 0; e < 4; ++e) {   // values *= scale * weights (src/gemma3.cpp:1097-1102)
+                    const float a = x[k][e] * (sc * (hh < H ? wq[e] : wk[e]));
+                    const float b = __shfl(a, static_cast<int>(partner & 63u));
+                    y[e] = lower ? a * cs[e] - b * sn[e] : a * cs[e] + b * sn[e];
+                }
+                if (hh < H) {
+                    const uint64_t o = (static_cast<uint64_t>(t) * H + hh) * hd + i;
+                    if (live) pf_split4(y, qhi + o, qlo + o);
+                } else {   // 16-bit KV: the key as the cache holds it, for the cache and the attention
+                    if (kv16) {
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) {
-            if (!live[e]) continue;
-            const uint32_t i = ic[e];
-            const float a = xw[ei[e]], b = xw[ei[e] + half];
-            const float y2 = i < half ? a * cs[e] - b * sn[e] : b * cs[e] + a * sn[e];
-            if (hh < H) {   // the query, [T][H * hd]
-                const uint64_t o = static_cast<uint64_t>(t) * H * hd + hh * hd + i;
-                pf_split(y2, qhi + o, qlo + o);
-            } else {   // 16-bit KV: the key as the cache holds it, for the cache and the attention
-                const float kk = kv16 ? kv16_float(kv16_bits(y2, kv16), kv16) : y2;
-                const uint64_t o = pf_kswz(kt, i, hd);
-                pf_split(kk, khi + o, klo + o);
-                if (keep) {
-                    if (kv16) reinterpret_cast<uint16_t*>(kc)[slot + i] = kv16_bits(kk, kv16);
-                    else kc[slot + i] = kk;
+                        for (int e = 0; e < 4; ++e) y[e] = kv16_float(kv16_bits(y[e], kv16), kv16);
+                    }
+                    const uint64_t o = pf_kswz(kt, i, hd);
+                    if (live) {
+                        pf_split4(y, khi + o, klo + o);
+                        if (keep) kv_store4(kc, slot, y, kv16);
+                    }
                 }
             }
         }
-        __builtin_amdgcn_wave_barrier();   // this head's reads of xw come before the next head's writes
-    }
-    for (uint32_t i = threadIdx.x; i < hd; i += blockDim.x) {   // v is not normed
-        const float vv0 = i == vi ? vr : at((H + 1u) * hd + i);
-        const float vv = kv16 ? kv16_float(kv16_bits(vv0, kv16), kv16) : vv0;
-        if (keep) {
-            if (kv16) reinterpret_cast<uint16_t*>(vc)[slot + i] = kv16_bits(vv, kv16);
-            else vc[slot + i] = vv;
+        if (kv16) {   // v is not normed
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = kv16_float(kv16_bits(v[e], kv16), kv16);
         }
-        const uint64_t o = pf_vswz(kt, i, hd);
-        pf_split(vv, vhi + o, vlo + o);
+        if (live && keep) kv_store4(vc, slot, v, kv16);
+    } else if (live) {
+        const uint64_t o = pf_kswz(kt, i, hd);
+        pf_split4(v, khi + o, klo + o);
+    }
+    if (live) *reinterpret_cast<f4*>(&s_v[wave][i]) = v;
+    __syncthreads();
+    for (uint32_t d = threadIdx.x; d < hd; d += 64u * kPfQkRows) {   // qo is a multiple of 32: eight keys of one run
+        half8 hi, lo;
+#pragma unroll
+        for (uint32_t r = 0; r < kPfQkRows; ++r) {
+            _Float16 a, b;
+            gm_split(s_v[r][d], a, b);
+            hi[r] = a;
+            lo[r] = b;
+        }
+        const uint64_t o = pf_vswz(kt - wave, d, hd);
+        *reinterpret_cast<half8*>(vhi + o) = hi;
+        *reinterpret_cast<half8*>(vlo + o) = lo;
     }
 }
 
@@ -602,27 +613,32 @@ __global__ void __launch_bounds__(kPfThreads) k_pf_kv_hist(const float* kc, cons
 
 // ---- causal attention ----------------------------------------------------------------------
 
-// One unit per (key chunk c, query tile i, head h): queries q0 = 32 i .. q0 + 31 of head h
-// against the keys of chunk c (A.kc keys, a multiple of 32) of the tile's key range [ks, ke)
-// in key coordinates (a segment's history first, its rows from A.qo: the tile's first query
-// sits at qk0 = A.qo + q0; ke = min(A.qo + T, qk0 + 32); ks = 0, or with a local window the
-// window's start for qk0, rounded down to 32). The four waves split the head dimension: wave w owns the k steps s = w mod 4 of
-// S^T = K Q^T and the d tiles dt = w mod 4 of O^T. Per 32-key tile, with lane l on query
-// q0 + l % 32: each wave's partial S^T (three f16 products of the hi/lo parts) goes through LDS
-// and every wave sums the four in wave order (the same scores in every wave), masks (key <= qk,
-// inside the window, key < ke) and scales them and runs the online softmax in base 2 (the
-// scale times log2 e, v_exp_f32): running max m, e_j = 2^(v_j - m), each tile's sum of e_j in
-// fp32 added to a running sum in double, its O^T tiles rescaled when m grows and O^T += V^T E^T
-// (V^T and E^T as hi/lo). The next tile's operands load during the current one.
-// A tile whose key range is one chunk is finished here (out = O / sum as f16 hi/lo into the
-// queries' own columns, which only this unit reads); otherwise the chunk's partial goes to
-// opart/mpart/lpart and k_pf_attn_merge combines them in the next launch. Same result as the
-// masked softmax of src/gemma3.cpp:1602-1696 over the full row up to the rounding of the
-// rescaling; a softmax sum that is not > 0 and finite flags the block.
+// The pairs (query tile i of 32 rows, head h), numbered i H + h, are dealt in groups of four to
+// workgroups, one pair per wave; a group's key range [ks, ke) is the union of its tiles' (one tile's
+// when H is a multiple of four), cut into chunks of A.kc keys, one workgroup each. In key
+// coordinates (a segment's history first, its rows from A.qo) tile i's first query sits at
+// qk0 = A.qo + 32 i; it sees the keys from the window's start for qk0, rounded down to 32, up to
+// min(A.qo + T, qk0 + 32).
+// All four waves read the same keys and values: a 32-key tile of both (64 KB at hd 256 with low
+// parts) is loaded straight to LDS during the previous tile's work, one barrier per tile. A wave keeps
+// its queries and its O^T in registers (one wave per SIMD). Per tile, lane l on query l % 32: S^T = K Q^T (three
+// f16 products of the hi/lo parts), mask, softmax in base 2 (the scale times log2 e, v_exp_f32) and
+// O^T += V^T E^T (V and E as hi/lo). The running maximum m moves, and O^T is rescaled, only when a
+// tile's scores exceed it by more than 2^kPfAttSlack for some query: e_j = 2^(v_j - m) then stays
+// below 2^kPfAttSlack, exact in the same relative precision. Each tile's sum of e_j in fp32 is added
+// to a running sum in double.
+// LO false: a 16-bit KV cache, whose entries are exact in f16, so the low parts of K and V are zero
+// and their products are left out.
+// A group whose range is one chunk is finished here (out = O / sum into the activation buffer);
+// otherwise the pairs' partials go to opart/mpart/lpart, in register order, and k_pf_attn_merge
+// combines them in the next launch. Same result as the masked softmax of src/gemma3.cpp:1602-1696
+// over the full row up to rounding; a softmax sum that is not > 0 and finite flags the block.
 // MFMA operand layouts (v_mfma_f32_32x32x16_f16): lane l gives A[m = l % 32][k = 8 (l / 32) + j]
 // and B[k = 8 (l / 32) + j][n = l % 32], j < 8; result r of lane l is C[8 (r / 4) + 4 (l / 32) +
 // r % 4][l % 32].
-constexpr uint32_t kPfAttKC = 128;   // keys per attention chunk (a multiple of 32)
+constexpr uint32_t kPfAttPairs = 4;        // pairs per workgroup (waves)
+constexpr uint32_t kPfAttParts = 8192;     // partials kept, at least
+constexpr float kPfAttSlack = 8.0f;
 struct PfAttn {
     const _Float16* qhi;   // [T][H * hd] queries, normed and rotated
     const _Float16* qlo;
@@ -632,303 +648,272 @@ struct PfAttn {
     const _Float16* vlo;
     _Float16* o;           // output, an activation buffer of H * hd columns: row q - o_row of query row q
     uint32_t o_row;        //   (earlier query rows of the first tile are not written)
-    float* opart;          // [H][qtmax][maxc][32][hd] chunk partials, sum_j e_j v_j
-    float* mpart;          // [H][qtmax][maxc][32] their maxima (base 2)
-    double* lpart;         // [H][qtmax][maxc][32] their sums of e_j
+    float* opart;          // [pairs][nch][32 hd] chunk partials sum_j e_j v_j (pairs of the launch)
+    float* mpart;          // [pairs][nch][32] their maxima (base 2)
+    double* lpart;         // [pairs][nch][32] their sums of e_j
     G3State* st;
-    uint32_t T, H, window, qtmax, maxc, block, kc;
-    uint32_t qt0;          // first query tile of the launch (blockIdx.y, merge: blockIdx.x, counts from it)
+    uint32_t T, H, window, block;
+    uint32_t kc, nch;      // keys per chunk (a multiple of 32), chunks of the longest range
+    uint32_t pair0, pairs, groups;   // first pair of the launch, pairs and groups of four from it
     uint32_t qo;           // key coordinate of query row 0 (keys before it: an earlier segment's history)
     float scale2;          // attention scale times log2(e): the scores in base 2
 };
 
-// Key range [ks, ke) of the query tile whose first row sits at key coordinate qk0, with keys
-// below kend (the key coordinates of a segment's history come first, then its own rows).
-__device__ __forceinline__ void pf_att_range(uint32_t qk0, uint32_t kend, uint32_t window, uint32_t& ks, uint32_t& ke) {
-    ke = min(kend, qk0 + 32u);
-    ks = window != 0u && qk0 + 1u > window ? (qk0 + 1u - window) & ~31u : 0u;
+// Key range [ks, ke) of the query tiles i0..i1 (key coordinates, 32 rows each).
+__host__ __device__ __forceinline__ void pf_att_range(uint32_t qo, uint32_t T, uint32_t window, uint32_t i0, uint32_t i1,
+                                                      uint32_t& ks, uint32_t& ke) {
+    const uint32_t q0 = qo + 32u * i0, q1 = qo + 32u * i1 + 32u;
+    ke = q1 < qo + T ? q1 : qo + T;
+    ks = window != 0u && q0 + 1u > window ? (q0 + 1u - window) & ~31u : 0u;
+}
+// ... of group g (four pairs from pair0 + 4 g).
+__host__ __device__ __forceinline__ void pf_att_group(const PfAttn& A, uint32_t g, uint32_t& ks, uint32_t& ke) {
+    const uint32_t a = A.pair0 + kPfAttPairs * g, last = A.pair0 + A.pairs - 1u;
+    const uint32_t b = a + kPfAttPairs - 1u < last ? a + kPfAttPairs - 1u : last;
+    pf_att_range(A.qo, A.T, A.window, a / A.H, b / A.H, ks, ke);
 }
 
-template <uint32_t HD>
-__global__ void __launch_bounds__(256) k_pf_attn(PfAttn A) {
+template <uint32_t HD, bool LO>
+__global__ void __launch_bounds__(256, 1) k_pf_attn(PfAttn A) {
 #pragma clang fp contract(off)
     constexpr uint32_t KS = HD / 16u;               // k steps of S^T
     constexpr uint32_t DT = HD / 32u;               // d tiles of O^T
-    constexpr uint32_t KW = (KS + 3u) / 4u;         // k steps per wave (at most)
-    constexpr uint32_t DW = (DT + 3u) / 4u;         // d tiles per wave (at most)
-    __shared__ __align__(16) float s_s[2][4][16 * 64];   // partial S^T per wave, double-buffered
-    // Workgroup b of the launch runs on XCD b % 8: each XCD takes a contiguous eighth of the
-    // (query tile, chunk, head) units, heads innermost, so the units that read one chunk's keys
-    // and values (the heads share them) run together on one XCD and its L2 (-1.6% on an
-    // 8192-token prefill, unchanged at 512).
-    uint32_t c, i, h;
+    constexpr uint32_t NP = LO ? 2u : 1u;           // parts of K and V
+    constexpr uint32_t UK = NP * KS, UV = NP * 2u * DT;   // 1 KB operand units of a key tile: K, V
+    constexpr uint32_t UW = (UK + UV) / 4u;         // units per wave (HD is a multiple of 32)
+    __shared__ __align__(1024) unsigned char s_kv[2][(UK + UV) * 1024u];
+    // Windowed ranges: workgroup b runs on XCD b % 8 and each XCD takes a contiguous eighth of the
+    // (group, chunk) units, so neighbouring groups share their keys in one L2. Full ranges: chunk by
+    // chunk, the groups in falling order of length, so every XCD works on the same chunk.
+    uint32_t c, g;
     {
-        const uint32_t nx = gridDim.x, ny = gridDim.y, nz = gridDim.z, N = nx * ny * nz;
-        uint32_t b = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
-        if ((N & 7u) == 0u) b = (b & 7u) * (N >> 3) + (b >> 3);
-        h = b % nz;
-        const uint32_t r = b / nz;
-        c = r % nx;
-        i = A.qt0 + r / nx;
+        const uint32_t N = gridDim.x;
+        uint32_t b = blockIdx.x;
+        if (A.window != 0u) {
+            if ((N & 7u) == 0u) b = (b & 7u) * (N >> 3) + (b >> 3);
+            g = b / A.nch;
+            c = b - g * A.nch;
+        } else {
+            c = b / A.groups;
+            g = A.groups - 1u - (b - c * A.groups);
+        }
     }
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, l32 = lane & 31u, hf = lane >> 5;
-    const uint32_t T = A.T, q0 = 32u * i, qw = A.H * HD;
-    const uint32_t qk0 = A.qo + q0;   // the tile's first query in key coordinates
     uint32_t ks, ke;
-    pf_att_range(qk0, A.qo + T, A.window, ks, ke);
+    pf_att_group(A, g, ks, ke);
     const uint32_t nch = (ke - ks + A.kc - 1u) / A.kc;
     if (c >= nch) return;   // whole workgroup
     const uint32_t k0 = ks + c * A.kc, k1 = min(ke, k0 + A.kc);
-    const uint32_t q = q0 + l32, qk = qk0 + l32;   // this lane's query: row, key coordinate
-    // this wave's k steps of the queries (B operand of S^T), rows past T clamped (never written)
-    v4u qb[KW][2];
-    {
-        const uint64_t qo = static_cast<uint64_t>(min(q, T - 1u)) * qw + h * HD + 8u * hf;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t l32 = lane & 31u, hf = lane >> 5;
+    const uint32_t rel = kPfAttPairs * g + wave;            // pair of the launch (its partials' index)
+    const bool mine = rel < A.pairs;                        // the last group may be short; every wave loads
+    const uint32_t pair = A.pair0 + (mine ? rel : A.pairs - 1u), i = pair / A.H, h = pair - i * A.H;
+    const uint32_t T = A.T, qw = A.H * HD;
+    const uint32_t q = 32u * i + l32, qk0 = A.qo + 32u * i, qk = qk0 + l32;   // this lane's query: row, key coordinate
+    // this wave's loads of a key tile: units u = wave UW + j; a tile advances every part by 64 HD bytes
+    const char* src[UW];
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+        (__attribute__((address_space(3))) unsigned char*)&s_kv[0][0]));
 #pragma unroll
-        for (uint32_t j = 0; j < KW; ++j) {
-            const uint32_t k = min(wave + 4u * j, KS - 1u);
-            qb[j][0] = *reinterpret_cast<const v4u*>(A.qhi + qo + 16u * k);
-            qb[j][1] = *reinterpret_cast<const v4u*>(A.qlo + qo + 16u * k);
+    for (uint32_t j = 0; j < UW; ++j) {
+        const uint32_t u = wave * UW + j;
+        const _Float16* part = u < UK ? (u < KS ? A.khi : A.klo) : (u - UK < 2u * DT ? A.vhi : A.vlo);
+        const uint32_t idx = u < UK ? u % KS : (u - UK) % (2u * DT);
+        src[j] = reinterpret_cast<const char*>(part) + static_cast<uint64_t>(k0 >> 5) * (64u * HD) + idx * 1024u;
+    }
+    auto issue = [&](uint32_t buf) {
+#pragma unroll
+        for (uint32_t j = 0; j < UW; ++j) {
+            gm_lds16(src[j], lane * 16u, lds0 + buf * ((UK + UV) * 1024u) + (wave * UW + j) * 1024u);
+            src[j] += 64u * HD;
+        }
+    };
+    issue(0u);
+    // the queries (B operand of S^T), rows past T clamped (never written)
+    half8 qb[KS][2];
+    {
+        const uint64_t o = static_cast<uint64_t>(min(q, T - 1u)) * qw + h * HD + 8u * hf;
+#pragma unroll
+        for (uint32_t k = 0; k < KS; ++k) {
+            qb[k][0] = *reinterpret_cast<const half8*>(A.qhi + o + 16u * k);
+            qb[k][1] = *reinterpret_cast<const half8*>(A.qlo + o + 16u * k);
         }
     }
-    // the operands of one 32-key tile for this wave
-    struct Ops {
-        v4u k[KW][2];       // [k step][hi, lo]
-        v4u v[DW][2][2];    // [d tile][k step][hi, lo]
-    };
-    auto load = [&](uint32_t kt, Ops& R) {
-        const uint64_t tile = kt >> 5;
-#pragma unroll
-        for (uint32_t j = 0; j < KW; ++j) {
-            const uint32_t k = min(wave + 4u * j, KS - 1u);
-            const uint64_t o = (tile * KS + k) * 512u + 8u * lane;
-            R.k[j][0] = *reinterpret_cast<const v4u*>(A.khi + o);
-            R.k[j][1] = *reinterpret_cast<const v4u*>(A.klo + o);
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < DW; ++j) {
-            const uint32_t dt = min(wave + 4u * j, DT - 1u);
-#pragma unroll
-            for (uint32_t sk = 0; sk < 2u; ++sk) {
-                const uint64_t o = ((tile * DT + dt) * 2u + sk) * 512u + 8u * lane;
-                R.v[j][sk][0] = *reinterpret_cast<const v4u*>(A.vhi + o);
-                R.v[j][sk][1] = *reinterpret_cast<const v4u*>(A.vlo + o);
-            }
-        }
-    };
-    float m = -INFINITY;   // running maximum of the scaled scores of query q
+    float m = -INFINITY;   // reference maximum of the scaled scores of query q
     double lsum = 0.0;     // this lane's share of sum_j e_j
-    float16v o[DW];        // O^T tiles of this wave: d = 32 dt + 8 (r / 4) + 4 hf + r % 4, query q
+    float16v o[DT];        // O^T tiles: d = 32 dt + 8 (r / 4) + 4 hf + r % 4, query q
 #pragma unroll
-    for (uint32_t j = 0; j < DW; ++j) o[j] = float16v{};
-    // one 32-key tile: partial S^T, exchange, online softmax, O^T update (operands in R)
+    for (uint32_t j = 0; j < DT; ++j) o[j] = float16v{};
     uint32_t buf = 0;
-    auto step = [&](uint32_t kt, const Ops& R) {
-        float16v sp = {};
+    for (uint32_t kt = k0; kt < k1; kt += 32u, buf ^= 1u) {
+        // this tile has arrived, and every wave is done with the other buffer
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (kt + 32u < k1) issue(buf ^ 1u);
+        const unsigned char* pk = &s_kv[buf][lane * 16u];
+        const unsigned char* pv = pk + UK * 1024u;
+        float16v sa = {}, sb = {};   // two chains
 #pragma unroll
-        for (uint32_t j = 0; j < KW; ++j) {
-            if (wave + 4u * j >= KS) continue;
-            const half8 ah = __builtin_bit_cast(half8, R.k[j][0]), al = __builtin_bit_cast(half8, R.k[j][1]);
-            const half8 bh = __builtin_bit_cast(half8, qb[j][0]), bl = __builtin_bit_cast(half8, qb[j][1]);
-            sp = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, sp, 0, 0, 0);
-            sp = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, sp, 0, 0, 0);
-            sp = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, sp, 0, 0, 0);
-        }
-        // the four partials through LDS (buffer buf was last read two tiles ago, before the
-        // barrier of the previous tile)
-#pragma unroll
-        for (uint32_t rq = 0; rq < 4u; ++rq)
-            *reinterpret_cast<f4*>(&s_s[buf][wave][(rq * 64u + lane) * 4u]) =
-                f4{sp[4 * rq], sp[4 * rq + 1], sp[4 * rq + 2], sp[4 * rq + 3]};
-        __syncthreads();
-        float v[16];
-#pragma unroll
-        for (uint32_t rq = 0; rq < 4u; ++rq) {
-            f4 t = *reinterpret_cast<const f4*>(&s_s[buf][0][(rq * 64u + lane) * 4u]);
-#pragma unroll
-            for (uint32_t w = 1; w < 4u; ++w) {
-                const f4 u = *reinterpret_cast<const f4*>(&s_s[buf][w][(rq * 64u + lane) * 4u]);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) t[e] += u[e];
+        for (uint32_t k = 0; k < KS; ++k) {
+            const half8 ah = *reinterpret_cast<const half8*>(pk + k * 1024u);
+            float16v& s0 = (k & 1u) ? sb : sa;
+            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, qb[k][0], s0, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, qb[k][1], s0, 0, 0, 0);
+            if constexpr (LO) {
+                const half8 al = *reinterpret_cast<const half8*>(pk + (KS + k) * 1024u);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, qb[k][0], s0, 0, 0, 0);
             }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[4 * rq + e] = t[e];
         }
-        buf ^= 1u;
         // scores in base 2 (scale * log2 e folded in): e_j = 2^(v_j - m) = exp(scale s_j - m ln 2)
+        float v[16];
         float tmax = -INFINITY;
-        if (kt + 31u < k1 && kt + 31u <= qk0 && (A.window == 0u || kt + A.window > qk0 + 31u)) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {   // every key of the tile visible to every query
-                v[r] *= A.scale2;
-                tmax = fmaxf(tmax, v[r]);
-            }
-        } else {
+        for (int r = 0; r < 16; ++r) v[r] = (sa[r] + sb[r]) * A.scale2;
+        if (!(kt + 31u < k1 && kt + 31u <= qk0 && (A.window == 0u || kt + A.window > qk0 + 31u))) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
+            for (int r = 0; r < 16; ++r) {   // some key of the tile is hidden from some query
                 const uint32_t key = kt + 16u * (r / 8) + 8u * hf + (r % 8);
                 const bool ok = key < k1 && key <= qk && (A.window == 0u || key + A.window > qk);
-                v[r] = ok ? v[r] * A.scale2 : -INFINITY;
-                tmax = fmaxf(tmax, v[r]);
+                v[r] = ok ? v[r] : -INFINITY;
             }
         }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float mn = fmaxf(m, tmax);
-        const float base = mn == -INFINITY ? 0.0f : mn;   // nothing visible yet: every e_j is 0
-        const float alpha = __builtin_amdgcn_exp2f(m - base);
-        float e[16];
-        float es = 0.0f;   // the tile's share in fp32, then into the double sum
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            e[r] = __builtin_amdgcn_exp2f(v[r] - base);
-            es += e[r];
+        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, v[r]);
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+        if (__any(tmax > m + kPfAttSlack)) {   // whole wave; a query with nothing visible yet has m = -inf
+            const float mn = fmaxf(m, tmax);
+            const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            m = mn;
+            lsum *= static_cast<double>(alpha);
+#pragma unroll
+            for (uint32_t j = 0; j < DT; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
         }
-        lsum = lsum * static_cast<double>(alpha) + static_cast<double>(es);
-        m = mn;
+        const float base = m == -INFINITY ? 0.0f : m;   // nothing visible yet: every e_j is 0
+        float es = 0.0f;   // the tile's share in fp32, then into the double sum
         half8 eh[2], el[2];
 #pragma unroll
-        for (int sk = 0; sk < 2; ++sk)
+        for (int r = 0; r < 16; ++r) {
+            const float e = __builtin_amdgcn_exp2f(v[r] - base);
+            es += e;
+            eh[r / 8][r % 8] = static_cast<_Float16>(e);
+            el[r / 8][r % 8] = static_cast<_Float16>(e - static_cast<float>(eh[r / 8][r % 8]));
+        }
+        lsum += static_cast<double>(es);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float x = e[8 * sk + j];
-                eh[sk][j] = static_cast<_Float16>(x);
-                el[sk][j] = static_cast<_Float16>(x - static_cast<float>(eh[sk][j]));
-            }
-#pragma unroll
-        for (uint32_t j = 0; j < DW; ++j) {
-            if (wave + 4u * j >= DT) continue;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
+        for (uint32_t j = 0; j < DT; ++j)
 #pragma unroll
             for (uint32_t sk = 0; sk < 2u; ++sk) {
-                const half8 avh = __builtin_bit_cast(half8, R.v[j][sk][0]);
-                const half8 avl = __builtin_bit_cast(half8, R.v[j][sk][1]);
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(avh, eh[sk], o[j], 0, 0, 0);
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(avl, eh[sk], o[j], 0, 0, 0);
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(avh, el[sk], o[j], 0, 0, 0);
+                const half8 vh = *reinterpret_cast<const half8*>(pv + (2u * j + sk) * 1024u);
+                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, eh[sk], o[j], 0, 0, 0);
+                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, el[sk], o[j], 0, 0, 0);
+                if constexpr (LO) {
+                    const half8 vl = *reinterpret_cast<const half8*>(pv + (2u * (DT + j) + sk) * 1024u);
+                    o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, eh[sk], o[j], 0, 0, 0);
+                }
             }
-        }
-    };
-    // two operand sets in turn, the next tile's loads in flight during the current tile
-    Ops ra, rb;
-    load(k0, ra);
-    for (uint32_t kt = k0; kt < k1; kt += 64u) {
-        if (kt + 32u < k1) load(kt + 32u, rb);
-        step(kt, ra);
-        if (kt + 32u >= k1) break;
-        if (kt + 64u < k1) load(kt + 64u, ra);
-        step(kt + 32u, rb);
     }
+    if (!mine) return;
     lsum += __shfl_xor(lsum, 32);   // both lane halves now hold query q's sum
-    const uint64_t unit = (static_cast<uint64_t>(h) * A.qtmax + i) * A.maxc + c;
     if (nch == 1u) {   // the whole key range: normalise and write the output rows
         if (q >= T || q < A.o_row) return;
         const double den = lsum;
-        if (wave == 0u && hf == 0u && (!(den > 0.0) || !__builtin_isfinite(den)))   // :1666-1670
+        if (hf == 0u && (!(den > 0.0) || !__builtin_isfinite(den)))   // :1666-1670
             atomicMin(&A.st->nonfinite, g3_code_softmax(A.block));
         const float inv = static_cast<float>(1.0 / den);
 #pragma unroll
-        for (uint32_t j = 0; j < DW; ++j) {
-            if (wave + 4u * j >= DT) continue;
+        for (uint32_t j = 0; j < DT; ++j)
 #pragma unroll
             for (uint32_t rq = 0; rq < 4u; ++rq) {
-                const uint64_t oo = gm_off(q - A.o_row, h * HD + 32u * (wave + 4u * j) + 8u * rq + 4u * hf, qw / 32u);
+                const uint64_t oo = gm_off(q - A.o_row, h * HD + 32u * j + 8u * rq + 4u * hf, qw / 32u);
                 pf_split4(f4{o[j][4 * rq] * inv, o[j][4 * rq + 1] * inv, o[j][4 * rq + 2] * inv, o[j][4 * rq + 3] * inv},
                           A.o + oo, A.o + oo + kGmLo);
             }
-        }
         return;
     }
-    float* op = A.opart + unit * 32u * HD + static_cast<uint64_t>(l32) * HD;
+    const uint64_t unit = static_cast<uint64_t>(rel) * A.nch + c;
+    float* op = A.opart + unit * 32u * HD + lane * 4u;
 #pragma unroll
-    for (uint32_t j = 0; j < DW; ++j) {
-        if (wave + 4u * j >= DT) continue;
+    for (uint32_t j = 0; j < DT; ++j)
 #pragma unroll
         for (uint32_t rq = 0; rq < 4u; ++rq)
-            *reinterpret_cast<f4*>(op + 32u * (wave + 4u * j) + 8u * rq + 4u * hf) =
-                f4{o[j][4 * rq], o[j][4 * rq + 1], o[j][4 * rq + 2], o[j][4 * rq + 3]};
-    }
-    if (wave == 0u && hf == 0u) {
+            *reinterpret_cast<f4*>(op + (4u * j + rq) * 256u) = f4{o[j][4 * rq], o[j][4 * rq + 1], o[j][4 * rq + 2], o[j][4 * rq + 3]};
+    if (hf == 0u) {
         A.mpart[unit * 32u + l32] = m;
         A.lpart[unit * 32u + l32] = lsum;
     }
 }
 
-// Column groups of a merge workgroup's head: 4, 2 or 1 (whole float4 runs per thread).
-template <uint32_t HD>
-constexpr uint32_t pf_merge_groups() {
-    return (HD / 32u) % 4u == 0u ? 4u : ((HD / 32u) % 2u == 0u ? 2u : 1u);
-}
-
-// Merge of the chunk partials of the query tiles k_pf_attn split (one workgroup per (tile, head,
-// column group); tiles of one chunk were finished by k_pf_attn): thread t on row r = t / 8 and
-// the eighth t % 8 of the group's columns; in chunk order, with M the running maximum of the
-// chunk maxima m_c, den = sum_c exp(m_c - M) sum_c (double), out = sum_c exp(m_c - M) O_c / den
-// as f16 hi/lo into the queries' columns.
+// Merge of the chunk partials of the groups that k_pf_attn split (one wave per (pair, d tile); pairs
+// of one-chunk groups were finished there): lane l on query l % 32, its 16 values of the d tile as
+// k_pf_attn held them; in chunk order, with M the running maximum of the chunk maxima m_c, den =
+// sum_c 2^(m_c - M) sum_c (double), out = sum_c 2^(m_c - M) O_c / den into the activation buffer.
 template <uint32_t HD>
 __global__ void __launch_bounds__(256) k_pf_attn_merge(PfAttn A) {
 #pragma clang fp contract(off)
-    constexpr uint32_t CG = pf_merge_groups<HD>();
-    constexpr uint32_t NF = HD / 32u / CG;   // float4 per thread
-    const uint32_t i = A.qt0 + blockIdx.x, h = blockIdx.y, T = A.T, q0 = 32u * i;
+    const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, hf = lane >> 5;
+    const uint32_t rel = blockIdx.x, j = blockIdx.y * 4u + (threadIdx.x >> 6);
+    if (j >= HD / 32u) return;   // whole wave
     uint32_t ks, ke;
-    pf_att_range(A.qo + q0, A.qo + T, A.window, ks, ke);
+    pf_att_group(A, rel / kPfAttPairs, ks, ke);
     const uint32_t nch = (ke - ks + A.kc - 1u) / A.kc;
-    const uint32_t r = threadIdx.x >> 3, g = blockIdx.z * 8u + (threadIdx.x & 7u);
-    if (nch == 1u || q0 + r >= T || q0 + r < A.o_row) return;
-    const uint64_t unit0 = (static_cast<uint64_t>(h) * A.qtmax + i) * A.maxc;
+    const uint32_t pair = A.pair0 + rel, i = pair / A.H, h = pair - i * A.H, q = 32u * i + l32;
+    if (nch == 1u) return;   // whole wave
+    const uint64_t unit0 = static_cast<uint64_t>(rel) * A.nch;
     // chunks in groups of kG, every load of a group issued together (indices clamped to the last
     // chunk; the clamped duplicates are not used): one round of loads for up to kG chunks
     constexpr uint32_t kG = 4;
     double den = 0.0;
-    f4 acc[NF];
+    f4 acc[4];
 #pragma unroll
-    for (uint32_t k = 0; k < NF; ++k) acc[k] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t k = 0; k < 4u; ++k) acc[k] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     float M = -INFINITY;
     for (uint32_t c0 = 0; c0 < nch; c0 += kG) {
         float mv[kG];
         double lv[kG];
-        f4 x[kG][NF];
+        f4 x[kG][4];
 #pragma unroll
-        for (uint32_t j = 0; j < kG; ++j) {
-            const uint64_t u = unit0 + min(c0 + j, nch - 1u);
-            mv[j] = A.mpart[u * 32u + r];
-            lv[j] = A.lpart[u * 32u + r];
-            const float* src = A.opart + (u * 32u + r) * HD + g * (4u * NF);
+        for (uint32_t k = 0; k < kG; ++k) {
+            const uint64_t u = unit0 + min(c0 + k, nch - 1u);
+            mv[k] = A.mpart[u * 32u + l32];
+            lv[k] = A.lpart[u * 32u + l32];
+            const float* src = A.opart + u * 32u * HD + j * 1024u + lane * 4u;
 #pragma unroll
-            for (uint32_t k = 0; k < NF; ++k) x[j][k] = *reinterpret_cast<const f4*>(src + 4u * k);
+            for (uint32_t rq = 0; rq < 4u; ++rq) x[k][rq] = *reinterpret_cast<const f4*>(src + rq * 256u);
         }
         __builtin_amdgcn_sched_barrier(0);   // the group's loads stay ahead of their first use
         // running merge: the group's maximum rescales what is accumulated so far
         float Mg = M;
 #pragma unroll
-        for (uint32_t j = 0; j < kG; ++j)
-            if (c0 + j < nch) Mg = fmaxf(Mg, mv[j]);
+        for (uint32_t k = 0; k < kG; ++k)
+            if (c0 + k < nch) Mg = fmaxf(Mg, mv[k]);
         const float fo = M == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(M - Mg);
         den *= static_cast<double>(fo);
 #pragma unroll
-        for (uint32_t k = 0; k < NF; ++k)
+        for (uint32_t rq = 0; rq < 4u; ++rq)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[k][e] *= fo;
+            for (int e = 0; e < 4; ++e) acc[rq][e] *= fo;
         M = Mg;
 #pragma unroll
-        for (uint32_t j = 0; j < kG; ++j) {
-            if (c0 + j >= nch) break;
-            const float f = __builtin_amdgcn_exp2f(mv[j] - M);
-            den += lv[j] * static_cast<double>(f);
+        for (uint32_t k = 0; k < kG; ++k) {
+            if (c0 + k >= nch) break;
+            // a chunk with no key that this query sees has m_c = -inf and weight 0
+            const float f = mv[k] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mv[k] - M);
+            den += lv[k] * static_cast<double>(f);
 #pragma unroll
-            for (uint32_t k = 0; k < NF; ++k)
+            for (uint32_t rq = 0; rq < 4u; ++rq)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[k][e] += f * x[j][k][e];
+                for (int e = 0; e < 4; ++e) acc[rq][e] += f * x[k][rq][e];
         }
     }
-    if (g == 0u && (!(den > 0.0) || !__builtin_isfinite(den)))   // :1666-1670
+    if (q >= A.T || q < A.o_row) return;
+    if (j == 0u && hf == 0u && (!(den > 0.0) || !__builtin_isfinite(den)))   // :1666-1670
         atomicMin(&A.st->nonfinite, g3_code_softmax(A.block));
     const float inv = static_cast<float>(1.0 / den);
 #pragma unroll
-    for (uint32_t k = 0; k < NF; ++k) {
-        const uint64_t oo = gm_off(q0 + r - A.o_row, h * HD + g * (4u * NF) + 4u * k, A.H * HD / 32u);
-        pf_split4(f4{acc[k][0] * inv, acc[k][1] * inv, acc[k][2] * inv, acc[k][3] * inv}, A.o + oo, A.o + oo + kGmLo);
+    for (uint32_t rq = 0; rq < 4u; ++rq) {
+        const uint64_t oo = gm_off(q - A.o_row, h * HD + 32u * j + 8u * rq + 4u * hf, A.H * HD / 32u);
+        pf_split4(f4{acc[rq][0] * inv, acc[rq][1] * inv, acc[rq][2] * inv, acc[rq][3] * inv}, A.o + oo, A.o + oo + kGmLo);
     }
 }
 
@@ -1076,13 +1061,14 @@ int pf_setup(vrt_g3* g, uint32_t max_t) {
     void* q;
     if (int rc = take(static_cast<size_t>(max_t) * d * 4u, &q)) return rc;
     p.h = static_cast<float*>(q);
-    if (int rc = take(static_cast<size_t>(max_t) * d * 4u * kPfMaxSplits, &q)) return rc;
+    // K splits only while their partials are few (gm_splits, pf_splits_q8)
+    if (int rc = take(std::max<size_t>(static_cast<size_t>(max_t) * d, kGmSplitFloats) * 4u, &q)) return rc;
     p.x = static_cast<float*>(q);
     if (int rc = take(gm_size(max_t, std::max(d, qw)) * 2u, &q)) return rc;
     p.a = static_cast<_Float16*>(q);
     if (int rc = take(gm_size(max_t, F) * 2u, &q)) return rc;
     p.g = static_cast<_Float16*>(q);
-    if (int rc = take(static_cast<size_t>(max_t) * nqkv * 4u * kPfMaxSplits, &q)) return rc;
+    if (int rc = take(std::max<size_t>(static_cast<size_t>(max_t) * nqkv, kGmSplitFloats) * 4u, &q)) return rc;
     p.qkv = static_cast<float*>(q);
     if (int rc = take(static_cast<size_t>(max_t) * qw * 2u, &q)) return rc;
     p.qhi = static_cast<_Float16*>(q);
@@ -1094,14 +1080,12 @@ int pf_setup(vrt_g3* g, uint32_t max_t) {
     void** kv[] = {&p.khi, &p.klo, &p.vhi, &p.vlo};
     for (void** b : kv)
         if (int rc = take(static_cast<size_t>(hd) * p.tkv * 2u, b)) return rc;
-    p.qtmax = (max_t + 31u) / 32u;
-    p.maxc = (max_t + 31u + kPfAttKC - 1u) / kPfAttKC;
-    const size_t units = static_cast<size_t>(H) * p.qtmax * p.maxc;
-    if (int rc = take(units * 32u * hd * 4u, &q)) return rc;
+    p.parts = std::max(kPfAttParts, H * ((max_t + 31u) / 32u));
+    if (int rc = take(static_cast<size_t>(p.parts) * 32u * hd * 4u, &q)) return rc;
     p.opart = static_cast<float*>(q);
-    if (int rc = take(units * 32u * 4u, &q)) return rc;
+    if (int rc = take(static_cast<size_t>(p.parts) * 32u * 4u, &q)) return rc;
     p.mpart = static_cast<float*>(q);
-    if (int rc = take(units * 32u * 8u, &q)) return rc;
+    if (int rc = take(static_cast<size_t>(p.parts) * 32u * 8u, &q)) return rc;
     p.lpart = static_cast<double*>(q);
     // Expanded weights: 2 bytes per quant + 4 per 32 (2.125 bytes per weight, twice the Q8_0
     // matrices' 1.0625), made once here when they fit kPfExpandBudget.
@@ -1137,14 +1121,49 @@ int pf_setup(vrt_g3* g, uint32_t max_t) {
 }
 
 template <uint32_t HD>
-static int pf_attn_launch(const PfAttn& A, dim3 grid, hipStream_t s) {
+static int pf_attn_launch(const PfAttn& A, bool lo, hipStream_t s) {
     PfAttn arg = A;
     void* args[] = {&arg};
-    VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_attn<HD>), grid, dim3(256), args, 0, s));
-    if (grid.x > 1u)   // some tile has several chunks
-        VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_attn_merge<HD>),
-                                      dim3(grid.y, grid.z, pf_merge_groups<HD>()), dim3(256), args, 0, s));
+    const void* fn = lo ? reinterpret_cast<const void*>(&k_pf_attn<HD, true>) : reinterpret_cast<const void*>(&k_pf_attn<HD, false>);
+    VRT_HIP_CHECK(hipLaunchKernel(fn, dim3(A.groups * A.nch), dim3(256), args, 0, s));
+    if (A.nch > 1u)   // some group has several chunks
+        VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_attn_merge<HD>), dim3(A.pairs, (HD / 32u + 3u) / 4u),
+                                      dim3(256), args, 0, s));
     return VRT_OK;
+}
+
+// Keys per chunk of a launch, by a model of its time in key-tile steps of one workgroup (~2 us): a
+// workgroup costs its steps and about one more to start and end, 256 CUs hold one each, and a
+// chunked launch adds the merge (about two steps, and ~0.03 per workgroup for the partials' traffic).
+static void pf_att_chunks(PfAttn& A, uint32_t max_parts) {
+    uint32_t longest = 1;   // key tiles of the longest range
+    uint64_t total = 0;
+    std::vector<uint32_t> len(A.groups);
+    for (uint32_t g = 0; g < A.groups; ++g) {
+        uint32_t ks, ke;
+        pf_att_group(A, g, ks, ke);
+        len[g] = (ke - ks + 31u) / 32u;
+        longest = std::max(longest, len[g]);
+        total += len[g];
+    }
+    double best = 0.0;
+    uint32_t best_kc = 0;
+    for (uint32_t n = 1; n <= longest; ++n) {   // n chunks of the longest range
+        const uint32_t tiles = (longest + n - 1u) / n;
+        if (n > 1u && (tiles < 2u || n > 64u || (longest + tiles - 1u) / tiles != n)) continue;
+        if (n > 1u && static_cast<uint64_t>(A.groups) * kPfAttPairs * n > max_parts) break;
+        uint64_t units = 0;
+        for (uint32_t g = 0; g < A.groups; ++g) units += (len[g] + tiles - 1u) / tiles;
+        const double avg = static_cast<double>(total + units) / 256.0;
+        double t = units <= 256u ? tiles + 1.0 : std::max(tiles + 1.0, avg + 0.5 * tiles);
+        if (n > 1u) t += 2.0 + 0.03 * static_cast<double>(units) / 4.0;
+        if (best_kc == 0u || t < best) {
+            best = t;
+            best_kc = 32u * tiles;
+        }
+    }
+    A.kc = best_kc;
+    A.nch = (32u * longest + A.kc - 1u) / A.kc;
 }
 
 // Causal local/global attention of one block (k_pf_attn) over the queries of p.qhi/p.qlo [T][H hd],
@@ -1157,7 +1176,6 @@ static int pf_attention(vrt_g3* g, const LayerParams& Ly, uint32_t T, uint32_t o
     A.qlo = p.qlo;
     A.o = p.a;
     A.o_row = o_row;
-    const uint32_t qt0 = o_row / 32u;
     A.khi = static_cast<const _Float16*>(p.khi);
     A.klo = static_cast<const _Float16*>(p.klo);
     A.vhi = static_cast<const _Float16*>(p.vhi);
@@ -1169,35 +1187,25 @@ static int pf_attention(vrt_g3* g, const LayerParams& Ly, uint32_t T, uint32_t o
     A.T = T;
     A.H = H;
     A.window = Ly.slots >= g->cfg.context_length ? 0u : Ly.slots;
-    A.qtmax = p.qtmax;
-    A.maxc = p.maxc;
     A.block = Ly.index;
     A.scale2 = g->P.attn_scale * 1.4426950408889634f;
-    const uint32_t qt = (T + 31u) / 32u;
-    A.qt0 = qt0;
     A.qo = qo;
-    // the longest key range of a query tile (the same ranges as pf_att_range), then a chunk size
-    // that keeps it within maxc chunks (a segment's history can reach back to position 0)
-    uint32_t span = 32;
-    for (uint32_t i = qt0; i < qt; ++i) {
-        const uint32_t qk0 = qo + 32u * i, ke = std::min(qo + T, qk0 + 32u);
-        const uint32_t ks = A.window != 0u && qk0 + 1u > A.window ? (qk0 + 1u - A.window) & ~31u : 0u;
-        span = std::max(span, ke - ks);
-    }
-    A.kc = std::max(kPfAttKC, (span + 32u * p.maxc - 1u) / (32u * p.maxc) * 32u);
-    const uint32_t nch = (span + A.kc - 1u) / A.kc;
-    if (qt > p.qtmax || nch > p.maxc || qt0 >= qt || pf_pad(qo + T) > p.tkv)
+    A.pair0 = o_row / 32u * H;
+    A.pairs = (T + 31u) / 32u * H - A.pair0;
+    A.groups = (A.pairs + kPfAttPairs - 1u) / kPfAttPairs;
+    pf_att_chunks(A, p.parts);
+    if (A.pairs * static_cast<uint64_t>(A.nch) > p.parts || pf_pad(qo + T) > p.tkv)
         return set_error(VRT_ERR_STATE, "prefill attention workspace too small");
-    const dim3 grid(nch, qt - qt0, H);
+    const bool lo = g->P.kv16 == 0u;   // 16-bit entries have no low parts
     switch (hd) {
-    case 32: return pf_attn_launch<32>(A, grid, s);
-    case 64: return pf_attn_launch<64>(A, grid, s);
-    case 96: return pf_attn_launch<96>(A, grid, s);
-    case 128: return pf_attn_launch<128>(A, grid, s);
-    case 160: return pf_attn_launch<160>(A, grid, s);
-    case 192: return pf_attn_launch<192>(A, grid, s);
-    case 224: return pf_attn_launch<224>(A, grid, s);
-    case 256: return pf_attn_launch<256>(A, grid, s);
+    case 32: return pf_attn_launch<32>(A, lo, s);
+    case 64: return pf_attn_launch<64>(A, lo, s);
+    case 96: return pf_attn_launch<96>(A, lo, s);
+    case 128: return pf_attn_launch<128>(A, lo, s);
+    case 160: return pf_attn_launch<160>(A, lo, s);
+    case 192: return pf_attn_launch<192>(A, lo, s);
+    case 224: return pf_attn_launch<224>(A, lo, s);
+    case 256: return pf_attn_launch<256>(A, lo, s);
     default: return set_error(VRT_ERR_INVALID, "prefill head_dim not supported");
     }
 }
@@ -1278,8 +1286,8 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0, bool final) {
             _Float16 *qhi = p.qhi, *qlo = p.qlo;
             void* args[] = {&qkv, &s_qkv, &qs, &T, &H, &hd, &qn, &kn, &ct, &sn, &eps, &kc, &vc, &slots, &qhi, &qlo, &khi, &klo, &vhi, &vlo,
                             &kvf, &p0_, &qo_};
-            const uint32_t waves = std::min(H + 1u, kPfQkMaxWaves);
-            VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_qk), dim3(tp), dim3(64u * waves), args, 0, s));
+            VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_qk), dim3(tp / kPfQkRows), dim3(64u * kPfQkRows),
+                                          args, 0, s));
         }
         // The last block's output feeds only the LM head, so past its q/k/v (every position's
         // keys and values go to the cache) it runs for the last position alone: attention for
