@@ -6,6 +6,7 @@ import os
 import numpy as np
 import pytest
 
+import oracle
 import synth
 import vrt
 
@@ -64,3 +65,51 @@ def _compare(ctx, path, rows, tol):
         assert _rel(lp, ld) <= tol
     finally:
         g.close()
+
+
+def _span(buf, offset, nbytes):
+    class At:
+        ptr, nbytes_ = buf.ptr + offset, nbytes
+        keep = buf
+    a = At()
+    a.nbytes = nbytes
+    return a
+
+
+@pytest.mark.parametrize("blocks", (1, 2, 7, 127, 128, 129, 300))
+@pytest.mark.parametrize("x_off,q_off", ((0, 0), (4, 0), (0, 2), (16, 32), (12, 1)))
+def test_codec_runs_and_alignments(ctx, blocks, x_off, q_off):
+    """Runs of 128 blocks and what is left of them, on arrays that are 16-byte aligned and not: the bytes and
+    values of the oracle, and nothing written past the end."""
+    x = synth.normal_f32(33 + blocks, 32 * blocks + blocks % 2, 0.7)[:32 * blocks]
+    x[:32] = 0.0   # an all-zero block
+    nq = 34 * blocks
+    xb, qb, yb = ctx.alloc(x.nbytes + 64), ctx.alloc(nq + 128), ctx.alloc(x.nbytes + 64)
+    host = np.zeros(x.nbytes + 64, dtype=np.uint8)
+    host[x_off:x_off + x.nbytes] = x.view(np.uint8)
+    xb.write(host)
+    for variant, name in ((0, "a"), (1, "b")):
+        qb.write(np.full(nq + 128, 0xA5, dtype=np.uint8))
+        vrt.q8_quantize(ctx, _span(xb, x_off, x.nbytes), x.size, variant, _span(qb, q_off, nq))
+        ctx.sync()
+        got = qb.read(np.uint8, nq + 128)
+        assert np.array_equal(got[q_off:q_off + nq], oracle.quantize(x, name))
+        assert np.all(got[:q_off] == 0xA5) and np.all(got[q_off + nq:] == 0xA5)
+        vrt.q8_dequantize(ctx, _span(qb, q_off, nq), blocks, _span(yb, x_off, x.nbytes))
+        ctx.sync()
+        y = yb.read(np.uint8, x.nbytes + 64)[x_off:x_off + x.nbytes].view(np.float32)
+        assert np.array_equal(y.view(np.uint32), oracle.dequant(oracle.quantize(x, name)).view(np.uint32))
+
+
+@pytest.mark.parametrize("k,rows", ((640, 32768), (576, 32773), (640, 32767), (544, 40001), (608, 33000)))
+def test_matvec_many_rows(ctx, k, rows):
+    """Both sides of the rule that gives many rows of 17 to 20 blocks five blocks per lane; odd block counts put
+    every other row two bytes off a dword."""
+    w = synth.q8_matrix(5, "t", rows, k)
+    x = synth.normal_f32(6, k, 1.0)
+    wd, xd, yd = ctx.upload(w), ctx.upload(x), ctx.alloc(rows * 4)
+    vrt.q8_matvec(ctx, wd, 0, xd, yd, k, rows, w_bytes=w.size)
+    ctx.sync()
+    ref = oracle.matvec_f64(w, x, rows)
+    # limb and summation error, as bounded per row in the standalone kernels' tests, over this matrix's rows
+    assert np.max(np.abs(yd.read(np.float32, rows) - ref)) <= 2e-6 * np.max(np.abs(ref))

@@ -58,6 +58,49 @@ bool mv_shape(uint32_t K, MvShape* out) {
 // Generic matvec: y[v] = row_v(W) . x over a virtual row space.
 // ---------------------------------------------------------------------------------------
 
+// q8_load without a branch: the scale, eight dwords from (block + 2) & ~3 and the 16 bits after them (used
+// where the quants start two bytes into the first dword; else a pair inside the block), all within
+// the 34 bytes. A load behind a branch waits for every load before it.
+__device__ __forceinline__ void q8_load_flat(const uint8_t* blk, Q8Raw& r) {
+    typedef uint32_t v4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef const __attribute__((address_space(1))) v4* gv4;
+    typedef const __attribute__((address_space(1))) uint16_t* gu16;
+    const uintptr_t q = reinterpret_cast<uintptr_t>(blk) + 2u, a = q & ~uintptr_t(3);
+    r.sh = static_cast<uint32_t>(q & 3u);
+    r.sbits = *(gu16)(blk);
+    const v4 lo = *reinterpret_cast<gv4>(a), hi = *reinterpret_cast<gv4>(a + 16u);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        r.d[j] = lo[j];
+        r.d[4 + j] = hi[j];
+    }
+    r.d[8] = *reinterpret_cast<gu16>(a + (r.sh ? 32u : 30u));
+}
+
+// U row groups of the calling wave: pass u takes group g0 + u * 4, rows RPW each from v_begin. Rows past v_end
+// and blocks past nblk are neither loaded nor counted.
+template <int S, int NB, int U, typename RowFn>
+__device__ __forceinline__ void mv_load(RowFn&& rowp, uint32_t nblk, uint32_t v_begin, uint32_t v_end, uint32_t g0,
+                                        RowBatch<S, NB, U>& rb) {
+    constexpr uint32_t RPW = 64u / S;
+    const uint32_t lane = threadIdx.x & 63u, slot = lane / S, sl = lane % S;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        rb.vrow[u] = v_begin + (g0 + 4u * u) * RPW + slot;
+        rb.live[u] = rb.vrow[u] < v_end;
+        const uint8_t* rp = rowp(min(rb.vrow[u], v_end - 1u));
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            const uint32_t b = sl + static_cast<uint32_t>(n) * S;
+            if (rb.live[u] && b < nblk) q8_load_flat(rp + 34u * b, rb.raw[u][n]);
+        }
+    }
+}
+
+// Four waves. A row on a whole wave loads its blocks as dwords (stream_rows): 64 lanes of 34-byte blocks gain nothing
+// from 16-byte loads (1120 x 5003: 6.97 against 7.27 us); with several rows per wave they do (640 x 1536: 7.13 -> 6.74).
+// (The first rows' loads ahead of the activations, to overlap the two latencies: 1120 x 5003 7.0 -> 7.2, the FFN
+// unchanged; the activations then wait behind the weights.)
 template <int S, int NB, int U>
 __global__ void __launch_bounds__(256) k_matvec(RowSpace rs, uint64_t row_bytes, uint32_t K, const uint8_t* w_end,
                                                 const float* __restrict__ x, float* __restrict__ y,
@@ -66,21 +109,30 @@ __global__ void __launch_bounds__(256) k_matvec(RowSpace rs, uint64_t row_bytes,
     float* xs = reinterpret_cast<float*>(smem);
     LimbLds L{reinterpret_cast<int8_t*>(xs + K), reinterpret_cast<int8_t*>(xs + K) + K,
               reinterpret_cast<int8_t*>(xs + K) + 2 * K, reinterpret_cast<float*>(reinterpret_cast<int8_t*>(xs + K) + 3 * K)};
-    for (uint32_t i = threadIdx.x; i < K; i += blockDim.x) xs[i] = x[i];
-    __syncthreads();
-    build_limbs(xs, K, L, blockDim.x >> 6);
-    const uint32_t nblk = K >> 5;
-    const uint32_t sl = (threadIdx.x & 63u) % S;
-    XLimb xl[NB];
-#pragma unroll
-    for (int n = 0; n < NB; ++n) {
-        const uint32_t b = sl + static_cast<uint32_t>(n) * S;
-        if (b < nblk) load_limb(L, b, xl[n]);
-    }
+    const uint32_t nblk = K >> 5, wave = threadIdx.x >> 6;
     const uint32_t v0 = blockIdx.x * rows_per_wg;
     const uint32_t v1 = min(rs.total, v0 + rows_per_wg);
     if (v0 >= v1) return;
-    stream_rows<S, NB, U>(rs, row_bytes, nblk, w_end, xl, v0, v1, [&](uint32_t v, float val) { y[v] = val; });
+    for (uint32_t i = threadIdx.x; i < K; i += 256u) xs[i] = x[i];
+    __syncthreads();
+    build_limbs(xs, K, L, 4u);
+    XLimb xl[NB];
+    lane_limbs<S, NB>(L, nblk, xl);
+    auto sink = [&](uint32_t v, float val) { y[v] = val; };
+    if constexpr (S == 64) {
+        stream_rows<S, NB, U>(rs, row_bytes, nblk, w_end, xl, v0, v1, sink);
+    } else {
+        const uint32_t ngroups = (v1 - v0 + 64u / S - 1u) / (64u / S);
+        auto rowp = [&](uint32_t v) {
+            uint32_t seg, local;
+            return row_ptr(rs, v, row_bytes, seg, local);
+        };
+        for (uint32_t g0 = wave; g0 < ngroups; g0 += 4u * U) {
+            RowBatch<S, NB, U> rb;
+            mv_load<S, NB, U>(rowp, nblk, v0, v1, g0, rb);
+            batch_consume<S, NB, U>(rb, nblk, xl, sink);
+        }
+    }
 }
 
 static size_t matvec_smem(uint32_t K) {
@@ -121,6 +173,10 @@ int launch_matvec(hipStream_t stream, const uint8_t* const* bases, const uint32_
     rs.total = static_cast<uint32_t>(total);
     rs.interleave = interleave ? 1u : 0u;
     const uint64_t row_bytes = static_cast<uint64_t>(K / 32u) * 34u;
+    // Many rows of 17 to 20 blocks: slots of 4 lanes x 5 blocks keep 85 to 100% of the lanes on a block, where one
+    // block on each of 32 lanes keeps 53 to 62% (262144 x 640: 50 -> 38 us). Fewer rows than fill the chip
+    // that way are better spread thin.
+    if (sh.S == 32 && K / 32u <= 20u && total >= 32768u) return launch_mv_t<4, 5, 1>(stream, rs, row_bytes, K, w_end, x, y);
     switch (sh.S * 16 + sh.NB) {
     case 1 * 16 + 1: return launch_mv_t<1, 1, 2>(stream, rs, row_bytes, K, w_end, x, y);
     case 2 * 16 + 1: return launch_mv_t<2, 1, 2>(stream, rs, row_bytes, K, w_end, x, y);
@@ -162,61 +218,41 @@ __global__ void __launch_bounds__(256) k_gelu_mul(float* __restrict__ gate, cons
 // * up (and up[i] for the workspace image). Pairs [pairs_per_wg * blockIdx.x, ...) per workgroup.
 template <int S, int NB, int U>
 __global__ void __launch_bounds__(256) k_ffn_gateup(const uint8_t* gate_w, const uint8_t* up_w, uint64_t row_bytes,
-                                                    uint32_t K, const uint8_t* w_end, const float* __restrict__ x,
-                                                    float* __restrict__ h, float* __restrict__ up_out, uint32_t F,
-                                                    uint32_t pairs_per_wg) {
+                                                    uint32_t K, const float* __restrict__ x, float* __restrict__ h,
+                                                    float* __restrict__ up_out, uint32_t F, uint32_t pairs_per_wg) {
 #pragma clang fp contract(off)
     static_assert(S <= 32, "a wave must hold whole gate/up pairs");
     extern __shared__ __align__(16) unsigned char smem[];
     float* xs = reinterpret_cast<float*>(smem);
     LimbLds L{reinterpret_cast<int8_t*>(xs + K), reinterpret_cast<int8_t*>(xs + K) + K,
               reinterpret_cast<int8_t*>(xs + K) + 2 * K, reinterpret_cast<float*>(reinterpret_cast<int8_t*>(xs + K) + 3 * K)};
-    for (uint32_t i = threadIdx.x; i < K; i += blockDim.x) xs[i] = x[i];
-    __syncthreads();
-    build_limbs(xs, K, L, blockDim.x >> 6);
-    const uint32_t nblk = K >> 5;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+    const uint32_t nblk = K >> 5, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t slot = lane / S, sl = lane % S;
-    XLimb xl[NB];
-#pragma unroll
-    for (int n = 0; n < NB; ++n) {
-        const uint32_t b = sl + static_cast<uint32_t>(n) * S;
-        if (b < nblk) load_limb(L, b, xl[n]);
-    }
-    constexpr uint32_t RPW = 64u / S;   // virtual rows per wave pass: RPW / 2 pairs
     const uint32_t v_begin = 2u * blockIdx.x * pairs_per_wg;
     const uint32_t v_end = min(2u * F, v_begin + 2u * pairs_per_wg);
     if (v_begin >= v_end) return;
+    constexpr uint32_t RPW = 64u / S;   // virtual rows per wave pass: RPW / 2 pairs
     const uint32_t ngroups = (v_end - v_begin + RPW - 1u) / RPW;
-    for (uint32_t g0 = wave; g0 < ngroups; g0 += U * nwaves) {
-        Q8Raw raw[U][NB];
-        uint32_t vrow[U];
-        bool live[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint32_t g = g0 + static_cast<uint32_t>(u) * nwaves;
-            vrow[u] = v_begin + g * RPW + slot;
-            live[u] = g < ngroups && vrow[u] < v_end;
-            const uint8_t* rp = ((vrow[u] & 1u) ? up_w : gate_w) + static_cast<uint64_t>(vrow[u] >> 1) * row_bytes;
-#pragma unroll
-            for (int n = 0; n < NB; ++n) {
-                const uint32_t b = sl + static_cast<uint32_t>(n) * S;
-                if (live[u] && b < nblk) q8_load(rp + 34u * b, w_end, raw[u][n]);
-            }
-        }
+    auto rowp = [&](uint32_t v) { return ((v & 1u) ? up_w : gate_w) + static_cast<uint64_t>(v >> 1) * row_bytes; };
+    for (uint32_t i = threadIdx.x; i < K; i += 256u) xs[i] = x[i];
+    __syncthreads();
+    build_limbs(xs, K, L, 4u);
+    XLimb xl[NB];
+    lane_limbs<S, NB>(L, nblk, xl);
+    for (uint32_t g0 = wave; g0 < ngroups; g0 += 4u * U) {
+        RowBatch<S, NB, U> rb;
+        mv_load<S, NB, U>(rowp, nblk, v_begin, v_end, g0, rb);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             float acc = 0.0f;
 #pragma unroll
-            for (int n = 0; n < NB; ++n) {
-                const uint32_t b = sl + static_cast<uint32_t>(n) * S;
-                if (live[u] && b < nblk) acc += q8_dot(raw[u][n], xl[n]);
-            }
+            for (int n = 0; n < NB; ++n)
+                if (rb.live[u] && sl + static_cast<uint32_t>(n) * S < nblk) acc += q8_dot(rb.raw[u][n], xl[n]);
             const float tot = slot_sum<S>(acc);
             // the up total of this pair, from the odd slot next to it (every lane takes part)
             const float upv = __shfl(tot, static_cast<int>(min(lane + static_cast<uint32_t>(S), 63u)));
-            if (live[u] && sl == 0u && (slot & 1u) == 0u) {
-                const uint32_t i = vrow[u] >> 1;
+            if (rb.live[u] && sl == 0u && (slot & 1u) == 0u) {
+                const uint32_t i = rb.vrow[u] >> 1;
                 h[i] = gelu_tanh_dev(tot) * upv;
                 up_out[i] = upv;
             }
@@ -287,31 +323,115 @@ __device__ __forceinline__ uint32_t f32_to_f16_ref(float f) {
     return sign | (static_cast<uint32_t>(exponent) << 10) | ((mantissa + 0x1000u) >> 13);
 }
 
-// One half-wave per 32-value block, one lane per value.
-__global__ void __launch_bounds__(256) k_quantize(const float* __restrict__ x, uint64_t nblocks, uint32_t variant,
-                                                  uint8_t* __restrict__ out) {
-    const uint64_t blk = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5;
-    const uint32_t k = threadIdx.x & 31u;
-    const bool live = blk < nblocks;
-    const float v = live ? x[blk * 32u + k] : 0.0f;
-    // abs_max starts at 0 and std::max(abs_max, fabs(v)) never takes a NaN: fmaxf(0, .)
-    float amax = fmaxf(0.0f, fabsf(v));
-    for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
-    if (!live) return;
+// src/q8_test_main.cpp:43-131 on one value: the quant of v against its block's divisor.
+__device__ __forceinline__ int quant_ref(float v, float div) {
+    const float r = rintf(v / div);
+    // static_cast<int> of NaN or |r| >= 2^31 is INT_MIN on x86-64; clamp -> -127
+    return !(fabsf(r) < 2147483648.0f) ? -127 : max(-127, min(127, static_cast<int>(r)));
+}
+// The block's scale bits and divisor from its largest magnitude.
+__device__ __forceinline__ uint32_t scale_ref(float amax, uint32_t variant, float& div) {
     float scale = amax / 127.0f;
     if (variant == 1u && amax == 0.0f) scale = 1.0f;
     const uint32_t half = f32_to_f16_ref(scale);
-    const float div = variant == 1u ? half_bits_to_float(half) : scale;
-    const float r = rintf(v / div);
-    // static_cast<int> of NaN or |r| >= 2^31 is INT_MIN on x86-64; clamp -> -127
-    const int q = !(fabsf(r) < 2147483648.0f) ? -127 : max(-127, min(127, static_cast<int>(r)));
-    uint8_t* o = out + blk * 34u;
-    o[2 + k] = static_cast<uint8_t>(static_cast<int8_t>(q));
-    if (k == 0) { o[0] = static_cast<uint8_t>(half & 0xffu); o[1] = static_cast<uint8_t>(half >> 8); }
+    div = variant == 1u ? half_bits_to_float(half) : scale;
+    return half;
+}
+
+// Both codec kernels move a workgroup's 128 blocks (16 KB of fp32, 4352 bytes of Q8_0) in 16-byte units: the
+// 34-byte blocks go through an LDS image of the packed run, whose start is 16-byte aligned whenever the
+// array's is. Eight lanes work on a block, four values each. Bound by memory: one byte per lane stores
+// and loads ran at 2.35 TB/s over the pair (181 us for 65536 x 640).
+constexpr uint32_t kCodecBlocks = 128;
+constexpr uint32_t kCodecBytes = kCodecBlocks * 34u;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+__global__ void __launch_bounds__(256) k_quantize(const float* __restrict__ x, uint64_t nblocks, uint32_t variant,
+                                                  uint8_t* __restrict__ out) {
+    __shared__ __align__(16) uint8_t s_b[kCodecBytes];
+    const uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * kCodecBlocks;
+    const uint32_t n = static_cast<uint32_t>(min(nblocks - b0, static_cast<uint64_t>(kCodecBlocks)));
+    const uint32_t j = threadIdx.x & 7u;
+    f32x4 v[kCodecBlocks / 32u];
+#pragma unroll
+    for (uint32_t k = 0; k < kCodecBlocks / 32u; ++k) {   // at a clamped, in-bounds block
+        const uint32_t b = min((threadIdx.x >> 3) + 32u * k, n - 1u);
+        v[k] = *reinterpret_cast<const f32x4*>(x + (b0 + b) * 32u + 4u * j);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kCodecBlocks / 32u; ++k) {
+        // abs_max starts at 0 and std::max(abs_max, fabs(v)) never takes a NaN: fmaxf(0, .)
+        float amax = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(v[k][e]));
+        amax = fmaxf(amax, dpp_mov<0xB1>(amax));    // the block's eight lanes: quad_perm [1,0,3,2],
+        amax = fmaxf(amax, dpp_mov<0x4E>(amax));    // quad_perm [2,3,0,1],
+        amax = fmaxf(amax, dpp_mov<0x141>(amax));   // row_half_mirror
+        float div;
+        const uint32_t half = scale_ref(amax, variant, div);
+        uint32_t q = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q |= (static_cast<uint32_t>(quant_ref(v[k][e], div)) & 0xffu) << (8 * e);
+        const uint32_t b = (threadIdx.x >> 3) + 32u * k;
+        uint16_t* o = reinterpret_cast<uint16_t*>(s_b + 34u * b);
+        o[1u + 2u * j] = static_cast<uint16_t>(q);
+        o[2u + 2u * j] = static_cast<uint16_t>(q >> 16);
+        if (j == 0u) o[0] = static_cast<uint16_t>(half);
+    }
+    __syncthreads();
+    uint8_t* dst = out + b0 * 34u;
+    const uint32_t bytes = n * 34u, n16 = bytes / 16u;
+    for (uint32_t i = threadIdx.x; i < n16; i += 256u)
+        *reinterpret_cast<u32x4*>(dst + 16u * i) = *reinterpret_cast<const u32x4*>(s_b + 16u * i);
+    for (uint32_t i = 16u * n16 + threadIdx.x; i < bytes; i += 256u) dst[i] = s_b[i];   // the last run's end
 }
 
 __global__ void __launch_bounds__(256) k_dequantize(const uint8_t* __restrict__ blocks, uint64_t nblocks,
                                                     float* __restrict__ out) {
+    __shared__ __align__(16) uint8_t s_b[kCodecBytes];
+    const uint64_t b0 = static_cast<uint64_t>(blockIdx.x) * kCodecBlocks;
+    const uint32_t n = static_cast<uint32_t>(min(nblocks - b0, static_cast<uint64_t>(kCodecBlocks)));
+    const uint8_t* src = blocks + b0 * 34u;
+    const uint32_t bytes = n * 34u, n16 = bytes / 16u;
+    for (uint32_t i = threadIdx.x; i < n16; i += 256u)
+        *reinterpret_cast<u32x4*>(s_b + 16u * i) = *reinterpret_cast<const u32x4*>(src + 16u * i);
+    for (uint32_t i = 16u * n16 + threadIdx.x; i < bytes; i += 256u) s_b[i] = src[i];
+    __syncthreads();
+    const uint32_t j = threadIdx.x & 7u;
+#pragma unroll
+    for (uint32_t k = 0; k < kCodecBlocks / 32u; ++k) {
+        const uint32_t b = (threadIdx.x >> 3) + 32u * k;
+        if (b >= n) break;
+        const uint16_t* o = reinterpret_cast<const uint16_t*>(s_b + 34u * b);
+        const float s = half_bits_to_float(o[0]);
+        const uint32_t q = o[1u + 2u * j] | (static_cast<uint32_t>(o[2u + 2u * j]) << 16);
+        f32x4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = s * static_cast<float>(static_cast<int8_t>(q >> (8 * e)));
+        *reinterpret_cast<f32x4*>(out + (b0 + b) * 32u + 4u * j) = y;
+    }
+}
+
+// The same for arrays that are not 16-byte aligned: one lane per value.
+__global__ void __launch_bounds__(256) k_quantize_any(const float* __restrict__ x, uint64_t nblocks, uint32_t variant,
+                                                      uint8_t* __restrict__ out) {
+    const uint64_t blk = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 5;
+    const uint32_t k = threadIdx.x & 31u;
+    const bool live = blk < nblocks;
+    const float v = live ? x[blk * 32u + k] : 0.0f;
+    float amax = fmaxf(0.0f, fabsf(v));
+    for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    if (!live) return;
+    float div;
+    const uint32_t half = scale_ref(amax, variant, div);
+    uint8_t* o = out + blk * 34u;
+    o[2 + k] = static_cast<uint8_t>(static_cast<int8_t>(quant_ref(v, div)));
+    if (k == 0) { o[0] = static_cast<uint8_t>(half & 0xffu); o[1] = static_cast<uint8_t>(half >> 8); }
+}
+
+__global__ void __launch_bounds__(256) k_dequantize_any(const uint8_t* __restrict__ blocks, uint64_t nblocks,
+                                                        float* __restrict__ out) {
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= nblocks * 32u) return;
     const uint8_t* b = blocks + (i >> 5) * 34u;
@@ -335,8 +455,8 @@ static int launch_ffn_gateup(hipStream_t stream, const uint8_t* gate_w, const ui
         uint32_t grid = std::min<uint32_t>(groups, 2048u);
         const uint32_t per = (groups + grid - 1u) / grid * pairs_per_pass;
         grid = (F + per - 1u) / per;
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), matvec_smem(K), stream, gate_w, up_w, row_bytes, K, w_end, x, h,
-                           up_out, F, per);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), matvec_smem(K), stream, gate_w, up_w, row_bytes, K, x, h, up_out,
+                           F, per);
         VRT_HIP_CHECK(hipGetLastError());
         return VRT_OK;
     };
@@ -636,6 +756,11 @@ extern "C" int vrt_argmax(vrt_ctx* ctx, const float* x, uint32_t n, vrt_argmax_r
     return VRT_OK;
 }
 
+// Whole 16-byte units on both sides (every run of kCodecBlocks blocks then starts on one).
+static bool codec_aligned(const void* a, const void* b) {
+    return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0u;
+}
+
 extern "C" int vrt_q8_quantize(vrt_ctx* ctx, const float* x, uint64_t n, uint32_t variant, void* out) {
     VRT_REQUIRE(ctx && x && out, "vrt_q8_quantize: null argument");
     VRT_REQUIRE(n % 32u == 0u, "test matrix input must be divisible by 32");
@@ -644,8 +769,12 @@ extern "C" int vrt_q8_quantize(vrt_ctx* ctx, const float* x, uint64_t n, uint32_
     const uint64_t nb = n / 32u;
     const uint64_t threads = nb * 32u;
     VRT_REQUIRE((threads + 255u) / 256u <= 0x7fffffffu, "vrt_q8_quantize: input too large");
-    hipLaunchKernelGGL(k_quantize, dim3(static_cast<uint32_t>((threads + 255u) / 256u)), dim3(256), 0, ctx->stream, x, nb,
-                       variant, static_cast<uint8_t*>(out));
+    if (codec_aligned(x, out))
+        hipLaunchKernelGGL(k_quantize, dim3(static_cast<uint32_t>((nb + kCodecBlocks - 1u) / kCodecBlocks)), dim3(256), 0,
+                           ctx->stream, x, nb, variant, static_cast<uint8_t*>(out));
+    else
+        hipLaunchKernelGGL(k_quantize_any, dim3(static_cast<uint32_t>((threads + 255u) / 256u)), dim3(256), 0, ctx->stream, x, nb,
+                           variant, static_cast<uint8_t*>(out));
     VRT_HIP_CHECK(hipGetLastError());
     return VRT_OK;
 }
@@ -655,8 +784,12 @@ extern "C" int vrt_q8_dequantize(vrt_ctx* ctx, const void* blocks, uint64_t nblo
     if (nblocks == 0) return VRT_OK;
     const uint64_t n = nblocks * 32u;
     VRT_REQUIRE((n + 255u) / 256u <= 0x7fffffffu, "vrt_q8_dequantize: input too large");
-    hipLaunchKernelGGL(k_dequantize, dim3(static_cast<uint32_t>((n + 255u) / 256u)), dim3(256), 0, ctx->stream,
-                       static_cast<const uint8_t*>(blocks), nblocks, out);
+    if (codec_aligned(blocks, out))
+        hipLaunchKernelGGL(k_dequantize, dim3(static_cast<uint32_t>((nblocks + kCodecBlocks - 1u) / kCodecBlocks)), dim3(256), 0,
+                           ctx->stream, static_cast<const uint8_t*>(blocks), nblocks, out);
+    else
+        hipLaunchKernelGGL(k_dequantize_any, dim3(static_cast<uint32_t>((n + 255u) / 256u)), dim3(256), 0, ctx->stream,
+                           static_cast<const uint8_t*>(blocks), nblocks, out);
     VRT_HIP_CHECK(hipGetLastError());
     return VRT_OK;
 }
