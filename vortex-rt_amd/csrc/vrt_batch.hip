@@ -33,7 +33,7 @@ namespace vrt {
 constexpr uint32_t kBdThreads = 256;
 constexpr uint32_t kBdMaxChunks = 64;     // history chunks per row and block, at most
 constexpr uint32_t kBdMaxRows = 64;       // sequences per step (one 64-row GEMM tile)
-constexpr uint32_t kBdArgParts = 256;     // argmax partials per row
+constexpr uint32_t kBdArgParts = kGmLmMaxChunks;   // argmax partials per row, at most
 constexpr uint32_t kBdMaxSplits = 4;      // K splits of a projection (the consumers' limit)
 
 // One block's attention over the rows of a step.
@@ -234,140 +234,146 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn(BdAttn A) {
     }
 }
 
-constexpr uint32_t kBdShort = 32;   // rows whose histories are all this short take k_bd_attn_short
-
 // Histories of at most kBdShort positions: one workgroup per (head h, row b) runs the head's whole
-// attention and writes its output, with no chunk partials to merge. The cached key and value rows
-// are loaded first, before the q|k|v split partials are added, so the loads overlap. Waves 0 and 1
-// apply QK-norm and NeoX RoPE to q_h and k (src/gemma3.cpp:1045-1104, :1371-1424); the head-0
-// workgroup appends k and v at slot pos % slots (:1590-1600). The scores (wave w: positions
-// t_first + w + 4 u), the maximum, e^(s - m) with their double sum, the weighted values (thread per
-// dimension, positions in order) and the division follow k_bd_attn and k_bd_merge for one chunk
-// (:1602-1696). The current position's k and v come from LDS, never from the cache.
+// attention and writes its output, with no chunk partials to merge. Every wave holds the head's q and the
+// row's k in registers (lane l: dims 4 l .. 4 l + 3) and applies QK-norm and NeoX RoPE itself
+// (src/gemma3.cpp:1045-1104, :1371-1424), so nothing waits for another wave before the end. Wave w takes
+// the positions t_first + w + 4 u, 4 NU of them per pass (every key and value row of a pass is
+// loaded together, the first pass's before the q|k|v row is added up), and keeps its own maximum, double sum
+// and weighted values (:1602-1696); the four are combined in double through LDS behind the only
+// barrier. The head-0 workgroup appends k and v at slot pos % slots (:1590-1600); the current position's k and
+// v come from registers, never from the cache. The launch is one memory latency, not bandwidth: staged through
+// LDS, with one wave's softmax over shuffles, it took 8.9 us at 8 rows.
+constexpr uint32_t kBdShort = 256;   // four passes; longer histories gain from more workgroups than (heads, rows)
+template <int NU>
 __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
 #pragma clang fp contract(off)
-    __shared__ float sq[256], sk[256], sv[256];
-    __shared__ float ssc[kBdShort];
-    __shared__ double s_l;
+    constexpr uint32_t NW = kBdThreads / 64u;
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) float s_acc[NW][256];
+    __shared__ float s_m[NW];
+    __shared__ double s_l[NW];
     const uint32_t h = blockIdx.x, b = blockIdx.y;
     const uint32_t H = A.H, hd = A.hd, half = hd >> 1, nq = (H + 2u) * hd;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t p = A.pos[b], sqn = A.seq[b];
-    const uint32_t n_full = min(p + 1u, A.slots), t_first = p + 1u - n_full;
-    const uint32_t n_hist = min(n_full, kBdShort);   // the host sends no longer history here
+    const uint32_t n_hist = min(p + 1u, A.slots), t_first = p + 1u - n_hist;
     const uint64_t cache0 = static_cast<uint64_t>(sqn) * A.slots * hd;
-    const uint32_t di = min(tid, hd - 1u);
-    // cached key rows (wave w: positions t_first + w + 4 u; lane: dims lane + 64 e) and value rows
-    // (thread: its dimension, every position), at clamped in-bounds positions
-    float kr[8][4], vv[kBdShort];
+    const uint32_t i = min(4u * lane, hd - 4u);   // lanes past hd hold copies and count nothing
+    const bool live = 4u * lane < hd, lower = i < half;
+    f4 kr[NU], vr[NU];
+    auto load = [&](uint32_t t0) {   // clamped, in-bounds positions
 #pragma unroll
-    for (uint32_t u = 0; u < 8u; ++u) {
-        const uint64_t row = cache0 + static_cast<uint64_t>(min(t_first + wave + 4u * u, p) % A.slots) * hd;
-#pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) kr[u][e] = A.kc[row + min(lane + 64u * e, hd - 1u)];
-    }
-#pragma unroll
-    for (uint32_t u = 0; u < kBdShort; ++u)
-        vv[u] = A.vc[cache0 + static_cast<uint64_t>(min(t_first + u, p) % A.slots) * hd + di];
-    float rc[4], rs[4];   // RoPE table entries of the dims lane + 64 e (waves 0 and 1 use them)
-#pragma unroll
-    for (uint32_t e = 0; e < 4u; ++e) {
-        const uint32_t ic = min(lane + 64u * e, hd - 1u), ei = ic < half ? ic : ic - half;
-        rc[e] = A.cos_t[static_cast<uint64_t>(p) * half + ei];
-        rs[e] = A.sin_t[static_cast<uint64_t>(p) * half + ei];
-    }
-    {   // q of head h, k and v: the split partials added in order
-        const float* src = A.qkv + static_cast<uint64_t>(b) * nq;
-        float pq[kBdMaxSplits], pk[kBdMaxSplits], pw[kBdMaxSplits];
-#pragma unroll
-        for (uint32_t z = 0; z < kBdMaxSplits; ++z) {
-            const uint64_t o = static_cast<uint64_t>(min(z, A.nsplit - 1u)) * A.sstride;
-            pq[z] = src[o + h * hd + di];
-            pk[z] = src[o + H * hd + di];
-            pw[z] = src[o + (H + 1u) * hd + di];
+        for (int u = 0; u < NU; ++u) {
+            const uint64_t row = cache0 + static_cast<uint64_t>(min(t0 + wave + NW * u, p) % A.slots) * hd + i;
+            kr[u] = *reinterpret_cast<const f4*>(A.kc + row);
+            vr[u] = *reinterpret_cast<const f4*>(A.vc + row);
         }
-        float a = 0.0f, c = 0.0f, e = 0.0f;
+    };
+    load(t_first);
+    const uint32_t ri = lower ? i : i - half;
+    const f4 cs = *reinterpret_cast<const f4*>(A.cos_t + static_cast<uint64_t>(p) * half + ri);
+    const f4 sn = *reinterpret_cast<const f4*>(A.sin_t + static_cast<uint64_t>(p) * half + ri);
+    f4 x[2], v;   // q of the head, k of the row
+    {
+        const f4 wq = *reinterpret_cast<const f4*>(A.q_norm + i), wk = *reinterpret_cast<const f4*>(A.k_norm + i);
+        const float* src = A.qkv + static_cast<uint64_t>(b) * nq + i;
+        auto at = [&](uint32_t o) {   // the split partials added in order
+            f4 y = *reinterpret_cast<const f4*>(src + o);
+            for (uint32_t z = 1; z < A.nsplit; ++z) {
+                const f4 w = *reinterpret_cast<const f4*>(src + z * A.sstride + o);
 #pragma unroll
-        for (uint32_t z = 0; z < kBdMaxSplits; ++z)
-            if (z < A.nsplit) { a += pq[z]; c += pk[z]; e += pw[z]; }
-        if (tid < hd) { sq[tid] = a; sk[tid] = c; sv[tid] = e; }
+                for (int e = 0; e < 4; ++e) y[e] += w[e];
+            }
+            return y;
+        };
+        x[0] = at(h * hd);
+        x[1] = at(H * hd);
+        v = at((H + 1u) * hd);
+        double ss[2] = {0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ss[k] += live ? static_cast<double>(x[k][e]) * static_cast<double>(x[k][e]) : 0.0;
+        const uint32_t partner = (lower ? lane + (hd >> 3) : lane - (hd >> 3)) & 63u;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float sc = 1.0f / sqrtf(static_cast<float>(wave_red_sum_d(ss[k]) / static_cast<double>(hd)) + A.eps);   // :1087-1093
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float a = x[k][e] * (sc * (k ? wk[e] : wq[e])), c = __shfl(a, static_cast<int>(partner));
+                x[k][e] = lower ? a * cs[e] - c * sn[e] : a * cs[e] + c * sn[e];
+            }
+        }
+    }
+    if (h == 0u && wave == 0u && live) {   // KV append of this row's position
+        const uint64_t o = cache0 + static_cast<uint64_t>(p % A.slots) * hd + i;
+        *reinterpret_cast<f4*>(A.kc + o) = x[1];
+        *reinterpret_cast<f4*>(A.vc + o) = v;
+    }
+    float m = -INFINITY;
+    double l = 0.0;
+    f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t t0 = t_first; t0 <= p; t0 += NW * NU) {
+        if (t0 != t_first) load(t0);
+        float s[NU], mx = m;
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const uint32_t t = t0 + wave + NW * u;
+            float d = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d += x[0][e] * (t == p ? x[1][e] : kr[u][e]);
+            d = wave_sum(live ? d : 0.0f) * A.attn_scale;
+            s[u] = t <= p ? d : -INFINITY;
+            mx = fmaxf(mx, s[u]);
+        }
+        if (t0 + wave > p) continue;   // no position of this wave in the pass
+        const float alpha = m == -INFINITY ? 0.0f : expf(m - mx);
+        m = mx;
+        l *= static_cast<double>(alpha);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] *= alpha;
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const uint32_t t = t0 + wave + NW * u;
+            const float w = expf(s[u] - mx);
+            l += static_cast<double>(w);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += w * (t == p ? v[e] : vr[u][e]);
+        }
+    }
+    if (live) *reinterpret_cast<f4*>(&s_acc[wave][i]) = acc;
+    if (lane == 0u) {
+        s_m[wave] = m;
+        s_l[wave] = l;
     }
     __syncthreads();
-    if (wave < 2u) {   // QK-norm and RoPE of q_h (wave 0) and k (wave 1); lane l: dims l + 64 e
-        float* x = wave == 0u ? sq : sk;
-        const float* w = wave == 0u ? A.q_norm : A.k_norm;
-        uint32_t ic[4], ei[4];
-        bool live[4];
-        float v[4], wv[4];
-        double ss = 0.0;
+    if (wave != 0u || !live) return;
+    float M = -INFINITY;
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) {
-            live[e] = lane + 64u * e < hd;
-            ic[e] = min(lane + 64u * e, hd - 1u);
-            ei[e] = ic[e] < half ? ic[e] : ic[e] - half;
-            wv[e] = w[ic[e]];
-            v[e] = live[e] ? x[ic[e]] : 0.0f;
-            ss += static_cast<double>(v[e]) * static_cast<double>(v[e]);
-        }
-        const double tot = wave_red_sum_d(ss);
-        const float sc = 1.0f / sqrtf(static_cast<float>(tot / static_cast<double>(hd)) + A.eps);   // :1087-1093
+    for (uint32_t w = 0; w < NW; ++w) M = fmaxf(M, s_m[w]);
+    double den = 0.0, num[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e)
-            if (live[e]) x[ic[e]] = v[e] * (sc * wv[e]);
-        __builtin_amdgcn_wave_barrier();   // a wave's LDS accesses complete in order
-        float y[4];
+    for (uint32_t w = 0; w < NW; ++w) {
+        const double f = s_m[w] == -INFINITY ? 0.0 : static_cast<double>(expf(s_m[w] - M));
+        den += f * s_l[w];
+        const f4 a = *reinterpret_cast<const f4*>(&s_acc[w][i]);
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) {
-            const float a = x[ei[e]], bb = x[ei[e] + half];
-            y[e] = ic[e] < half ? a * rc[e] - bb * rs[e] : bb * rc[e] + a * rs[e];
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e)
-            if (live[e]) x[ic[e]] = y[e];
+        for (int e = 0; e < 4; ++e) num[e] += f * static_cast<double>(a[e]);
     }
-    __syncthreads();
-    if (h == 0u && tid < hd) {   // KV append of this row's position
-        const uint64_t o = cache0 + static_cast<uint64_t>(p % A.slots) * hd + tid;
-        A.kc[o] = sk[tid];
-        A.vc[o] = sv[tid];
-    }
+    if (lane == 0u && (!(den > 0.0) || !__builtin_isfinite(den))) atomicMin(&A.st->nonfinite, g3_code_softmax(A.block));
+    const uint64_t o = gm_off(b, h * hd + i, H * hd / 32u);
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    half4 hi, lo;
 #pragma unroll
-    for (uint32_t u = 0; u < 8u; ++u) {
-        const uint32_t t = t_first + wave + 4u * u;
-        if (t > p) break;
-        float d = 0.0f;
-#pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e)
-            if (lane + 64u * e < hd) d += sq[lane + 64u * e] * (t == p ? sk[lane + 64u * e] : kr[u][e]);
-        d = wave_sum(d);
-        if (lane == 0u) ssc[t - t_first] = d * A.attn_scale;
+    for (int e = 0; e < 4; ++e) {
+        _Float16 a, c;
+        gm_split(static_cast<float>(num[e] / den), a, c);
+        hi[e] = a;
+        lo[e] = c;
     }
-    __syncthreads();
-    if (wave == 0u) {   // m = max, e = exp(s - m), l = sum e (double)
-        float mx = lane < n_hist ? ssc[lane] : -INFINITY;
-        mx = wave_max(mx);
-        double l = 0.0;
-        if (lane < n_hist) {
-            const float e = expf(ssc[lane] - mx);
-            ssc[lane] = e;
-            l = e;
-        }
-        l = wave_sum_f64(l);
-        if (lane == 0u) s_l = l;
-    }
-    __syncthreads();
-    if (tid < hd) {
-        float acc = 0.0f;
-#pragma unroll
-        for (uint32_t u = 0; u < kBdShort; ++u)
-            if (u < n_hist) acc += ssc[u] * (t_first + u == p ? sv[tid] : vv[u]);
-        const double den = static_cast<double>(static_cast<float>(s_l));
-        if (tid == 0u && (!(den > 0.0) || !__builtin_isfinite(den))) atomicMin(&A.st->nonfinite, g3_code_softmax(A.block));
-        const float v = static_cast<float>(static_cast<double>(acc) / den);
-        const uint64_t o = gm_off(b, h * hd + tid, H * hd / 32u);
-        gm_split(v, A.o[o], A.o[o + kGmLo]);
-    }
+    *reinterpret_cast<half4*>(A.o + o) = hi;
+    *reinterpret_cast<half4*>(A.o + o + kGmLo) = lo;
 }
 
 // One workgroup per (head h, row b): att = sum_c e^(m_c - M) acc_c / sum_c e^(m_c - M) l_c over the
@@ -409,7 +415,7 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_merge(BdAttn A) {
 // Greedy argmax of each row's logits [n][V] (the tie rule of am_better, shaders/argmax.comp:30-43):
 // k_bd_argmax, grid (kBdArgParts, n), leaves one partial per (part, row); k_bd_argmax_final,
 // one workgroup per row, reduces them into results[b].
-__global__ void __launch_bounds__(kBdThreads) k_bd_argmax(const float* logits, uint32_t V, LmPartial* parts) {
+__global__ void __launch_bounds__(kBdThreads) k_bd_argmax(const float* logits, uint32_t V, GmBest* parts) {
     __shared__ float bvs[kBdThreads / 64u];
     __shared__ uint32_t bis[kBdThreads / 64u];
     const uint32_t b = blockIdx.y;
@@ -441,7 +447,7 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_argmax(const float* logits, u
     }
 }
 
-__global__ void __launch_bounds__(kBdThreads) k_bd_argmax_final(const LmPartial* parts, uint32_t nparts,
+__global__ void __launch_bounds__(kBdThreads) k_bd_argmax_final(const GmBest* parts, uint32_t nparts,
                                                                 vrt_argmax_result* results) {
     __shared__ float bvs[kBdThreads / 64u];
     __shared__ uint32_t bis[kBdThreads / 64u];
@@ -449,7 +455,7 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_argmax_final(const LmPartial*
     float bv = -INFINITY;
     uint32_t bi = 0xffffffffu;
     for (uint32_t k = threadIdx.x; k < nparts; k += kBdThreads) {
-        const LmPartial pp = parts[static_cast<uint64_t>(b) * nparts + k];
+        const GmBest pp = parts[static_cast<uint64_t>(b) * nparts + k];
         if (am_better(pp.value, pp.index, bv, bi)) {
             bv = pp.value;
             bi = pp.index;
@@ -495,14 +501,15 @@ struct vrt_g3_batch {
     vrt_argmax_result* host_res = nullptr;   // pinned
     G3State* st = nullptr;          // device: failure word (nonfinite)
     G3State* host_st = nullptr;     // pinned
-    float* h = nullptr;             // [rows][d] residual stream
+    float* h = nullptr;             // [rows][d] residual stream, and its other buffer (pf_norm_project)
+    float* h2 = nullptr;
     float* x = nullptr;             // [kBdMaxSplits][rows][d] O / down projection partials
     float* qkv = nullptr;           // [kBdMaxSplits][rows][(H + 2) hd] q|k|v partials
     _Float16* a = nullptr;          // activation buffer of max(d, H hd) columns: GEMM input
     _Float16* gg = nullptr;         // activation buffer of F columns: gelu(gate) * up
     float* part = nullptr;          // [rows][max G][2 H + H hd] attention chunk partials
     float* logits = nullptr;        // [rows][V]
-    LmPartial* amx = nullptr;       // [rows][kBdArgParts]
+    GmBest* amx = nullptr;       // [rows][kBdArgParts]
 };
 
 static int bd_alloc(vrt_g3_batch* B, size_t bytes, void** out) {
@@ -578,6 +585,8 @@ extern "C" int vrt_g3_batch_create(vrt_g3* g, uint32_t max_seqs, uint32_t max_ct
     B->st = static_cast<G3State*>(p);
     if (int rc = bd_alloc(B, R * d * 4u, &p)) return fail(rc);
     B->h = static_cast<float*>(p);
+    if (int rc = bd_alloc(B, R * d * 4u, &p)) return fail(rc);
+    B->h2 = static_cast<float*>(p);
     if (int rc = bd_alloc(B, kBdMaxSplits * R * d * 4u, &p)) return fail(rc);
     B->x = static_cast<float*>(p);
     if (int rc = bd_alloc(B, kBdMaxSplits * R * nqkv * 4u, &p)) return fail(rc);
@@ -590,8 +599,8 @@ extern "C" int vrt_g3_batch_create(vrt_g3* g, uint32_t max_seqs, uint32_t max_ct
     B->part = static_cast<float*>(p);
     if (int rc = bd_alloc(B, R * c.vocab_size * 4u, &p)) return fail(rc);
     B->logits = static_cast<float*>(p);
-    if (int rc = bd_alloc(B, R * kBdArgParts * sizeof(LmPartial), &p)) return fail(rc);
-    B->amx = static_cast<LmPartial*>(p);
+    if (int rc = bd_alloc(B, R * kBdArgParts * sizeof(GmBest), &p)) return fail(rc);
+    B->amx = static_cast<GmBest*>(p);
     {
         hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&B->host_rows), 3u * R * 4u, hipHostMallocDefault);
         if (e == hipSuccess)
@@ -602,6 +611,7 @@ extern "C" int vrt_g3_batch_create(vrt_g3* g, uint32_t max_seqs, uint32_t max_ct
     size_t lds = 0;
     for (const BdLayer& L : B->layers) lds = std::max(lds, static_cast<size_t>((H + 2u) * hd + H * L.cmax) * 4u);
     if (lds > 64u * 1024u) return fail(set_error(VRT_ERR_INVALID, "batched decode: attention chunk does not fit in LDS"));
+    if (int rc = gm_setup()) return fail(rc);
     VRT_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_bd_attn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(lds)));
     *out = B;
@@ -639,15 +649,15 @@ static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
     if (int rc = pf_embed_rows(g, tok, n, B->h, s)) return rc;
     const uint64_t xs = static_cast<uint64_t>(n) * d;   // one O / down partial
     uint32_t s_down = 1;
+    float *h = B->h, *spare = B->h2;
     for (uint32_t l = 0; l < L; ++l) {
         const LayerParams& Ly = g->layers[l];
         const BdLayer& BL = B->layers[l];
-        // previous block's FFN output into the residual, then the attention norm
-        if (int rc = pf_norm(B->h, l ? B->x : nullptr, s_down, xs, l ? g->layers[l - 1].post_ffw : nullptr, Ly.attn_norm,
-                             d, eps, B->a, B->st, l ? l - 1u : 0u, n, s, true))
-            return rc;
+        // previous block's FFN output into the residual, the attention norm, q|k|v
         uint32_t s_qkv = 1;
-        if (int rc = pf_project(g, l, kProjQkv, B->a, n, B->qkv, &s_qkv, s))
+        if (int rc = pf_norm_project(g, l, false, &h, &spare, l ? B->x : nullptr, s_down, xs,
+                                     l ? g->layers[l - 1].post_ffw : nullptr, l ? l - 1u : 0u, B->a, n, B->qkv, &s_qkv, nullptr,
+                                     B->st, s))
             return rc;
         BdAttn A{};
         A.qkv = B->qkv;
@@ -676,9 +686,10 @@ static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
             void* args[] = {&A};
             uint32_t nh_max = 0;   // longest history of the step's rows in this block
             for (uint32_t i = 0; i < n; ++i) nh_max = std::max(nh_max, std::min(B->host_rows[kBdMaxRows + i] + 1u, BL.slots));
-            if (nh_max <= kBdShort && hd <= 256u) {
-                VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_bd_attn_short), dim3(H, n), dim3(kBdThreads),
-                                              args, 0, s));
+            if (nh_max <= kBdShort && hd % 8u == 0u) {   // whole runs of four on both sides of a RoPE pair
+                const void* fn = nh_max <= 32u ? reinterpret_cast<const void*>(&k_bd_attn_short<8>)
+                                               : reinterpret_cast<const void*>(&k_bd_attn_short<16>);
+                VRT_HIP_CHECK(hipLaunchKernel(fn, dim3(H, n), dim3(kBdThreads), args, 0, s));
             } else {
                 const size_t lds = static_cast<size_t>((H + 2u) * hd + H * BL.cmax) * 4u;
                 VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_bd_attn), dim3(BL.G, n), dim3(kBdThreads), args,
@@ -690,26 +701,32 @@ static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
         uint32_t s_o = 1;
         if (int rc = pf_project(g, l, kProjO, B->a, n, B->x, &s_o, s))
             return rc;
-        if (int rc = pf_norm(B->h, B->x, s_o, xs, Ly.post_attn, Ly.ffn_norm, d, eps, B->a, B->st, l, n, s, true))
+        if (int rc = pf_norm_project(g, l, true, &h, &spare, B->x, s_o, xs, Ly.post_attn, l, B->a, n, nullptr, nullptr, B->gg,
+                                     B->st, s))
             return rc;
-        if (int rc = pf_ffn_glu(g, l, B->a, n, B->gg, s)) return rc;
         if (int rc = pf_project(g, l, kProjDown, B->gg, n, B->x, &s_down, s))
             return rc;
     }
     // final residual (:1849-1855) and output norm (rms_norm_inplace, :1866-1868) as the LM input
-    if (int rc = pf_norm(B->h, B->x, s_down, xs, g->layers[L - 1u].post_ffw, g->out_norm_dev, d, eps, B->a, B->st,
+    if (int rc = pf_norm(h, B->x, s_down, xs, g->layers[L - 1u].post_ffw, g->out_norm_dev, d, eps, B->a, B->st,
                          L - 1u, n, s, false))
         return rc;
-    if (int rc = pf_lm_logits(g, B->a, n, B->logits, s)) return rc;
-    {
+    uint32_t nparts = kBdArgParts;
+    if (gm_lm_fits(g->P.tok_embd, static_cast<uint64_t>(g->P.arena_end - g->P.tok_embd), c.vocab_size, d / 32u)) {
+        if (int rc = gm_lm(g->P.tok_embd, c.vocab_size, d / 32u, B->a, n, B->logits, B->amx, s)) return rc;
+        nparts = gm_lm_chunks(n, d / 32u);
+    } else {
+        if (int rc = pf_lm_logits(g, B->a, n, B->logits, s)) return rc;
         const float* lg = B->logits;
         uint32_t V = c.vocab_size;
-        LmPartial* parts = B->amx;
+        GmBest* parts = B->amx;
         void* a1[] = {&lg, &V, &parts};
         VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_bd_argmax), dim3(kBdArgParts, n), dim3(kBdThreads),
                                       a1, 0, s));
-        const LmPartial* cp = B->amx;
-        uint32_t np = kBdArgParts;
+    }
+    {
+        const GmBest* cp = B->amx;
+        uint32_t np = nparts;
         vrt_argmax_result* res = B->res;
         void* a2[] = {&cp, &np, &res};
         VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_bd_argmax_final), dim3(n), dim3(kBdThreads), a2,

@@ -110,11 +110,12 @@ struct PfLayerW {
 struct PfState {
     uint32_t max_t = 0;     // prompt positions per call
     float* h = nullptr;     // [max_t][d] residual stream
+    float* h2 = nullptr;    // [16][d] its other buffer where a projection folds it (pf_norm_project)
     float* x = nullptr;     // [max_t][d] sublayer outputs (O projection, down projection)
     _Float16* a = nullptr;  // activation buffer (vrt_gemm.hpp) of max(d, H*hd) columns: normed rows, attention output
     _Float16* g = nullptr;  // activation buffer of F columns: gelu(gate) * up
     float* qkv = nullptr;   // [splits][max_t][H*hd + 2*hd] q|k|v rows
-    _Float16* qhi = nullptr;   // [max_t][H*hd] queries after QK-norm and RoPE, f16 high part
+    _Float16* qhi = nullptr;   // queries after QK-norm and RoPE in operand order (pf_qswz), f16 high part
     _Float16* qlo = nullptr;   //   ... and low part
     void* khi = nullptr;    // attention keys (tkv x hd), f16 high part: a segment's history, then its rows
     void* klo = nullptr;    //   ... and low part
@@ -189,6 +190,9 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0 = 0, bool final = true);
 // norms over rows, embedding rows, and the logits of M rows against the tied embedding table.
 enum PfProj : uint32_t { kProjQkv = 0, kProjO = 1, kProjDown = 2 };
 int pf_project(vrt_g3* g, uint32_t l, uint32_t which, const _Float16* a, uint32_t M, float* c, uint32_t* used, hipStream_t s);
+int pf_norm_project(vrt_g3* g, uint32_t l, bool glu, float** h, float** spare, const float* f, uint32_t nsplit, uint64_t sstride,
+                    const float* w_post, uint32_t fold_block, _Float16* a, uint32_t M, float* c, uint32_t* used, _Float16* o,
+                    G3State* st, hipStream_t s);
 int pf_ffn_glu(vrt_g3* g, uint32_t l, const _Float16* a, uint32_t M, _Float16* o, hipStream_t s);
 int pf_norm(float* h, const float* f, uint32_t nsplit, uint64_t sstride, const float* w_post, const float* w_next,
             uint32_t n, float eps, _Float16* x, G3State* st, uint32_t block, uint32_t rows, hipStream_t s, bool into);

@@ -69,10 +69,39 @@ constexpr uint32_t kGmSplitWgs = 160;   // K is split up to this many 64 x 64 ti
 constexpr uint64_t kGmSplitFloats = 4ull * kGmSplitWgs * 64u * 64u;   //   so many partial sums
 uint32_t gm_splits(uint32_t M, uint32_t N, uint32_t nkb);
 int gm_run(const GmArgs& G, uint32_t splits, bool glu, hipStream_t s);
+// The same with the residual fold and norm that come before it (G.a unused; at most 16 rows):
+// h_out = f * (scale(f) * w_post) + h (f nullptr: no fold, nothing written), and the projection of
+// (h_out * scale(h_out)) * w_next. h_out is another buffer than h. A non-finite h_out lowers *nonfinite to code.
+struct GmNorm {
+    const float* h;
+    const float* f;
+    float* h_out;
+    const float* w_post;
+    const float* w_next;
+    uint32_t* nonfinite;
+    uint32_t code;
+    float eps;
+};
+bool gm_norm_fits(uint32_t M, uint32_t nkb);
+int gm_run_norm(const GmArgs& G, const GmNorm& R, bool glu, hipStream_t s);
+int gm_setup();   // once per device before gm_lm: its LDS limit
 // One-time expansion of Q8_0 rows into a weight matrix: up to three matrices concatenated
 // (rows0, rows1, the rest), or with glu the gate (w0) and up (w1) rows interleaved. Rows N..npad-1
 // are zero with scale 0.
 int gm_expand(const uint8_t* w0, const uint8_t* w1, const uint8_t* w2, uint32_t rows0, uint32_t rows1, uint32_t N,
               uint32_t nkb, bool glu, _Float16* wh, float* ws, hipStream_t s);
+// logits [M][V] = x W^T over V Q8_0 rows of nkb blocks in their file layout, x an activation buffer, and the best
+// logit (am_better) of each row in each of gm_lm_chunks runs of the V rows: best [M][chunks]. gm_lm_fits: the table is
+// 16-byte aligned and readable in whole 16-byte units, and a tile of it fits LDS.
+constexpr uint32_t kGmLdsMax = 160u * 1024u;
+constexpr uint32_t kGmLmMaxChunks = 512;
+struct GmBest {
+    float value;
+    uint32_t index;
+};
+bool gm_lm_fits(const uint8_t* table, uint64_t readable, uint32_t V, uint32_t nkb);
+uint32_t gm_lm_chunks(uint32_t M, uint32_t nkb);
+int gm_lm(const uint8_t* table, uint32_t V, uint32_t nkb, const _Float16* x, uint32_t M, float* logits, GmBest* best,
+          hipStream_t s);
 
 }  // namespace vrt

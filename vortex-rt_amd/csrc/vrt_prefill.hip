@@ -466,6 +466,12 @@ __device__ __forceinline__ uint64_t pf_vswz(uint32_t t, uint32_t d, uint32_t hd)
            (d & 31u) * 8u + (w & 7u);
 }
 
+// Queries in operand order: per (32-row tile, head) and k step s, lane half f and row m of the B operand of
+// S^T hold Q[32 tile + m][16 s + 8 f + j], j < 8 (1 KB per step).
+__device__ __forceinline__ uint64_t pf_qswz(uint32_t t, uint32_t h, uint32_t d, uint32_t H, uint32_t hd) {
+    return ((static_cast<uint64_t>(t >> 5) * H + h) * (hd / 16u) + (d >> 4)) * 512u + ((d >> 3) & 1u) * 256u + (t & 31u) * 8u + (d & 7u);
+}
+
 // ---- QK-norm, RoPE, KV cache ------------------------------------------------------------
 
 // Four consecutive cache entries from entry i on (fp32, or 16-bit in the first half of the buffer).
@@ -482,8 +488,8 @@ __device__ __forceinline__ void kv_store4(float* c, uint64_t i, f4 x, uint32_t k
 }
 
 // Row t of qkv = [q (H heads x hd) | k (hd) | v (hd)], the sum of nsplit partials: QK-norm per head
-// (src/gemma3.cpp:1045-1104), NeoX RoPE at position p0 + t (:1371-1424), q as f16 hi/lo rows of
-// qhi/qlo; then k and v go to the KV cache slot of the position when it is still in the window
+// (src/gemma3.cpp:1045-1104), NeoX RoPE at position p0 + t (:1371-1424), q as f16 hi/lo in
+// pf_qswz order; then k and v go to the KV cache slot of the position when it is still in the window
 // after the segment (the serial loop's eviction leaves exactly those, :1590-1600); with kv16 (1 fp16,
 // 2 bf16) the cache holds 16-bit entries and k and v are rounded to them first (the attention below
 // then sees the cached values, as the serial loop does). The attention operands as f16 hi/lo: k and
@@ -495,7 +501,7 @@ __device__ __forceinline__ void kv_store4(float* c, uint64_t i, f4 x, uint32_t k
 // rows, consecutive in the value operand, meet in LDS and leave as 16-byte stores (one row per
 // workgroup and two-byte stores: 14.4 us at 2048 rows).
 constexpr uint32_t kPfQkRows = 8;
-constexpr uint32_t kPfQkHeads = 4;   // heads in flight per wave
+constexpr uint32_t kPfQkHeads = 5;   // heads in flight per wave (four query heads and the key: one round)
 __global__ void __launch_bounds__(64 * kPfQkRows) k_pf_qk(const float* qkv, uint32_t nsplit, uint64_t sstride, uint32_t T,
                                                           uint32_t H, uint32_t hd, const float* q_norm,
                                                           const float* k_norm, const float* cos_t, const float* sin_t,
@@ -551,7 +557,7 @@ __global__ void __launch_bounds__(64 * kPfQkRows) k_pf_qk(const float* qkv, uint
                     y[e] = lower ? a * cs[e] - b * sn[e] : a * cs[e] + b * sn[e];
                 }
                 if (hh < H) {
-                    const uint64_t o = (static_cast<uint64_t>(t) * H + hh) * hd + i;
+                    const uint64_t o = pf_qswz(t, hh, i, H, hd);
                     if (live) pf_split4(y, qhi + o, qlo + o);
                 } else {   // 16-bit KV: the key as the cache holds it, for the cache and the attention
                     if (kv16) {
@@ -619,14 +625,17 @@ __global__ void __launch_bounds__(kPfThreads) k_pf_kv_hist(const float* kc, cons
 // coordinates (a segment's history first, its rows from A.qo) tile i's first query sits at
 // qk0 = A.qo + 32 i; it sees the keys from the window's start for qk0, rounded down to 32, up to
 // min(A.qo + T, qk0 + 32).
-// All four waves read the same keys and values: a 32-key tile of both (64 KB at hd 256 with low
-// parts) is loaded straight to LDS during the previous tile's work, one barrier per tile. A wave keeps
-// its queries and its O^T in registers (one wave per SIMD). Per tile, lane l on query l % 32: S^T = K Q^T (three
-// f16 products of the hi/lo parts), mask, softmax in base 2 (the scale times log2 e, v_exp_f32) and
-// O^T += V^T E^T (V and E as hi/lo). The running maximum m moves, and O^T is rescaled, only when a
-// tile's scores exceed it by more than 2^kPfAttSlack for some query: e_j = 2^(v_j - m) then stays
-// below 2^kPfAttSlack, exact in the same relative precision. Each tile's sum of e_j in fp32 is added
-// to a running sum in double.
+// All four waves read the same keys and values, loaded straight to LDS one tile ahead (128 KB in two
+// stages at hd 256 with low parts), one barrier per tile. A wave keeps its queries and its O^T in
+// registers, which leaves one wave per SIMD: what overlaps has to be in one instruction stream. Tile
+// n's softmax runs between the products S^T = K Q^T of tile n + 1, and the scores of tile n + 1 are
+// read out between the products O^T += V^T E^T of tile n (three f16 products each of the hi/lo parts; lane l on
+// query l % 32). One after the other (and with the operand reads left to the scheduler, behind a full
+// wait each) a tile took 9000 cycles, 3072 of them products.
+// The softmax is in base 2 (the scale times log2 e, v_exp_f32). The running maximum m moves, and O^T
+// is rescaled, only when a tile's scores exceed it by more than kPfAttSlack for some query: e_j =
+// 2^(v_j - m) then stays below 2^kPfAttSlack, in the same relative precision. Each tile's sum of e_j
+// in fp32 is added to a running sum in double.
 // LO false: a 16-bit KV cache, whose entries are exact in f16, so the low parts of K and V are zero
 // and their products are left out.
 // A group whose range is one chunk is finished here (out = O / sum into the activation buffer);
@@ -638,9 +647,10 @@ __global__ void __launch_bounds__(kPfThreads) k_pf_kv_hist(const float* kc, cons
 // r % 4][l % 32].
 constexpr uint32_t kPfAttPairs = 4;        // pairs per workgroup (waves)
 constexpr uint32_t kPfAttParts = 8192;     // partials kept, at least
+constexpr uint32_t kPfAttFew = 32;         // pairs of a k_pf_attn_few launch, at most
 constexpr float kPfAttSlack = 8.0f;
 struct PfAttn {
-    const _Float16* qhi;   // [T][H * hd] queries, normed and rotated
+    const _Float16* qhi;   // queries, normed and rotated, in pf_qswz order
     const _Float16* qlo;
     const _Float16* khi;   // keys in pf_kswz order, by key coordinate (32-key tiles)
     const _Float16* klo;
@@ -654,7 +664,8 @@ struct PfAttn {
     G3State* st;
     uint32_t T, H, window, block;
     uint32_t kc, nch;      // keys per chunk (a multiple of 32), chunks of the longest range
-    uint32_t pair0, pairs, groups;   // first pair of the launch, pairs and groups of four from it
+    uint32_t pair0, pairs;   // first pair of the launch, pairs from it
+    uint32_t per, groups;    // pairs per group (kPfAttPairs; k_pf_attn_few: 1), groups
     uint32_t qo;           // key coordinate of query row 0 (keys before it: an earlier segment's history)
     float scale2;          // attention scale times log2(e): the scores in base 2
 };
@@ -666,11 +677,30 @@ __host__ __device__ __forceinline__ void pf_att_range(uint32_t qo, uint32_t T, u
     ke = q1 < qo + T ? q1 : qo + T;
     ks = window != 0u && q0 + 1u > window ? (q0 + 1u - window) & ~31u : 0u;
 }
-// ... of group g (four pairs from pair0 + 4 g).
+// ... of group g (pairs pair0 + per g and on).
 __host__ __device__ __forceinline__ void pf_att_group(const PfAttn& A, uint32_t g, uint32_t& ks, uint32_t& ke) {
-    const uint32_t a = A.pair0 + kPfAttPairs * g, last = A.pair0 + A.pairs - 1u;
-    const uint32_t b = a + kPfAttPairs - 1u < last ? a + kPfAttPairs - 1u : last;
+    const uint32_t a = A.pair0 + A.per * g, last = A.pair0 + A.pairs - 1u;
+    const uint32_t b = a + A.per - 1u < last ? a + A.per - 1u : last;
     pf_att_range(A.qo, A.T, A.window, a / A.H, b / A.H, ks, ke);
+}
+
+// O^T tiles times alpha, in the accumulation registers they live in: as plain code the multiplication
+// would move all of them to VGPRs and back in every tile, taken or not. The leading waits cover an
+// MFMA's last write, the trailing one the next MFMA's read.
+template <uint32_t DT>
+__device__ __forceinline__ void att_rescale(float16v (&o)[DT], float alpha) {
+    asm volatile("s_nop 15\n\ts_nop 7");
+#pragma unroll
+    for (uint32_t j = 0; j < DT; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float x = o[j][r], t;
+            asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\tv_accvgpr_write_b32 %0, %1"
+                         : "+a"(x), "=&v"(t)
+                         : "v"(alpha));
+            o[j][r] = x;
+        }
+    asm volatile("s_nop 7");
 }
 
 template <uint32_t HD, bool LO>
@@ -680,8 +710,9 @@ __global__ void __launch_bounds__(256, 1) k_pf_attn(PfAttn A) {
     constexpr uint32_t DT = HD / 32u;               // d tiles of O^T
     constexpr uint32_t NP = LO ? 2u : 1u;           // parts of K and V
     constexpr uint32_t UK = NP * KS, UV = NP * 2u * DT;   // 1 KB operand units of a key tile: K, V
-    constexpr uint32_t UW = (UK + UV) / 4u;         // units per wave (HD is a multiple of 32)
-    __shared__ __align__(1024) unsigned char s_kv[2][(UK + UV) * 1024u];
+    constexpr uint32_t kAhead = 3u;                 // operand reads ahead of their products
+    __shared__ __align__(1024) unsigned char s_k[2][UK * 1024u];
+    __shared__ __align__(1024) unsigned char s_v[2][UV * 1024u];
     // Windowed ranges: workgroup b runs on XCD b % 8 and each XCD takes a contiguous eighth of the
     // (group, chunk) units, so neighbouring groups share their keys in one L2. Full ranges: chunk by
     // chunk, the groups in falling order of length, so every XCD works on the same chunk.
@@ -710,109 +741,220 @@ __global__ void __launch_bounds__(256, 1) k_pf_attn(PfAttn A) {
     const uint32_t pair = A.pair0 + (mine ? rel : A.pairs - 1u), i = pair / A.H, h = pair - i * A.H;
     const uint32_t T = A.T, qw = A.H * HD;
     const uint32_t q = 32u * i + l32, qk0 = A.qo + 32u * i, qk = qk0 + l32;   // this lane's query: row, key coordinate
-    // this wave's loads of a key tile: units u = wave UW + j; a tile advances every part by 64 HD bytes
-    const char* src[UW];
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-        (__attribute__((address_space(3))) unsigned char*)&s_kv[0][0]));
+    // Loads of key tile n of the chunk: the keys' units, the values' units (unit u by wave u % 4)
+    const uint32_t lk = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)&s_k[0][0]));
+    const uint32_t lv = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)&s_v[0][0]));
+    const uint32_t n_tiles = (k1 - k0 + 31u) >> 5;
+    auto load_k = [&](uint32_t n) {
+        const uint64_t o = static_cast<uint64_t>((k0 >> 5) + n) * (64u * HD);   // bytes of a tile in each part
 #pragma unroll
-    for (uint32_t j = 0; j < UW; ++j) {
-        const uint32_t u = wave * UW + j;
-        const _Float16* part = u < UK ? (u < KS ? A.khi : A.klo) : (u - UK < 2u * DT ? A.vhi : A.vlo);
-        const uint32_t idx = u < UK ? u % KS : (u - UK) % (2u * DT);
-        src[j] = reinterpret_cast<const char*>(part) + static_cast<uint64_t>(k0 >> 5) * (64u * HD) + idx * 1024u;
-    }
-    auto issue = [&](uint32_t buf) {
-#pragma unroll
-        for (uint32_t j = 0; j < UW; ++j) {
-            gm_lds16(src[j], lane * 16u, lds0 + buf * ((UK + UV) * 1024u) + (wave * UW + j) * 1024u);
-            src[j] += 64u * HD;
-        }
+        for (uint32_t j = 0; j < UK; j += 4u)
+            if (const uint32_t u = j + wave; UK % 4u == 0u || u < UK)
+                gm_lds16(reinterpret_cast<const char*>(u < KS ? A.khi : A.klo) + o + (u < KS ? u : u - KS) * 1024u, lane * 16u,
+                         lk + (n & 1u) * (UK * 1024u) + u * 1024u);
     };
-    issue(0u);
-    // the queries (B operand of S^T), rows past T clamped (never written)
+    auto load_v = [&](uint32_t n) {
+        const uint64_t o = static_cast<uint64_t>((k0 >> 5) + n) * (64u * HD);
+#pragma unroll
+        for (uint32_t j = 0; j < UV; j += 4u)
+            if (const uint32_t u = j + wave; UV % 4u == 0u || u < UV)
+                gm_lds16(reinterpret_cast<const char*>(u < 2u * DT ? A.vhi : A.vlo) + o + (u < 2u * DT ? u : u - 2u * DT) * 1024u,
+                         lane * 16u, lv + (n & 1u) * (UV * 1024u) + u * 1024u);
+    };
+    load_k(0u);
+    // the queries (B operand of S^T); rows past T hold stale values, and their results are never written
     half8 qb[KS][2];
     {
-        const uint64_t o = static_cast<uint64_t>(min(q, T - 1u)) * qw + h * HD + 8u * hf;
+        const uint64_t o = (static_cast<uint64_t>(i) * A.H + h) * (KS * 512u) + 8u * lane;
 #pragma unroll
         for (uint32_t k = 0; k < KS; ++k) {
-            qb[k][0] = *reinterpret_cast<const half8*>(A.qhi + o + 16u * k);
-            qb[k][1] = *reinterpret_cast<const half8*>(A.qlo + o + 16u * k);
+            qb[k][0] = *reinterpret_cast<const half8*>(A.qhi + o + 512u * k);
+            qb[k][1] = *reinterpret_cast<const half8*>(A.qlo + o + 512u * k);
         }
+        // waited for here: left to the first tile, the wait would be in the loop and drain its loads too
+#pragma unroll
+        for (uint32_t k = 0; k < KS; ++k)
+#pragma unroll
+            for (uint32_t e = 0; e < 2u; ++e) asm volatile("" : "+v"(qb[k][e]));
     }
     float m = -INFINITY;   // reference maximum of the scaled scores of query q
     double lsum = 0.0;     // this lane's share of sum_j e_j
     float16v o[DT];        // O^T tiles: d = 32 dt + 8 (r / 4) + 4 hf + r % 4, query q
 #pragma unroll
     for (uint32_t j = 0; j < DT; ++j) o[j] = float16v{};
-    uint32_t buf = 0;
-    for (uint32_t kt = k0; kt < k1; kt += 32u, buf ^= 1u) {
-        // this tile has arrived, and every wave is done with the other buffer
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (kt + 32u < k1) issue(buf ^ 1u);
-        const unsigned char* pk = &s_kv[buf][lane * 16u];
-        const unsigned char* pv = pk + UK * 1024u;
-        float16v sa = {}, sb = {};   // two chains
+    // S^T of tile n as two chains, sa + sb. Operand reads run kAhead units ahead of their products, in
+    // this order; `between(s)`, s < 2 KS, is work for the products around it to cover.
+    float16v sa, sb;
+    auto scores = [&](uint32_t n, auto between) {
+        const unsigned char* pk = &s_k[n & 1u][lane * 16u];
+        half8 kf[KS][NP];
+        sa = float16v{};
+        sb = float16v{};
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead && k < KS; ++k)
+#pragma unroll
+            for (uint32_t e = 0; e < NP; ++e) kf[k][e] = *reinterpret_cast<const half8*>(pk + (e * KS + k) * 1024u);
 #pragma unroll
         for (uint32_t k = 0; k < KS; ++k) {
-            const half8 ah = *reinterpret_cast<const half8*>(pk + k * 1024u);
-            float16v& s0 = (k & 1u) ? sb : sa;
-            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, qb[k][0], s0, 0, 0, 0);
-            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, qb[k][1], s0, 0, 0, 0);
+            if (k + kAhead < KS)
+#pragma unroll
+                for (uint32_t e = 0; e < NP; ++e)
+                    kf[k + kAhead][e] = *reinterpret_cast<const half8*>(pk + (e * KS + k + kAhead) * 1024u);
+            __builtin_amdgcn_sched_barrier(0);
+            sa = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[k][0], qb[k][0], sa, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            between(2u * k);
+            __builtin_amdgcn_sched_barrier(0);
+            sb = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[k][0], qb[k][1], sb, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            between(2u * k + 1u);
+            __builtin_amdgcn_sched_barrier(0);
             if constexpr (LO) {
-                const half8 al = *reinterpret_cast<const half8*>(pk + (KS + k) * 1024u);
-                s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, qb[k][0], s0, 0, 0, 0);
+                if (k & 1u) sb = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[k][1], qb[k][0], sb, 0, 0, 0);
+                else sa = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[k][1], qb[k][0], sa, 0, 0, 0);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        // scores in base 2 (scale * log2 e folded in): e_j = 2^(v_j - m) = exp(scale s_j - m ln 2)
-        float v[16];
-        float tmax = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = (sa[r] + sb[r]) * A.scale2;
+    };
+    // Tile n's scores v in base 2 (scale * log2 e folded in, tmax their maximum): masked where some key of
+    // the tile is hidden from some query, then the new reference maximum.
+    float v[16], tmax = -INFINITY, alpha = 1.0f;
+    bool grown = false;   // O^T is to be rescaled by alpha before the tile's products
+    auto settle = [&](uint32_t n) {
+        const uint32_t kt = k0 + 32u * n;
         if (!(kt + 31u < k1 && kt + 31u <= qk0 && (A.window == 0u || kt + A.window > qk0 + 31u))) {
+            tmax = -INFINITY;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {   // some key of the tile is hidden from some query
+            for (int r = 0; r < 16; ++r) {
                 const uint32_t key = kt + 16u * (r / 8) + 8u * hf + (r % 8);
                 const bool ok = key < k1 && key <= qk && (A.window == 0u || key + A.window > qk);
                 v[r] = ok ? v[r] : -INFINITY;
+                tmax = fmaxf(tmax, v[r]);
             }
         }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, v[r]);
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
         if (__any(tmax > m + kPfAttSlack)) {   // whole wave; a query with nothing visible yet has m = -inf
             const float mn = fmaxf(m, tmax);
-            const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            grown = n != 0u;   // O^T is zero before the first tile
             m = mn;
             lsum *= static_cast<double>(alpha);
-#pragma unroll
-            for (uint32_t j = 0; j < DT; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
         }
-        const float base = m == -INFINITY ? 0.0f : m;   // nothing visible yet: every e_j is 0
-        float es = 0.0f;   // the tile's share in fp32, then into the double sum
+    };
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");   // queries and the first keys
+    load_v(0u);
+    if (n_tiles > 1u) load_k(1u);
+    scores(0u, [](uint32_t) {});
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        v[r] = (sa[r] + sb[r]) * A.scale2;
+        tmax = fmaxf(tmax, v[r]);
+    }
+    settle(0u);
+    float base, es;   // the tile's sum of e_j in fp32, then into the double sum
+    float ev[16];
+    uint32_t ehu[8], elu[8];   // e as f16 hi and lo, two per register
+    // The asm statements keep a value's computation where it stands, between the products (the
+    // compiler would sink it to its first use).
+    auto soft_exp = [&](uint32_t r) {
+        ev[r] = __builtin_amdgcn_exp2f(v[r] - base);   // exp(scale s_j - m ln 2)
+        es += ev[r];
+        asm volatile("" : "+v"(ev[r]));
+    };
+    auto soft_split = [&](uint32_t p) {
+        typedef _Float16 half2 __attribute__((ext_vector_type(2)));
+        half2 h, l;
+#pragma unroll
+        for (uint32_t e = 0; e < 2u; ++e) {
+            h[e] = static_cast<_Float16>(ev[2u * p + e]);
+            l[e] = static_cast<_Float16>(ev[2u * p + e] - static_cast<float>(h[e]));
+        }
+        ehu[p] = __builtin_bit_cast(uint32_t, h);
+        elu[p] = __builtin_bit_cast(uint32_t, l);
+        asm volatile("" : "+v"(ehu[p]), "+v"(elu[p]));
+    };
+    // slot t of S: its share of the exponentials, and the splits of the slots before it
+    auto soft_slot = [&](uint32_t t, uint32_t S) {
+#pragma unroll
+        for (uint32_t r = 0; r < 16u; ++r)
+            if (r >= 16u * t / S && r < 16u * (t + 1u) / S) soft_exp(r);
+        if (t != 0u)
+#pragma unroll
+            for (uint32_t p = 0; p < 8u; ++p)
+                if (p >= 16u * (t - 1u) / S / 2u && p < 16u * t / S / 2u) soft_split(p);
+    };
+    auto soft_rest = [&](uint32_t S) {
+#pragma unroll
+        for (uint32_t p = 0; p < 8u; ++p)
+            if (p >= 16u * (S - 1u) / S / 2u) soft_split(p);
+    };
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    // O^T += V^T E^T of tile n; `between(k)` is work for the products of unit k to cover
+    auto values = [&](uint32_t n, auto between) {
+        if (grown) {
+            att_rescale<DT>(o, alpha);
+            grown = false;
+        }
         half8 eh[2], el[2];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float e = __builtin_amdgcn_exp2f(v[r] - base);
-            es += e;
-            eh[r / 8][r % 8] = static_cast<_Float16>(e);
-            el[r / 8][r % 8] = static_cast<_Float16>(e - static_cast<float>(eh[r / 8][r % 8]));
+        for (uint32_t e = 0; e < 2u; ++e) {
+            eh[e] = __builtin_bit_cast(half8, u4{ehu[4u * e], ehu[4u * e + 1u], ehu[4u * e + 2u], ehu[4u * e + 3u]});
+            el[e] = __builtin_bit_cast(half8, u4{elu[4u * e], elu[4u * e + 1u], elu[4u * e + 2u], elu[4u * e + 3u]});
         }
+        const unsigned char* pv = &s_v[n & 1u][lane * 16u];
+        half8 vf[2u * DT][NP];   // unit 2 j + sk
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead && k < 2u * DT; ++k)
+#pragma unroll
+            for (uint32_t e = 0; e < NP; ++e) vf[k][e] = *reinterpret_cast<const half8*>(pv + (e * 2u * DT + k) * 1024u);
+#pragma unroll
+        for (uint32_t k = 0; k < 2u * DT; ++k) {
+            if (k + kAhead < 2u * DT)
+#pragma unroll
+                for (uint32_t e = 0; e < NP; ++e)
+                    vf[k + kAhead][e] = *reinterpret_cast<const half8*>(pv + (e * 2u * DT + k + kAhead) * 1024u);
+            __builtin_amdgcn_sched_barrier(0);
+            float16v& oj = o[k >> 1];
+            oj = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[k][0], eh[k & 1u], oj, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            between(k);
+            __builtin_amdgcn_sched_barrier(0);
+            oj = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[k][0], el[k & 1u], oj, 0, 0, 0);
+            if constexpr (LO) oj = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[k][1], eh[k & 1u], oj, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto begin = [&]() {   // the loads before the last barrier have arrived, and every wave is past them
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    for (uint32_t n = 0; n + 1u < n_tiles; ++n) {
+        begin();   // the keys of tile n + 1 and the values of tile n
+        if (n + 2u < n_tiles) load_k(n + 2u);
+        load_v(n + 1u);
+        base = m == -INFINITY ? 0.0f : m;   // nothing visible yet: every e_j is 0
+        es = 0.0f;
+        scores(n + 1u, [&](uint32_t t) { soft_slot(t, 2u * KS); });
+        soft_rest(2u * KS);
         lsum += static_cast<double>(es);
+        tmax = -INFINITY;
+        values(n, [&](uint32_t k) {         // the next tile's scores
 #pragma unroll
-        for (uint32_t j = 0; j < DT; ++j)
-#pragma unroll
-            for (uint32_t sk = 0; sk < 2u; ++sk) {
-                const half8 vh = *reinterpret_cast<const half8*>(pv + (2u * j + sk) * 1024u);
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, eh[sk], o[j], 0, 0, 0);
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, el[sk], o[j], 0, 0, 0);
-                if constexpr (LO) {
-                    const half8 vl = *reinterpret_cast<const half8*>(pv + (2u * (DT + j) + sk) * 1024u);
-                    o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, eh[sk], o[j], 0, 0, 0);
+            for (uint32_t r = 0; r < 16u; ++r)
+                if (r >= 16u * k / (2u * DT) && r < 16u * (k + 1u) / (2u * DT)) {
+                    v[r] = (sa[r] + sb[r]) * A.scale2;
+                    tmax = fmaxf(tmax, v[r]);
+                    asm volatile("" : "+v"(v[r]), "+v"(tmax));
                 }
-            }
+        });
+        settle(n + 1u);
     }
+    begin();
+    base = m == -INFINITY ? 0.0f : m;
+    es = 0.0f;
+    soft_slot(0u, 1u);
+    soft_rest(1u);
+    lsum += static_cast<double>(es);
+    values(n_tiles - 1u, [](uint32_t) {});
     if (!mine) return;
     lsum += __shfl_xor(lsum, 32);   // both lane halves now hold query q's sum
     if (nch == 1u) {   // the whole key range: normalise and write the output rows
@@ -844,6 +986,168 @@ __global__ void __launch_bounds__(256, 1) k_pf_attn(PfAttn A) {
     }
 }
 
+// k_pf_attn for launches of few pairs, which four pairs per workgroup would put on a handful of CUs, each with
+// a long chain: one pair per workgroup, its four waves splitting the head dimension (wave w: the k steps w,
+// w + 4, ... of S^T and the d tiles w, w + 4, ... of O^T). The operands come straight to registers, the
+// next tile's during the current one; each wave's partial S^T goes through LDS and every wave adds the
+// four in wave order (the same scores in every wave), one barrier per tile. Softmax, results and
+// partials as in k_pf_attn. 37 rows: 11.6 -> FEWUS us.
+template <uint32_t HD, bool LO>
+__global__ void __launch_bounds__(256) k_pf_attn_few(PfAttn A) {
+#pragma clang fp contract(off)
+    constexpr uint32_t KS = HD / 16u, DT = HD / 32u, NP = LO ? 2u : 1u;
+    constexpr uint32_t KW = (KS + 3u) / 4u, DW = (DT + 3u) / 4u;   // k steps and d tiles per wave, at most
+    __shared__ __align__(16) float s_s[2][4][16 * 64];
+    const uint32_t c = blockIdx.x / A.groups, rel = blockIdx.x - c * A.groups;
+    uint32_t ks, ke;
+    pf_att_group(A, rel, ks, ke);
+    const uint32_t nch = (ke - ks + A.kc - 1u) / A.kc;
+    if (c >= nch) return;   // whole workgroup
+    const uint32_t k0 = ks + c * A.kc, k1 = min(ke, k0 + A.kc);
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t l32 = lane & 31u, hf = lane >> 5;
+    const uint32_t pair = A.pair0 + rel, i = pair / A.H, h = pair - i * A.H, T = A.T, qw = A.H * HD;
+    const uint32_t q = 32u * i + l32, qk0 = A.qo + 32u * i, qk = qk0 + l32;
+    struct Ops {
+        half8 k[KW][NP], v[DW][2][NP];
+    };
+    auto load = [&](uint32_t kt, Ops& R) {   // steps and tiles past the end: the last one (not used)
+        const uint64_t tile = static_cast<uint64_t>(kt >> 5) * (32u * HD) + 8u * lane;
+#pragma unroll
+        for (uint32_t j = 0; j < KW; ++j) {
+            const uint64_t o = tile + min(wave + 4u * j, KS - 1u) * 512u;
+            R.k[j][0] = *reinterpret_cast<const half8*>(A.khi + o);
+            if constexpr (LO) R.k[j][1] = *reinterpret_cast<const half8*>(A.klo + o);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < DW; ++j)
+#pragma unroll
+            for (uint32_t sk = 0; sk < 2u; ++sk) {
+                const uint64_t o = tile + (min(wave + 4u * j, DT - 1u) * 2u + sk) * 512u;
+                R.v[j][sk][0] = *reinterpret_cast<const half8*>(A.vhi + o);
+                if constexpr (LO) R.v[j][sk][1] = *reinterpret_cast<const half8*>(A.vlo + o);
+            }
+    };
+    half8 qb[KW][2];
+    {
+        const uint64_t o = (static_cast<uint64_t>(i) * A.H + h) * (KS * 512u) + 8u * lane;
+#pragma unroll
+        for (uint32_t j = 0; j < KW; ++j) {
+            qb[j][0] = *reinterpret_cast<const half8*>(A.qhi + o + 512u * min(wave + 4u * j, KS - 1u));
+            qb[j][1] = *reinterpret_cast<const half8*>(A.qlo + o + 512u * min(wave + 4u * j, KS - 1u));
+        }
+    }
+    float m = -INFINITY;
+    double lsum = 0.0;
+    float16v o[DW];
+#pragma unroll
+    for (uint32_t j = 0; j < DW; ++j) o[j] = float16v{};
+    uint32_t buf = 0;
+    auto step = [&](uint32_t kt, const Ops& R) {
+        float16v sp = {};
+#pragma unroll
+        for (uint32_t j = 0; j < KW; ++j) {
+            if (wave + 4u * j >= KS) continue;
+            sp = __builtin_amdgcn_mfma_f32_32x32x16_f16(R.k[j][0], qb[j][0], sp, 0, 0, 0);
+            sp = __builtin_amdgcn_mfma_f32_32x32x16_f16(R.k[j][0], qb[j][1], sp, 0, 0, 0);
+            if constexpr (LO) sp = __builtin_amdgcn_mfma_f32_32x32x16_f16(R.k[j][1], qb[j][0], sp, 0, 0, 0);
+        }
+        // (buffer buf was last read two tiles ago, before the barrier of the previous tile)
+#pragma unroll
+        for (uint32_t rq = 0; rq < 4u; ++rq)
+            *reinterpret_cast<f4*>(&s_s[buf][wave][(rq * 64u + lane) * 4u]) = f4{sp[4 * rq], sp[4 * rq + 1], sp[4 * rq + 2], sp[4 * rq + 3]};
+        __syncthreads();
+        float v[16], tmax = -INFINITY;
+#pragma unroll
+        for (uint32_t rq = 0; rq < 4u; ++rq) {
+            f4 t = *reinterpret_cast<const f4*>(&s_s[buf][0][(rq * 64u + lane) * 4u]);
+#pragma unroll
+            for (uint32_t w = 1; w < 4u; ++w) {
+                const f4 u = *reinterpret_cast<const f4*>(&s_s[buf][w][(rq * 64u + lane) * 4u]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) t[e] += u[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[4 * rq + e] = t[e] * A.scale2;
+        }
+        buf ^= 1u;
+        const bool whole = kt + 31u < k1 && kt + 31u <= qk0 && (A.window == 0u || kt + A.window > qk0 + 31u);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t key = kt + 16u * (r / 8) + 8u * hf + (r % 8);
+            if (!whole && !(key < k1 && key <= qk && (A.window == 0u || key + A.window > qk))) v[r] = -INFINITY;
+            tmax = fmaxf(tmax, v[r]);
+        }
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+        const float mn = fmaxf(m, tmax), base = mn == -INFINITY ? 0.0f : mn;   // nothing visible yet: every e_j is 0
+        const float alpha = __builtin_amdgcn_exp2f(m - base);
+        m = mn;
+        float es = 0.0f;
+        half8 eh[2], el[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float e = __builtin_amdgcn_exp2f(v[r] - base);
+            es += e;
+            eh[r / 8][r % 8] = static_cast<_Float16>(e);
+            el[r / 8][r % 8] = static_cast<_Float16>(e - static_cast<float>(eh[r / 8][r % 8]));
+        }
+        lsum = lsum * static_cast<double>(alpha) + static_cast<double>(es);
+#pragma unroll
+        for (uint32_t j = 0; j < DW; ++j) {
+            if (wave + 4u * j >= DT) continue;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[j][r] *= alpha;
+#pragma unroll
+            for (uint32_t sk = 0; sk < 2u; ++sk) {
+                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(R.v[j][sk][0], eh[sk], o[j], 0, 0, 0);
+                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(R.v[j][sk][0], el[sk], o[j], 0, 0, 0);
+                if constexpr (LO) o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(R.v[j][sk][1], eh[sk], o[j], 0, 0, 0);
+            }
+        }
+    };
+    Ops ra, rb;   // two operand sets in turn
+    load(k0, ra);
+    for (uint32_t kt = k0; kt < k1; kt += 64u) {
+        if (kt + 32u < k1) load(kt + 32u, rb);
+        step(kt, ra);
+        if (kt + 32u >= k1) break;
+        if (kt + 64u < k1) load(kt + 64u, ra);
+        step(kt + 32u, rb);
+    }
+    lsum += __shfl_xor(lsum, 32);
+    if (nch == 1u) {
+        if (q >= T || q < A.o_row) return;
+        const double den = lsum;
+        if (wave == 0u && hf == 0u && (!(den > 0.0) || !__builtin_isfinite(den)))   // :1666-1670
+            atomicMin(&A.st->nonfinite, g3_code_softmax(A.block));
+        const float inv = static_cast<float>(1.0 / den);
+#pragma unroll
+        for (uint32_t j = 0; j < DW; ++j) {
+            if (wave + 4u * j >= DT) continue;
+#pragma unroll
+            for (uint32_t rq = 0; rq < 4u; ++rq) {
+                const uint64_t oo = gm_off(q - A.o_row, h * HD + 32u * (wave + 4u * j) + 8u * rq + 4u * hf, qw / 32u);
+                pf_split4(f4{o[j][4 * rq] * inv, o[j][4 * rq + 1] * inv, o[j][4 * rq + 2] * inv, o[j][4 * rq + 3] * inv},
+                          A.o + oo, A.o + oo + kGmLo);
+            }
+        }
+        return;
+    }
+    const uint64_t unit = static_cast<uint64_t>(rel) * A.nch + c;
+#pragma unroll
+    for (uint32_t j = 0; j < DW; ++j) {
+        if (wave + 4u * j >= DT) continue;
+#pragma unroll
+        for (uint32_t rq = 0; rq < 4u; ++rq)
+            *reinterpret_cast<f4*>(A.opart + unit * 32u * HD + (4u * (wave + 4u * j) + rq) * 256u + lane * 4u) =
+                f4{o[j][4 * rq], o[j][4 * rq + 1], o[j][4 * rq + 2], o[j][4 * rq + 3]};
+    }
+    if (wave == 0u && hf == 0u) {
+        A.mpart[unit * 32u + l32] = m;
+        A.lpart[unit * 32u + l32] = lsum;
+    }
+}
+
 // Merge of the chunk partials of the groups that k_pf_attn split (one wave per (pair, d tile); pairs
 // of one-chunk groups were finished there): lane l on query l % 32, its 16 values of the d tile as
 // k_pf_attn held them; in chunk order, with M the running maximum of the chunk maxima m_c, den =
@@ -855,7 +1159,7 @@ __global__ void __launch_bounds__(256) k_pf_attn_merge(PfAttn A) {
     const uint32_t rel = blockIdx.x, j = blockIdx.y * 4u + (threadIdx.x >> 6);
     if (j >= HD / 32u) return;   // whole wave
     uint32_t ks, ke;
-    pf_att_group(A, rel / kPfAttPairs, ks, ke);
+    pf_att_group(A, rel / A.per, ks, ke);
     const uint32_t nch = (ke - ks + A.kc - 1u) / A.kc;
     const uint32_t pair = A.pair0 + rel, i = pair / A.H, h = pair - i * A.H, q = 32u * i + l32;
     if (nch == 1u) return;   // whole wave
@@ -1005,6 +1309,37 @@ int pf_norm(float* h, const float* f, uint32_t nsplit, uint64_t sstride, const f
     return VRT_OK;
 }
 
+// Block l's attention norm and q|k|v projection over M rows (glu false: c, *used partials), or its FFN norm and
+// gelu_tanh(gate) * up (glu true: the activation buffer o): first h = f * (scale(f) * w_post) + h with f the sum
+// of nsplit partials (nullptr: none). Few rows run as one launch, which leaves the new residual in *spare and
+// swaps the two pointers; otherwise the norm goes through the activation buffer a.
+int pf_norm_project(vrt_g3* g, uint32_t l, bool glu, float** h, float** spare, const float* f, uint32_t nsplit, uint64_t sstride,
+                    const float* w_post, uint32_t fold_block, _Float16* a, uint32_t M, float* c, uint32_t* used, _Float16* o,
+                    G3State* st, hipStream_t s) {
+    const LayerParams& Ly = g->layers[l];
+    const uint32_t d = g->cfg.embedding_length, nkb = d / 32u;
+    const float* w_next = glu ? Ly.ffn_norm : Ly.attn_norm;
+    if (g->pf.lw.empty() || (f && nsplit != 1u) || !gm_norm_fits(M, nkb)) {
+        if (int rc = pf_norm(*h, f, nsplit, sstride, w_post, w_next, d, g->P.eps, a, st, fold_block, M, s, true)) return rc;
+        return glu ? pf_ffn_glu(g, l, a, M, o, s) : pf_project(g, l, kProjQkv, a, M, c, used, s);
+    }
+    const PfMatrix& m = glu ? g->pf.lw[l].gu : g->pf.lw[l].qkv;
+    GmArgs G{};
+    G.w = static_cast<const _Float16*>(m.h);
+    G.ws = m.s;
+    G.c = c;
+    G.o = o;
+    G.M = M;
+    G.N = glu ? 2u * g->cfg.feed_forward_length : (g->cfg.head_count + 2u) * g->cfg.head_dim;
+    G.ldc = G.N;
+    G.nkb = nkb;
+    G.npad = (G.N + kGmRowPad - 1u) / kGmRowPad * kGmRowPad;
+    const GmNorm R{*h, f, *spare, w_post, w_next, &st->nonfinite, g3_code_nonfinite(fold_block), g->P.eps};
+    if (used) *used = 1u;
+    if (f) std::swap(*h, *spare);
+    return gm_run_norm(G, R, glu, s);
+}
+
 // Block l's projection `which` over the M rows of the activation buffer a: C = A x W^T, or partial
 // z of *used K splits at c + z * M * N.
 int pf_project(vrt_g3* g, uint32_t l, uint32_t which, const _Float16* a, uint32_t M, float* c, uint32_t* used, hipStream_t s) {
@@ -1061,6 +1396,8 @@ int pf_setup(vrt_g3* g, uint32_t max_t) {
     void* q;
     if (int rc = take(static_cast<size_t>(max_t) * d * 4u, &q)) return rc;
     p.h = static_cast<float*>(q);
+    if (int rc = take(16u * static_cast<size_t>(d) * 4u, &q)) return rc;   // rows of gm_norm_fits
+    p.h2 = static_cast<float*>(q);
     // K splits only while their partials are few (gm_splits, pf_splits_q8)
     if (int rc = take(std::max<size_t>(static_cast<size_t>(max_t) * d, kGmSplitFloats) * 4u, &q)) return rc;
     p.x = static_cast<float*>(q);
@@ -1070,9 +1407,9 @@ int pf_setup(vrt_g3* g, uint32_t max_t) {
     p.g = static_cast<_Float16*>(q);
     if (int rc = take(std::max<size_t>(static_cast<size_t>(max_t) * nqkv, kGmSplitFloats) * 4u, &q)) return rc;
     p.qkv = static_cast<float*>(q);
-    if (int rc = take(static_cast<size_t>(max_t) * qw * 2u, &q)) return rc;
+    if (int rc = take(static_cast<size_t>(tp) * qw * 2u, &q)) return rc;
     p.qhi = static_cast<_Float16*>(q);
-    if (int rc = take(static_cast<size_t>(max_t) * qw * 2u, &q)) return rc;
+    if (int rc = take(static_cast<size_t>(tp) * qw * 2u, &q)) return rc;
     p.qlo = static_cast<_Float16*>(q);
     // keys and values of a segment's history and rows (f16 each): prompts longer than max_t run
     // in segments whose keys reach back to position 0 in a global block
@@ -1124,7 +1461,10 @@ template <uint32_t HD>
 static int pf_attn_launch(const PfAttn& A, bool lo, hipStream_t s) {
     PfAttn arg = A;
     void* args[] = {&arg};
-    const void* fn = lo ? reinterpret_cast<const void*>(&k_pf_attn<HD, true>) : reinterpret_cast<const void*>(&k_pf_attn<HD, false>);
+    const void* fn = A.per == 1u ? (lo ? reinterpret_cast<const void*>(&k_pf_attn_few<HD, true>)
+                                       : reinterpret_cast<const void*>(&k_pf_attn_few<HD, false>))
+                     : lo        ? reinterpret_cast<const void*>(&k_pf_attn<HD, true>)
+                                 : reinterpret_cast<const void*>(&k_pf_attn<HD, false>);
     VRT_HIP_CHECK(hipLaunchKernel(fn, dim3(A.groups * A.nch), dim3(256), args, 0, s));
     if (A.nch > 1u)   // some group has several chunks
         VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_attn_merge<HD>), dim3(A.pairs, (HD / 32u + 3u) / 4u),
@@ -1192,8 +1532,22 @@ static int pf_attention(vrt_g3* g, const LayerParams& Ly, uint32_t T, uint32_t o
     A.qo = qo;
     A.pair0 = o_row / 32u * H;
     A.pairs = (T + 31u) / 32u * H - A.pair0;
-    A.groups = (A.pairs + kPfAttPairs - 1u) / kPfAttPairs;
-    pf_att_chunks(A, p.parts);
+    // up to kPfAttFew pairs: one per workgroup, in chunks of four key tiles
+    A.per = A.pairs <= kPfAttFew ? 1u : kPfAttPairs;
+    A.groups = (A.pairs + A.per - 1u) / A.per;
+    if (A.per == 1u) {
+        uint32_t longest = 1;
+        for (uint32_t i = 0; i < A.groups; ++i) {
+            uint32_t ks, ke;
+            pf_att_group(A, i, ks, ke);
+            longest = std::max(longest, ke - ks);
+        }
+        const uint32_t most = std::min(32u, p.parts / A.pairs);   // chunks: the merge reads them four at a time
+        A.kc = std::max(128u, (longest + 32u * most - 1u) / (32u * most) * 32u);
+        A.nch = (longest + A.kc - 1u) / A.kc;
+    } else {
+        pf_att_chunks(A, p.parts);
+    }
     if (A.pairs * static_cast<uint64_t>(A.nch) > p.parts || pf_pad(qo + T) > p.tkv)
         return set_error(VRT_ERR_STATE, "prefill attention workspace too small");
     const bool lo = g->P.kv16 == 0u;   // 16-bit entries have no low parts
@@ -1221,7 +1575,8 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0, bool final) {
     const uint32_t nqkv = (H + 2u) * hd, L = g->cfg.block_count;
     const G3Params& P = g->P;
     _Float16* a = p.a;
-    float* h = p.h;
+    float* h = p.h;          // residual stream; from the last block's attention on, its last row
+    float* spare = p.h2;
     float* x = p.x;
     float* qkv = p.qkv;
     float eps = P.eps;
@@ -1243,14 +1598,11 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0, bool final) {
     uint32_t s_down = 1;                         // splits of the previous block's down projection
     for (uint32_t l = 0; l < L; ++l) {
         const LayerParams& Ly = g->layers[l];
-        {   // previous block's FFN output into the residual, then the attention norm
-            const float* f = l ? x : nullptr;
-            const float* wpost = l ? g->layers[l - 1].post_ffw : nullptr;
-            if (int rc = pf_norm(h, f, s_down, xs, wpost, Ly.attn_norm, d, eps, a, st, l ? l - 1u : 0u, T, s, true))
-                return rc;
-        }
+        // previous block's FFN output into the residual, the attention norm, q|k|v
         uint32_t s_qkv = 1;
-        if (int rc = pf_project(g, l, kProjQkv, a, T, qkv, &s_qkv, s)) return rc;
+        if (int rc = pf_norm_project(g, l, false, &h, &spare, l ? x : nullptr, s_down, xs, l ? g->layers[l - 1].post_ffw : nullptr,
+                                     l ? l - 1u : 0u, a, T, qkv, &s_qkv, nullptr, st, s))
+            return rc;
         // key coordinates: the history this segment's queries can see (from kb: position 0 in a
         // global block, the window's start rounded down to 32 in a local one), then its rows
         const uint32_t window = Ly.slots >= g->cfg.context_length ? 0u : Ly.slots;
@@ -1295,15 +1647,14 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0, bool final) {
         const bool last = l + 1u == L;
         if (last && !final) break;   // an earlier segment: the last block's keys and values are all it leaves
         const uint32_t fr = last ? 1u : T;
-        float* hr = last ? h + static_cast<uint64_t>(T - 1u) * d : h;
+        if (last) h += static_cast<uint64_t>(T - 1u) * d;
         if (int rc = pf_attention(g, Ly, T, last ? T - 1u : 0u, s, qo)) return rc;
         uint32_t so = 1;
         if (int rc = pf_project(g, l, kProjO, a, fr, x, &so, s)) return rc;
-        // attention output into the residual, then the FFN norm (the O partials of fr rows)
-        if (int rc = pf_norm(hr, x, so, static_cast<uint64_t>(fr) * d, Ly.post_attn, Ly.ffn_norm, d, eps, a, st, Ly.index,
-                             fr, s, true))
+        // attention output into the residual (the O partials of fr rows), the FFN norm, gate/up
+        if (int rc = pf_norm_project(g, l, true, &h, &spare, x, so, static_cast<uint64_t>(fr) * d, Ly.post_attn, Ly.index, a, fr,
+                                     nullptr, nullptr, p.g, st, s))
             return rc;
-        if (int rc = pf_ffn_glu(g, l, a, fr, p.g, s)) return rc;
         if (int rc = pf_project(g, l, kProjDown, p.g, fr, x, &s_down, s)) return rc;
     }
     if (!final) return VRT_OK;
@@ -1314,7 +1665,7 @@ int pf_run(vrt_g3* g, uint32_t T, uint32_t p0, bool final) {
         void* args[] = {&x, &nsplit, &d, &out};
         if (int rc = launch(reinterpret_cast<const void*>(&k_pf_sum), dim3(1), args)) return rc;
     }
-    VRT_HIP_CHECK(hipMemcpyAsync(P.hmid, h + static_cast<uint64_t>(T - 1u) * d, d * 4u, hipMemcpyDeviceToDevice, s));
+    VRT_HIP_CHECK(hipMemcpyAsync(P.hmid, h, d * 4u, hipMemcpyDeviceToDevice, s));
     return g3_enqueue_lm(g, s);
 }
 
