@@ -447,8 +447,10 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_argmax(const float* logits, u
     }
 }
 
+// (results: pinned host memory, with the failure word: the step's only way back to the host)
 __global__ void __launch_bounds__(kBdThreads) k_bd_argmax_final(const GmBest* parts, uint32_t nparts,
-                                                                vrt_argmax_result* results) {
+                                                                vrt_argmax_result* results, const G3State* st,
+                                                                uint32_t* nonfinite) {
     __shared__ float bvs[kBdThreads / 64u];
     __shared__ uint32_t bis[kBdThreads / 64u];
     const uint32_t b = blockIdx.x;
@@ -474,6 +476,26 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_argmax_final(const GmBest* pa
                 bis[0] = bis[k];
             }
         results[b] = {bis[0], bvs[0]};
+        if (b == 0u) *nonfinite = st->nonfinite;
+    }
+}
+
+// The step's rows, by value: tokens, positions and sequences to device memory, the failure word cleared, and
+// each row's embedding (one workgroup per row; the dequantised row * emb_scale, src/gemma3.cpp:1106-1136).
+struct BdRows {
+    uint32_t v[3][kBdMaxRows];
+};
+__global__ void __launch_bounds__(kBdThreads) k_bd_begin(BdRows R, uint32_t* rows, G3State* st, const uint8_t* tok_embd, uint32_t d,
+                                                         float emb_scale, float* h) {
+#pragma clang fp contract(off)
+    const uint32_t b = blockIdx.x;
+    if (threadIdx.x < 3u) rows[threadIdx.x * kBdMaxRows + b] = R.v[threadIdx.x][b];
+    if (b == 0u && threadIdx.x == 3u) st->nonfinite = 0xffffffffu;
+    const uint8_t* row = tok_embd + static_cast<uint64_t>(R.v[0][b]) * (d / 32u) * 34u;
+    for (uint32_t i = threadIdx.x; i < d; i += kBdThreads) {
+        const uint8_t* q = row + (i >> 5) * 34u;
+        const float sc = half_bits_to_float(static_cast<uint32_t>(q[0]) | (static_cast<uint32_t>(q[1]) << 8));
+        h[static_cast<uint64_t>(b) * d + i] = (sc * static_cast<float>(static_cast<int8_t>(q[2 + (i & 31u)]))) * emb_scale;
     }
 }
 
@@ -496,11 +518,10 @@ struct vrt_g3_batch {
     std::vector<BdLayer> layers;
     std::vector<void*> allocs;
     uint32_t* rows = nullptr;       // device: [3][kBdMaxRows] tokens, positions, sequences
-    uint32_t* host_rows = nullptr;  // pinned staging of the same
-    vrt_argmax_result* res = nullptr;        // device [kBdMaxRows]
+    BdRows host_rows{};             // the same on the host, a kernel argument
     vrt_argmax_result* host_res = nullptr;   // pinned
     G3State* st = nullptr;          // device: failure word (nonfinite)
-    G3State* host_st = nullptr;     // pinned
+    uint32_t* host_bad = nullptr;   // pinned: its value after the step
     float* h = nullptr;             // [rows][d] residual stream, and its other buffer (pf_norm_project)
     float* h2 = nullptr;
     float* x = nullptr;             // [kBdMaxSplits][rows][d] O / down projection partials
@@ -529,9 +550,8 @@ extern "C" int vrt_g3_batch_destroy(vrt_g3_batch* B) {
     (void)hipStreamSynchronize(B->g->ctx->stream);
     for (void* p : B->allocs) (void)hipFree(p);
     B->g->live_batches--;
-    if (B->host_rows) (void)hipHostFree(B->host_rows);
     if (B->host_res) (void)hipHostFree(B->host_res);
-    if (B->host_st) (void)hipHostFree(B->host_st);
+    if (B->host_bad) (void)hipHostFree(B->host_bad);
     delete B;
     return VRT_OK;
 }
@@ -579,8 +599,6 @@ extern "C" int vrt_g3_batch_create(vrt_g3* g, uint32_t max_seqs, uint32_t max_ct
     }
     if (int rc = bd_alloc(B, 3u * R * 4u, &p)) return fail(rc);
     B->rows = static_cast<uint32_t*>(p);
-    if (int rc = bd_alloc(B, R * sizeof(vrt_argmax_result), &p)) return fail(rc);
-    B->res = static_cast<vrt_argmax_result*>(p);
     if (int rc = bd_alloc(B, sizeof(G3State), &p)) return fail(rc);
     B->st = static_cast<G3State*>(p);
     if (int rc = bd_alloc(B, R * d * 4u, &p)) return fail(rc);
@@ -602,10 +620,8 @@ extern "C" int vrt_g3_batch_create(vrt_g3* g, uint32_t max_seqs, uint32_t max_ct
     if (int rc = bd_alloc(B, R * kBdArgParts * sizeof(GmBest), &p)) return fail(rc);
     B->amx = static_cast<GmBest*>(p);
     {
-        hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&B->host_rows), 3u * R * 4u, hipHostMallocDefault);
-        if (e == hipSuccess)
-            e = hipHostMalloc(reinterpret_cast<void**>(&B->host_res), R * sizeof(vrt_argmax_result), hipHostMallocDefault);
-        if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&B->host_st), sizeof(G3State), hipHostMallocDefault);
+        hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&B->host_res), R * sizeof(vrt_argmax_result), hipHostMallocDefault);
+        if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&B->host_bad), 64u, hipHostMallocDefault);
         if (e != hipSuccess) return fail(set_error(VRT_ERR_HIP, "hipHostMalloc failed: %s", hipGetErrorString(e)));
     }
     size_t lds = 0;
@@ -636,17 +652,22 @@ extern "C" int vrt_g3_batch_position(vrt_g3_batch* B, uint32_t seq, uint32_t* po
     return VRT_OK;
 }
 
-// Enqueues one step over the n rows already uploaded to B->rows.
+// Enqueues one step over the n rows of B->host_rows.
 static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
     vrt_g3* g = B->g;
     const vrt_g3_config& c = g->cfg;
     const uint32_t d = c.embedding_length, H = c.head_count, hd = c.head_dim, qw = H * hd, nqkv = qw + 2u * hd;
     const uint32_t L = c.block_count;
     const float eps = g->P.eps;
-    const uint32_t* tok = B->rows;
     const uint32_t* pos = B->rows + kBdMaxRows;
     const uint32_t* seq = B->rows + 2u * kBdMaxRows;
-    if (int rc = pf_embed_rows(g, tok, n, B->h, s)) return rc;
+    {
+        const uint8_t* te = g->P.tok_embd;
+        uint32_t dd = d;
+        float es = g->P.emb_scale;
+        void* args[] = {&B->host_rows, &B->rows, &B->st, &te, &dd, &es, &B->h};
+        VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_bd_begin), dim3(n), dim3(kBdThreads), args, 0, s));
+    }
     const uint64_t xs = static_cast<uint64_t>(n) * d;   // one O / down partial
     uint32_t s_down = 1;
     float *h = B->h, *spare = B->h2;
@@ -685,7 +706,7 @@ static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
         {
             void* args[] = {&A};
             uint32_t nh_max = 0;   // longest history of the step's rows in this block
-            for (uint32_t i = 0; i < n; ++i) nh_max = std::max(nh_max, std::min(B->host_rows[kBdMaxRows + i] + 1u, BL.slots));
+            for (uint32_t i = 0; i < n; ++i) nh_max = std::max(nh_max, std::min(B->host_rows.v[1][i] + 1u, BL.slots));
             if (nh_max <= kBdShort && hd % 8u == 0u) {   // whole runs of four on both sides of a RoPE pair
                 const void* fn = nh_max <= 32u ? reinterpret_cast<const void*>(&k_bd_attn_short<8>)
                                                : reinterpret_cast<const void*>(&k_bd_attn_short<16>);
@@ -727,8 +748,10 @@ static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
     {
         const GmBest* cp = B->amx;
         uint32_t np = nparts;
-        vrt_argmax_result* res = B->res;
-        void* a2[] = {&cp, &np, &res};
+        vrt_argmax_result* res = B->host_res;
+        const G3State* st = B->st;
+        uint32_t* bad = B->host_bad;
+        void* a2[] = {&cp, &np, &res, &st, &bad};
         VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_bd_argmax_final), dim3(n), dim3(kBdThreads), a2,
                                       0, s));
     }
@@ -761,18 +784,13 @@ extern "C" int vrt_g3_batch_step(vrt_g3_batch* B, const uint32_t* seqs, const ui
     }
     hipStream_t s = g->ctx->stream;
     for (uint32_t i = 0; i < n; ++i) {
-        B->host_rows[i] = tokens[i];
-        B->host_rows[kBdMaxRows + i] = B->pos[seqs[i]];
-        B->host_rows[2u * kBdMaxRows + i] = seqs[i];
+        B->host_rows.v[0][i] = tokens[i];
+        B->host_rows.v[1][i] = B->pos[seqs[i]];
+        B->host_rows.v[2][i] = seqs[i];
     }
-    B->host_st->nonfinite = 0xffffffffu;
-    VRT_HIP_CHECK(hipMemcpyAsync(B->rows, B->host_rows, 3u * kBdMaxRows * 4u, hipMemcpyHostToDevice, s));
-    VRT_HIP_CHECK(hipMemcpyAsync(&B->st->nonfinite, &B->host_st->nonfinite, 4u, hipMemcpyHostToDevice, s));
     if (int rc = bd_enqueue(B, n, s)) return bd_fail(B, seqs, n, rc, vrt_last_error());
-    VRT_HIP_CHECK(hipMemcpyAsync(B->host_res, B->res, n * sizeof(vrt_argmax_result), hipMemcpyDeviceToHost, s));
-    VRT_HIP_CHECK(hipMemcpyAsync(&B->host_st->nonfinite, &B->st->nonfinite, 4u, hipMemcpyDeviceToHost, s));
     VRT_HIP_CHECK(hipStreamSynchronize(s));
-    const G3Failure f = g3_map_failure(B->host_st->nonfinite, 0u);
+    const G3Failure f = g3_map_failure(*B->host_bad, 0u);
     if (f.code != VRT_OK) return bd_fail(B, seqs, n, f.code, f.msg);
     for (uint32_t i = 0; i < n; ++i) {
         const vrt_argmax_result r = B->host_res[i];

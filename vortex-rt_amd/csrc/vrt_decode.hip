@@ -1798,10 +1798,7 @@ int mk_read_exchange(vrt_g3* g, uint32_t which, uint64_t* out, uint64_t cap, uin
     return VRT_OK;
 }
 
-int mk_read_abort(vrt_g3* g, uint32_t* dst) {
-    VRT_HIP_CHECK(hipMemcpyAsync(dst, g->mk->P.abort_flag, 4, hipMemcpyDeviceToHost, g->ctx->stream));
-    return VRT_OK;
-}
+const uint32_t* mk_abort_word(const vrt_g3* g) { return g->mk ? g->mk->P.abort_flag : nullptr; }
 
 int mk_clear_abort(vrt_g3* g) {
     if (!g->mk) return VRT_OK;

@@ -174,8 +174,8 @@ constexpr int kMkRefused = 1000;
 int mk_run(vrt_g3* g, uint32_t nsteps);
 void mk_destroy(vrt_g3* g);
 int mk_clear_abort(vrt_g3* g);
-// Enqueues a copy of the abort word into host memory at *dst (stream-ordered, no sync).
-int mk_read_abort(vrt_g3* g, uint32_t* dst);
+// The kernel's abort word in device memory (nullptr: no such kernel).
+const uint32_t* mk_abort_word(const vrt_g3* g);
 int mk_read_exchange(vrt_g3* g, uint32_t which, uint64_t* out, uint64_t cap, uint64_t* n);
 int mk_set_trace(vrt_g3* g, bool on);
 int mk_set_kv_format(vrt_g3* g, uint32_t fmt);
@@ -187,7 +187,7 @@ int pf_setup(vrt_g3* g, uint32_t max_t);
 int pf_run(vrt_g3* g, uint32_t T, uint32_t p0 = 0, bool final = true);
 // Row-batch building blocks shared by the prefill and the batched decode (vrt_prefill.hip):
 // block l's projections over M rows as (split-K) GEMMs, its gate/up product, the residual
-// norms over rows, embedding rows, and the logits of M rows against the tied embedding table.
+// norms over rows, and the logits of M rows against the tied embedding table.
 enum PfProj : uint32_t { kProjQkv = 0, kProjO = 1, kProjDown = 2 };
 int pf_project(vrt_g3* g, uint32_t l, uint32_t which, const _Float16* a, uint32_t M, float* c, uint32_t* used, hipStream_t s);
 int pf_norm_project(vrt_g3* g, uint32_t l, bool glu, float** h, float** spare, const float* f, uint32_t nsplit, uint64_t sstride,
@@ -196,7 +196,6 @@ int pf_norm_project(vrt_g3* g, uint32_t l, bool glu, float** h, float** spare, c
 int pf_ffn_glu(vrt_g3* g, uint32_t l, const _Float16* a, uint32_t M, _Float16* o, hipStream_t s);
 int pf_norm(float* h, const float* f, uint32_t nsplit, uint64_t sstride, const float* w_post, const float* w_next,
             uint32_t n, float eps, _Float16* x, G3State* st, uint32_t block, uint32_t rows, hipStream_t s, bool into);
-int pf_embed_rows(vrt_g3* g, const uint32_t* tokens, uint32_t rows, float* h, hipStream_t s);
 int pf_lm_logits(vrt_g3* g, const _Float16* x, uint32_t M, float* logits, hipStream_t s);
 // Final residual + output norm + LM head + argmax of the current step (vrt_gemma3.hip).
 int g3_enqueue_lm(vrt_g3* g, hipStream_t s);
@@ -210,7 +209,7 @@ uint32_t tk_chunk_from(const vrt_g3* g);
 // workgroup holds on chip); the other one for earlier steps.
 int tk_run(vrt_g3* g, uint32_t nsteps, bool chunked);
 void tk_destroy(vrt_g3* g);
-int tk_read_abort(vrt_g3* g, uint32_t* dst);
+const uint32_t* tk_abort_word(const vrt_g3* g);
 int tk_clear_abort(vrt_g3* g);
 int tk_set_trace(vrt_g3* g, bool on);
 int tk_set_kv_format(vrt_g3* g, uint32_t fmt);

@@ -991,7 +991,7 @@ __global__ void __launch_bounds__(256, 1) k_pf_attn(PfAttn A) {
 // w + 4, ... of S^T and the d tiles w, w + 4, ... of O^T). The operands come straight to registers, the
 // next tile's during the current one; each wave's partial S^T goes through LDS and every wave adds the
 // four in wave order (the same scores in every wave), one barrier per tile. Softmax, results and
-// partials as in k_pf_attn. 37 rows: 11.6 -> FEWUS us.
+// partials as in k_pf_attn. 37 rows: 11.5 -> 8.3 us.
 template <uint32_t HD, bool LO>
 __global__ void __launch_bounds__(256) k_pf_attn_few(PfAttn A) {
 #pragma clang fp contract(off)
@@ -1361,16 +1361,6 @@ int pf_ffn_glu(vrt_g3* g, uint32_t l, const _Float16* a, uint32_t M, _Float16* o
     const PfLayerW* lw = g->pf.lw.empty() ? nullptr : &g->pf.lw[l];
     const uint32_t F = g->cfg.feed_forward_length;
     return pf_gemm(a, M, g->cfg.embedding_length, {{Ly.wg, F}, {Ly.wu, F}}, lw ? &lw->gu : nullptr, nullptr, o, true, nullptr, s);
-}
-
-// Embedding rows of `rows` tokens (device array) into h [rows][d].
-int pf_embed_rows(vrt_g3* g, const uint32_t* tokens, uint32_t rows, float* h, hipStream_t s) {
-    const uint8_t* te = g->P.tok_embd;
-    uint32_t d = g->cfg.embedding_length;
-    float es = g->P.emb_scale;
-    void* args[] = {&te, &tokens, &d, &es, &h};
-    VRT_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void*>(&k_pf_embed), dim3(rows), dim3(kPfThreads), args, 0, s));
-    return VRT_OK;
 }
 
 // Logits of M rows against the tied Q8_0 embedding table: logits [M][vocab] = x W_embd^T, x an

@@ -2462,10 +2462,7 @@ int tk_read_trace(vrt_g3* g, uint64_t* out, uint64_t cap, uint32_t* nwg, uint32_
     return VRT_OK;
 }
 
-int tk_read_abort(vrt_g3* g, uint32_t* dst) {
-    VRT_HIP_CHECK(hipMemcpyAsync(dst, g->tk->P.abort_flag, 4, hipMemcpyDeviceToHost, g->ctx->stream));
-    return VRT_OK;
-}
+const uint32_t* tk_abort_word(const vrt_g3* g) { return g->tk ? g->tk->P.abort_flag : nullptr; }
 
 int tk_clear_abort(vrt_g3* g) {
     if (!g->tk) return VRT_OK;
