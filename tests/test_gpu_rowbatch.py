@@ -49,9 +49,11 @@ def test_prefill_matches_decode_three_heads(ctx, narrow, rows):
     _compare(ctx, narrow, rows, TOL)
 
 
-def _compare(ctx, path, rows, tol):
+def _compare(ctx, path, rows, tol, kv="f32"):
     g = vrt.Gemma3(ctx, path)
     try:
+        if kv != "f32":
+            g.set_kv_format(kv)
         ids = synth.uniform_ids(900 + rows, rows, 2, 1000)
         print(f"[rowbatch] {rows} rows", flush=True)
         _, hp = g.prefill(ids, top_k=2, hidden=True)
@@ -113,3 +115,28 @@ def test_matvec_many_rows(ctx, k, rows):
     ref = oracle.matvec_f64(w, x, rows)
     # limb and summation error, as bounded per row in the standalone kernels' tests, over this matrix's rows
     assert np.max(np.abs(yd.read(np.float32, rows) - ref)) <= 2e-6 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("k", (32, 96, 512, 544, 2048, 2080, 8224, 16384))
+def test_matvec_input_lengths(ctx, k):
+    """Activations read by whole and partly filled passes of the limb build (128 values per wave, four waves, four
+    passes in flight), from an address that is only 4-byte aligned, with NaNs on both sides of them."""
+    rows = 67
+    w = synth.q8_matrix(7, "t", rows, k)
+    x = synth.normal_f32(8, k, 1.0)
+    host = np.full(k + 160, np.nan, dtype=np.float32)
+    host[1:1 + k] = x
+    wd, xd, yd = ctx.upload(w), ctx.upload(host), ctx.alloc(rows * 4)
+    vrt.q8_matvec(ctx, wd, 0, _span(xd, 4, x.nbytes), yd, k, rows, w_bytes=w.size)
+    ctx.sync()
+    ref = oracle.matvec_f64(w, x, rows)
+    # limb and summation error, as bounded per row in the standalone kernels' tests, over this matrix's rows
+    assert np.max(np.abs(yd.read(np.float32, rows) - ref)) <= 2e-6 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("kv,tol", (("f16", 4e-4), ("bf16", 2e-3)))
+@pytest.mark.parametrize("rows", (37, 700, 8300))
+def test_prefill_matches_decode_16bit_cache(ctx, model, kv, tol, rows):
+    """Both paths round keys and values to the cache's entries; one that lies near a tie may round the other way (the
+    tolerances are an entry's rounding, 2^-11 and 2^-8, spread over the row)."""
+    _compare(ctx, model, rows, tol, kv)

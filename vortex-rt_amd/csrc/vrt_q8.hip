@@ -77,6 +77,31 @@ __device__ __forceinline__ void q8_load_flat(const uint8_t* blk, Q8Raw& r) {
     r.d[8] = *reinterpret_cast<gu16>(a + (r.sh ? 32u : 30u));
 }
 
+__device__ __forceinline__ LimbLds limb_lds(unsigned char* smem, uint32_t K) {
+    int8_t* q = reinterpret_cast<int8_t*>(smem);
+    return {q, q + K, q + 2u * K, reinterpret_cast<float*>(q + 3u * K)};
+}
+
+// Limbs of x[0..K) for a workgroup of four waves, every wave straight from memory with up to four quads' loads in
+// flight. Staging x in LDS first cost a loop of one load at a time, a barrier and LDS that fewer workgroups could
+// share: 640 x 16384 8.9 -> 7.5 us, 2048 x 2048 6.5 -> 5.0, 8192 x 16384 88 -> 49, FFN 640 -> 2048 -> 640 11.2 -> 8.2.
+__device__ __forceinline__ void x_limbs(const float* __restrict__ x, uint32_t K, const LimbLds& L) {
+    typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
+    const uint32_t nblk = K >> 5, e = 2u * (threadIdx.x & 63u);
+    for (uint32_t q0 = threadIdx.x >> 6; q0 * 4u < nblk; q0 += 16u) {
+        f2 v[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; ++j) v[j] = *reinterpret_cast<const f2*>(x + min((q0 + 4u * j) * 128u + e, K - 2u));
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; ++j) {
+            const uint32_t quad = q0 + 4u * j;
+            const bool live = quad * 128u + e < K;
+            if (quad * 4u < nblk) limb_quad(L, quad, nblk, live ? make_float2(v[j][0], v[j][1]) : make_float2(0.0f, 0.0f));
+        }
+    }
+    __syncthreads();
+}
+
 // U row groups of the calling wave: pass u takes group g0 + u * 4, rows RPW each from v_begin. Rows past v_end
 // and blocks past nblk are neither loaded nor counted.
 template <int S, int NB, int U, typename RowFn>
@@ -97,32 +122,27 @@ __device__ __forceinline__ void mv_load(RowFn&& rowp, uint32_t nblk, uint32_t v_
     }
 }
 
-// Four waves. A row on a whole wave loads its blocks as dwords (stream_rows): 64 lanes of 34-byte blocks gain nothing
-// from 16-byte loads (1120 x 5003: 6.97 against 7.27 us); with several rows per wave they do (640 x 1536: 7.13 -> 6.74).
-// (The first rows' loads ahead of the activations, to overlap the two latencies: 1120 x 5003 7.0 -> 7.2, the FFN
-// unchanged; the activations then wait behind the weights.)
+// Four waves. Slots of several blocks per lane (4 x 5, many rows) load each block as two 16-byte units without a branch
+// (mv_load); one block per lane as dwords with stream_rows: 34-byte blocks on neighbouring lanes gain nothing from
+// the wider loads and lose where rows are many (640 x 16384: 8.9 against 11.1 us with the activations staged).
 template <int S, int NB, int U>
 __global__ void __launch_bounds__(256) k_matvec(RowSpace rs, uint64_t row_bytes, uint32_t K, const uint8_t* w_end,
                                                 const float* __restrict__ x, float* __restrict__ y,
                                                 uint32_t rows_per_wg) {
     extern __shared__ __align__(16) unsigned char smem[];
-    float* xs = reinterpret_cast<float*>(smem);
-    LimbLds L{reinterpret_cast<int8_t*>(xs + K), reinterpret_cast<int8_t*>(xs + K) + K,
-              reinterpret_cast<int8_t*>(xs + K) + 2 * K, reinterpret_cast<float*>(reinterpret_cast<int8_t*>(xs + K) + 3 * K)};
-    const uint32_t nblk = K >> 5, wave = threadIdx.x >> 6;
+    const LimbLds L = limb_lds(smem, K);
+    const uint32_t nblk = K >> 5;
     const uint32_t v0 = blockIdx.x * rows_per_wg;
     const uint32_t v1 = min(rs.total, v0 + rows_per_wg);
     if (v0 >= v1) return;
-    for (uint32_t i = threadIdx.x; i < K; i += 256u) xs[i] = x[i];
-    __syncthreads();
-    build_limbs(xs, K, L, 4u);
+    x_limbs(x, K, L);
     XLimb xl[NB];
     lane_limbs<S, NB>(L, nblk, xl);
     auto sink = [&](uint32_t v, float val) { y[v] = val; };
-    if constexpr (S == 64) {
+    if constexpr (S == 64 || NB == 1) {
         stream_rows<S, NB, U>(rs, row_bytes, nblk, w_end, xl, v0, v1, sink);
     } else {
-        const uint32_t ngroups = (v1 - v0 + 64u / S - 1u) / (64u / S);
+        const uint32_t wave = threadIdx.x >> 6, ngroups = (v1 - v0 + 64u / S - 1u) / (64u / S);
         auto rowp = [&](uint32_t v) {
             uint32_t seg, local;
             return row_ptr(rs, v, row_bytes, seg, local);
@@ -136,8 +156,8 @@ __global__ void __launch_bounds__(256) k_matvec(RowSpace rs, uint64_t row_bytes,
 }
 
 static size_t matvec_smem(uint32_t K) {
-    // xs fp32[K] + limbs int8[3K] + scales fp32[K/32], 16-byte rounded
-    return (static_cast<size_t>(K) * 4 + static_cast<size_t>(K) * 3 + (K / 32u) * 4 + 15) & ~size_t(15);
+    // limbs int8[3K] + scales fp32[K/32], 16-byte rounded
+    return (static_cast<size_t>(K) * 3 + (K / 32u) * 4 + 15) & ~size_t(15);
 }
 
 template <int S, int NB, int U>
@@ -223,9 +243,7 @@ __global__ void __launch_bounds__(256) k_ffn_gateup(const uint8_t* gate_w, const
 #pragma clang fp contract(off)
     static_assert(S <= 32, "a wave must hold whole gate/up pairs");
     extern __shared__ __align__(16) unsigned char smem[];
-    float* xs = reinterpret_cast<float*>(smem);
-    LimbLds L{reinterpret_cast<int8_t*>(xs + K), reinterpret_cast<int8_t*>(xs + K) + K,
-              reinterpret_cast<int8_t*>(xs + K) + 2 * K, reinterpret_cast<float*>(reinterpret_cast<int8_t*>(xs + K) + 3 * K)};
+    const LimbLds L = limb_lds(smem, K);
     const uint32_t nblk = K >> 5, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t slot = lane / S, sl = lane % S;
     const uint32_t v_begin = 2u * blockIdx.x * pairs_per_wg;
@@ -234,9 +252,7 @@ __global__ void __launch_bounds__(256) k_ffn_gateup(const uint8_t* gate_w, const
     constexpr uint32_t RPW = 64u / S;   // virtual rows per wave pass: RPW / 2 pairs
     const uint32_t ngroups = (v_end - v_begin + RPW - 1u) / RPW;
     auto rowp = [&](uint32_t v) { return ((v & 1u) ? up_w : gate_w) + static_cast<uint64_t>(v >> 1) * row_bytes; };
-    for (uint32_t i = threadIdx.x; i < K; i += 256u) xs[i] = x[i];
-    __syncthreads();
-    build_limbs(xs, K, L, 4u);
+    x_limbs(x, K, L);
     XLimb xl[NB];
     lane_limbs<S, NB>(L, nblk, xl);
     for (uint32_t g0 = wave; g0 < ngroups; g0 += 4u * U) {

@@ -205,44 +205,46 @@ __device__ __forceinline__ void limb3(float v, float m, int8_t& qa, int8_t& qb, 
     qc = static_cast<int8_t>(c);
 }
 
-// Cooperative limb build for xs[0..K) (LDS) by all threads of the block. A block of 32
-// elements is one 16-lane row of a wave (two elements per lane), so its amax is a DPP
-// reduction within the row and a wave covers four blocks per pass. A non-finite element
-// enters the amax as +inf and makes the block scale NaN. `nwaves` is the workgroup's wave
-// count. Ends with __syncthreads().
+// Limbs of the four blocks of quad `quad` by one wave: a block of 32 elements is one 16-lane row
+// (v: the lane's two elements, 0 past nblk), so its amax is a DPP reduction within the row. A
+// non-finite element enters the amax as +inf and makes the block scale NaN.
+__device__ __forceinline__ void limb_quad(const LimbLds& L, uint32_t quad, uint32_t nblk, float2 v) {
+    const uint32_t lane = threadIdx.x & 63u, blk = quad * 4u + (lane >> 4);
+    const uint32_t k = blk * 32u + 2u * (lane & 15u);
+    auto mag = [](float x) { return __builtin_isfinite(x) ? fabsf(x) : INFINITY; };
+    float m = fmaxf(mag(v.x), mag(v.y));
+    m = fmaxf(m, dpp_mov<0xB1>(m));    // quad_perm [1,0,3,2]
+    m = fmaxf(m, dpp_mov<0x4E>(m));    // quad_perm [2,3,0,1]
+    m = fmaxf(m, dpp_mov<0x141>(m));   // row_half_mirror
+    m = fmaxf(m, dpp_mov<0x140>(m));   // row_mirror: every lane of the row holds its amax
+    int8_t qa0 = 0, qb0 = 0, qc0 = 0, qa1 = 0, qb1 = 0, qc1 = 0;
+    float s = 0.0f;
+    if (m == INFINITY) {
+        s = __builtin_nanf("");
+    } else if (m >= 1e-30f) {
+        s = m * (1.0f / 127.0f);
+        limb3(v.x, m, qa0, qb0, qc0);
+        limb3(v.y, m, qa1, qb1, qc1);
+    }
+    if (blk < nblk) {
+        auto pk = [](int8_t lo, int8_t hi) {
+            return static_cast<uint16_t>(static_cast<uint8_t>(lo) | (static_cast<uint16_t>(static_cast<uint8_t>(hi)) << 8));
+        };
+        *reinterpret_cast<uint16_t*>(L.a + k) = pk(qa0, qa1);
+        *reinterpret_cast<uint16_t*>(L.b + k) = pk(qb0, qb1);
+        *reinterpret_cast<uint16_t*>(L.c + k) = pk(qc0, qc1);
+        if ((lane & 15u) == 0u) L.s[blk] = s;
+    }
+}
+
+// Cooperative limb build for xs[0..K) (LDS) by all threads of the block, four blocks per wave and
+// pass. `nwaves` is the workgroup's wave count. Ends with __syncthreads().
 __device__ __forceinline__ void build_limbs(const float* xs, uint32_t K, LimbLds L, uint32_t nwaves) {
-    const uint32_t nblk = K >> 5;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = threadIdx.x >> 6;
-    for (uint32_t quad = wave; quad * 4u < nblk; quad += nwaves) {
+    const uint32_t nblk = K >> 5, lane = threadIdx.x & 63u;
+    for (uint32_t quad = threadIdx.x >> 6; quad * 4u < nblk; quad += nwaves) {
         const uint32_t blk = quad * 4u + (lane >> 4);
-        const bool live = blk < nblk;
-        const uint32_t k = blk * 32u + 2u * (lane & 15u);
-        const float2 v = live ? *reinterpret_cast<const float2*>(xs + k) : make_float2(0.0f, 0.0f);
-        auto mag = [](float x) { return __builtin_isfinite(x) ? fabsf(x) : INFINITY; };
-        float m = fmaxf(mag(v.x), mag(v.y));
-        m = fmaxf(m, dpp_mov<0xB1>(m));    // quad_perm [1,0,3,2]
-        m = fmaxf(m, dpp_mov<0x4E>(m));    // quad_perm [2,3,0,1]
-        m = fmaxf(m, dpp_mov<0x141>(m));   // row_half_mirror
-        m = fmaxf(m, dpp_mov<0x140>(m));   // row_mirror: every lane of the row holds its amax
-        int8_t qa0 = 0, qb0 = 0, qc0 = 0, qa1 = 0, qb1 = 0, qc1 = 0;
-        float s = 0.0f;
-        if (m == INFINITY) {
-            s = __builtin_nanf("");
-        } else if (m >= 1e-30f) {
-            s = m * (1.0f / 127.0f);
-            limb3(v.x, m, qa0, qb0, qc0);
-            limb3(v.y, m, qa1, qb1, qc1);
-        }
-        if (live) {
-            auto pk = [](int8_t lo, int8_t hi) {
-                return static_cast<uint16_t>(static_cast<uint8_t>(lo) | (static_cast<uint16_t>(static_cast<uint8_t>(hi)) << 8));
-            };
-            *reinterpret_cast<uint16_t*>(L.a + k) = pk(qa0, qa1);
-            *reinterpret_cast<uint16_t*>(L.b + k) = pk(qb0, qb1);
-            *reinterpret_cast<uint16_t*>(L.c + k) = pk(qc0, qc1);
-            if ((lane & 15u) == 0u) L.s[blk] = s;
-        }
+        limb_quad(L, quad, nblk,
+                  blk < nblk ? *reinterpret_cast<const float2*>(xs + blk * 32u + 2u * (lane & 15u)) : make_float2(0.0f, 0.0f));
     }
     __syncthreads();
 }
