@@ -134,6 +134,20 @@ def test_matvec_input_lengths(ctx, k):
     assert np.max(np.abs(yd.read(np.float32, rows) - ref)) <= 2e-6 * np.max(np.abs(ref))
 
 
+@pytest.mark.parametrize("n", (1, 1023, 1025, 8191, 8192, 8193, 10240, 2097152, 2100001))
+def test_argmax_lengths(ctx, n):
+    """One workgroup and several, runs that end inside, at and past a pass; ties and NaNs across runs."""
+    x = synth.normal_f32(n, n, 1.0)
+    x[n // 3::97] = np.nan
+    x[[n // 2, n - 1]] = 9.0
+    xd, out = ctx.upload(x), ctx.alloc(8)
+    vrt.argmax(ctx, xd, n, out)
+    ctx.sync()
+    got = out.read(np.uint32, 2)
+    index, value = oracle.argmax(x)
+    assert got[0] == index and got[1:].view(np.float32)[0] == np.float32(value)
+
+
 @pytest.mark.parametrize("kv,tol", (("f16", 4e-4), ("bf16", 2e-3)))
 @pytest.mark.parametrize("rows", (37, 700, 8300))
 def test_prefill_matches_decode_16bit_cache(ctx, model, kv, tol, rows):

