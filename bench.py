@@ -167,7 +167,7 @@ def prefill_flops(cfg, T: int) -> int:
 
 
 MFMA_F16_PEAK_TFLOPS = 2500.0
-PREFILL_SEGMENT = 2048   # positions per batched prefill pass (longer prompts run as segments)
+PREFILL_SEGMENT = 8192   # positions per batched prefill pass (longer prompts run as segments)
 
 
 def prefill_bench(ctx, g, cfg, T: int = 512, reps: int = 5):

@@ -7,14 +7,17 @@
 // prefill's kernels, vrt_prefill.hip): the weights stream once per step for all n rows, which
 // is what makes a batch cheaper per token than n batch-1 steps. Per block:
 //   k_pf_norm_w   residual fold of the previous block's FFN output + attention RMSNorm (rows)
-//   GEMM          q|k|v of the n rows (K split, partials summed by the consumer)
-//   k_bd_attn     per (history chunk, row): QK-norm, RoPE at the row's position, KV append to
-//                 the row's sequence, chunk of the attention (max, sum, weighted V per head)
-//   k_bd_merge    per (head, row): the chunks combined, as f16 hi/lo GEMM input
+//   GEMM          q|k|v of the n rows (up to 16 rows the norm and the GEMM are one launch)
+//   k_bd_attn_short  when no row's history in the block is past 256 positions, per (head, row):
+//                 QK-norm, RoPE at the row's position, KV append to the row's sequence, attention;
+//                 else k_bd_attn, per (history chunk, row), the same with a chunk of the attention
+//                 (max, sum, weighted V per head), and k_bd_merge, per (head, row): the chunks
+//                 combined, as f16 hi/lo GEMM input
 //   GEMM          O projection; k_pf_norm_w (post-attention norm + residual + FFN norm)
-//   GEMM          gelu_tanh(gate) * up; GEMM down projection
+//   GEMM          gelu_tanh(gate) * up (with its norm up to 16 rows); GEMM down projection
 // then the final residual + output norm (k_pf_norm_w), the logits of the n rows against the
-// tied embedding table (GEMM) and a greedy argmax per row (k_bd_argmax, k_bd_argmax_final).
+// tied embedding table with every workgroup's greedy candidates (k_gm_lm; or the general GEMM and
+// k_bd_argmax) and k_bd_argmax_final. k_bd_begin takes the step's rows as launch arguments.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
