@@ -7,9 +7,12 @@ oracle's, as on the single-sequence path. (The oracle's smallest top-2 margin ov
 7.1e-4 of the top logit in the tiny-model cases and 2.9e-3 at the full shape; each row's margin
 is printed with the failure.) Sequences join at different steps, so every step mixes rows at
 different positions, local windows and chunk counts."""
+import os
+
 import numpy as np
 import pytest
 
+import gguf
 import oracle
 import synth
 import vrt
@@ -199,4 +202,52 @@ def test_batch_errors(ctx, tiny_model):
         finally:
             b.close()
     finally:
+        g.close()
+
+
+def _poisoned(src, dst, token, d_model):
+    """A copy of the model whose embedding row of `token` starts with a block of NaN scale: the token's hidden state
+    is not finite, and its logit is NaN (never the greedy token)."""
+    f = gguf.GgufFile.open(src)
+    at = f.data_offset + f.tensors["token_embd.weight"].offset + token * (d_model // 32) * 34
+    buf = bytearray(f._mm[:])
+    f.close()
+    buf[at:at + 2] = (0x7E00).to_bytes(2, "little")
+    with open(dst, "wb") as fp:
+        fp.write(buf)
+    return dst
+
+
+@pytest.mark.parametrize("fail_at", (0, 5, 40))
+def test_batch_restarts_after_a_failed_step(ctx, tiny_model, model_dir, fail_at):
+    """A step whose hidden state is not finite fails and puts its sequences back to position 0. What it left in their
+    caches (NaN keys and values at the failing position, in the ring slot of it in the local blocks) is not part of
+    any later step: the restarted sequences repeat, bit for bit, what a fresh batch gives, up to the failing
+    position and past it (one pass of the short attention and several)."""
+    bad = 999
+    path = _poisoned(tiny_model, os.path.join(str(model_dir), "tiny_poisoned.gguf"), bad, synth.TINY["d_model"])
+    g = vrt.Gemma3(ctx, path)
+    toks = synth.uniform_ids(700, 2 * (fail_at + 6), 2, 900).reshape(-1, 2)
+
+    def run(b):
+        out = []
+        for t in toks:
+            idx, val = b.step([0, 1], t)
+            out.append((idx, val, b.logits(0), b.logits(1)))
+        return out
+    fresh, b = vrt.Gemma3Batch(g, 2, 64), vrt.Gemma3Batch(g, 2, 64)
+    try:
+        print(f"[batch] failed step at position {fail_at}", flush=True)
+        want = run(fresh)
+        for t in toks[:fail_at]:
+            b.step([0, 1], t)
+        with pytest.raises(RuntimeError):
+            b.step([0, 1], [bad, 7])
+        assert b.position(0) == 0 and b.position(1) == 0
+        for p, (got, ref) in enumerate(zip(run(b), want)):
+            for x, y in zip(got, ref):
+                np.testing.assert_array_equal(x, y, err_msg=f"position {p}")
+    finally:
+        b.close()
+        fresh.close()
         g.close()

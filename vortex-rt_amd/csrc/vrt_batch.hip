@@ -245,8 +245,10 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn(BdAttn A) {
 // loaded together, the first pass's before the q|k|v row is added up), and keeps its own maximum, double sum
 // and weighted values (:1602-1696); the four are combined in double through LDS behind the only
 // barrier. The head-0 workgroup appends k and v at slot pos % slots (:1590-1600); the current position's k and
-// v come from registers, never from the cache. The launch is one memory latency, not bandwidth: staged through
-// LDS, with one wave's softmax over shuffles, it took 8.9 us at 8 rows.
+// v, and those of the pass's slots past it (weight 0), come from registers, never from the cache: the clamped row
+// of a slot past it is the row being written, which may still hold a failed step's NaN, and 0 x NaN would be
+// in the sum. The launch is one memory latency, not bandwidth: staged through LDS, with one wave's softmax over
+// shuffles, it took 8.9 us at 8 rows.
 constexpr uint32_t kBdShort = 256;   // four passes; longer histories gain from more workgroups than (heads, rows)
 template <int NU>
 __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
@@ -325,7 +327,7 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
             const uint32_t t = t0 + wave + NW * u;
             float d = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) d += x[0][e] * (t == p ? x[1][e] : kr[u][e]);
+            for (int e = 0; e < 4; ++e) d += x[0][e] * (t < p ? kr[u][e] : x[1][e]);
             d = wave_sum(live ? d : 0.0f) * A.attn_scale;
             s[u] = t <= p ? d : -INFINITY;
             mx = fmaxf(mx, s[u]);
@@ -342,7 +344,7 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
             const float w = expf(s[u] - mx);
             l += static_cast<double>(w);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] += w * (t == p ? v[e] : vr[u][e]);
+            for (int e = 0; e < 4; ++e) acc[e] += w * (t < p ? vr[u][e] : v[e]);
         }
     }
     if (live) *reinterpret_cast<f4*>(&s_acc[wave][i]) = acc;
