@@ -154,3 +154,32 @@ def test_prefill_matches_decode_16bit_cache(ctx, model, kv, tol, rows):
     """Both paths round keys and values to the cache's entries; one that lies near a tie may round the other way (the
     tolerances are an entry's rounding, 2^-11 and 2^-8, spread over the row)."""
     _compare(ctx, model, rows, tol, kv)
+
+
+@pytest.mark.parametrize("base", (0, 1, 2, 3))
+def test_weights_at_any_address(ctx, base):
+    """Only the weights' offsets have to be multiples of four; the buffer itself may start anywhere (a view of a
+    larger one). One kernel per load form: the FFN's gate/up rows, many rows of 20 blocks, a plain matrix."""
+    k, ffn, out, many = 640, 96, 64, 32768
+    x = synth.normal_f32(12, k, 1.0)
+    parts = [synth.q8_matrix(13, n, r, c) for n, r, c in (("gate", ffn, k), ("up", ffn, k), ("down", out, ffn), ("big", many, k))]
+    offs = np.concatenate([[0], np.cumsum([(p.size + 3) // 4 * 4 for p in parts])]).astype(int)
+    host = np.zeros(offs[-1] + 64, dtype=np.uint8)
+    for p, o in zip(parts, offs):
+        host[base + o:base + o + p.size] = p
+    wd, xd = ctx.upload(host), ctx.upload(x)
+    w = _span(wd, base, int(offs[-1]) + 8)
+    ws, y, yb = ctx.alloc(2 * ffn * 4), ctx.alloc(out * 4), ctx.alloc(many * 4)
+    vrt.q8_ffn(ctx, w, *(int(o) for o in offs[:3]), k, ffn, out, xd, ws, y)
+    vrt.q8_matvec(ctx, w, int(offs[3]), xd, yb, k, many)
+    ctx.sync()
+    up = oracle.matvec_f64(parts[1], x, ffn)
+    gate = oracle.matvec_f64(parts[0], x, ffn)
+    h = 0.5 * gate * (1.0 + np.tanh(0.7978845608028654 * (gate + 0.044715 * gate ** 3))) * up
+    got = ws.read(np.float32, 2 * ffn)
+    down = oracle.matvec_f64(parts[2], h.astype(np.float32), out)
+    # limb and summation error, as in test_matvec_many_rows; h: that of its two factors and the GELU's own; the
+    # product of h by the down matrix carries h's over
+    for a, ref, tol in ((got[ffn:], up, 2e-6), (got[:ffn], h, 6e-6), (y.read(np.float32, out), down, 8e-6),
+                        (yb.read(np.float32, many), oracle.matvec_f64(parts[3], x, many), 2e-6)):
+        assert np.max(np.abs(a - ref)) <= tol * np.max(np.abs(ref))

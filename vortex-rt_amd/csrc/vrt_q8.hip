@@ -60,7 +60,8 @@ bool mv_shape(uint32_t K, MvShape* out) {
 
 // q8_load without a branch: the scale, eight dwords from (block + 2) & ~3 and the 16 bits after them (used
 // where the quants start two bytes into the first dword; else a pair inside the block), all within
-// the 34 bytes. A load behind a branch waits for every load before it.
+// the 34 bytes. A load behind a branch waits for every load before it. For blocks at even addresses only
+// (q8_even): at an odd one the quants would start one or three bytes into the first dword.
 __device__ __forceinline__ void q8_load_flat(const uint8_t* blk, Q8Raw& r) {
     typedef uint32_t v4 __attribute__((ext_vector_type(4), aligned(4)));
     typedef const __attribute__((address_space(1))) v4* gv4;
@@ -76,6 +77,8 @@ __device__ __forceinline__ void q8_load_flat(const uint8_t* blk, Q8Raw& r) {
     }
     r.d[8] = *reinterpret_cast<gu16>(a + (r.sh ? 32u : 30u));
 }
+
+static bool q8_even(const uint8_t* a) { return (reinterpret_cast<uintptr_t>(a) & 1u) == 0u; }   // blocks are 34 bytes apart
 
 __device__ __forceinline__ LimbLds limb_lds(unsigned char* smem, uint32_t K) {
     int8_t* q = reinterpret_cast<int8_t*>(smem);
@@ -182,7 +185,9 @@ int launch_matvec(hipStream_t stream, const uint8_t* const* bases, const uint32_
     VRT_REQUIRE(nseg >= 1 && nseg <= static_cast<uint32_t>(kMaxSeg), "Q8 matvec segment count must be 1..%d", kMaxSeg);
     RowSpace rs{};
     uint64_t total = 0;
+    bool even = true;
     for (uint32_t i = 0; i < nseg; ++i) {
+        even = even && q8_even(bases[i]);
         rs.base[i] = bases[i];
         rs.rows[i] = rows[i];
         rs.first[i] = static_cast<uint32_t>(total);
@@ -196,7 +201,7 @@ int launch_matvec(hipStream_t stream, const uint8_t* const* bases, const uint32_
     // Many rows of 17 to 20 blocks: slots of 4 lanes x 5 blocks keep 85 to 100% of the lanes on a block, where one
     // block on each of 32 lanes keeps 53 to 62% (262144 x 640: 50 -> 38 us). Fewer rows than fill the chip
     // that way are better spread thin.
-    if (sh.S == 32 && K / 32u <= 20u && total >= 32768u) return launch_mv_t<4, 5, 1>(stream, rs, row_bytes, K, w_end, x, y);
+    if (sh.S == 32 && K / 32u <= 20u && total >= 32768u && even) return launch_mv_t<4, 5, 1>(stream, rs, row_bytes, K, w_end, x, y);
     switch (sh.S * 16 + sh.NB) {
     case 1 * 16 + 1: return launch_mv_t<1, 1, 2>(stream, rs, row_bytes, K, w_end, x, y);
     case 2 * 16 + 1: return launch_mv_t<2, 1, 2>(stream, rs, row_bytes, K, w_end, x, y);
@@ -473,8 +478,8 @@ __global__ void __launch_bounds__(256) k_dequantize_any(const uint8_t* __restric
 }
 
 // The gate/up launch of the fused FFN into the workspace image ws = [h | up]: gelu_tanh(gate) *
-// up into ws[0..F), up into ws[F..2F). K of more than 32 blocks (64-lane row slots) runs the
-// gate/up matvec and the GELU as two kernels.
+// up into ws[0..F), up into ws[F..2F). K of more than 32 blocks (64-lane row slots), and matrices at an odd
+// address, run the gate/up matvec and the GELU as two kernels.
 static int launch_ffn_gateup(hipStream_t stream, const uint8_t* gate_w, const uint8_t* up_w, uint32_t K, uint32_t F,
                              const uint8_t* w_end, const float* x, float* ws) {
     float* h = ws;
@@ -493,7 +498,7 @@ static int launch_ffn_gateup(hipStream_t stream, const uint8_t* gate_w, const ui
         VRT_HIP_CHECK(hipGetLastError());
         return VRT_OK;
     };
-    switch (sh.S) {
+    switch (q8_even(gate_w) && q8_even(up_w) ? sh.S : 64) {
     case 1: return go(k_ffn_gateup<1, 1, 2>, 1);
     case 2: return go(k_ffn_gateup<2, 1, 2>, 2);
     case 4: return go(k_ffn_gateup<4, 1, 2>, 4);
