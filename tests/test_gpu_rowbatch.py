@@ -183,3 +183,27 @@ def test_weights_at_any_address(ctx, base):
     for a, ref, tol in ((got[ffn:], up, 2e-6), (got[:ffn], h, 6e-6), (y.read(np.float32, out), down, 8e-6),
                         (yb.read(np.float32, many), oracle.matvec_f64(parts[3], x, many), 2e-6)):
         assert np.max(np.abs(a - ref)) <= tol * np.max(np.abs(ref))
+
+
+def test_prefill_repeats_after_other_prompts(ctx, model, tmp_path):
+    """A prompt's results do not depend, in any bit, on the prompts before it: the query tile that its length leaves
+    partly filled holds another prompt's queries in the rows past the end. QK-norm weights of 2 spread the scores
+    so far that those rows' maxima would move where the prompt's own do not."""
+    path = os.path.join(str(tmp_path), "spread.gguf")
+    hd = SHAPE["head_dim"]
+    synth.edit_gguf(model, path, f32={f"blk.{l}.attn_{n}_norm.weight": np.full(hd, 2.0, np.float32) for l in range(2) for n in "qk"})
+    ids = synth.uniform_ids(41, 300, 2, 1000)
+    g = vrt.Gemma3(ctx, path)
+    try:
+        def run():
+            (i, v), hid = g.prefill(ids, top_k=2, hidden=True)
+            return hid, g.logits()
+        runs = [run()]
+        for seed in (42, 43, 44, 45):
+            g.prefill(synth.uniform_ids(seed, 320, 2, 1000), top_k=0)
+            runs.append(run())
+        for hid, logits in runs[1:]:
+            np.testing.assert_array_equal(hid, runs[0][0])
+            np.testing.assert_array_equal(logits, runs[0][1])
+    finally:
+        g.close()

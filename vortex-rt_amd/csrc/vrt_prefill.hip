@@ -762,7 +762,8 @@ __global__ void __launch_bounds__(256, 1) k_pf_attn(PfAttn A) {
                          lane * 16u, lv + (n & 1u) * (UV * 1024u) + u * 1024u);
     };
     load_k(0u);
-    // the queries (B operand of S^T); rows past T hold stale values, and their results are never written
+    // the queries (B operand of S^T); rows past T hold stale values, which stay in their own lanes (settle), and
+    // their results are never written
     half8 qb[KS][2];
     {
         const uint64_t o = (static_cast<uint64_t>(i) * A.H + h) * (KS * 512u) + 8u * lane;
@@ -833,7 +834,9 @@ __global__ void __launch_bounds__(256, 1) k_pf_attn(PfAttn A) {
             }
         }
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        if (__any(tmax > m + kPfAttSlack)) {   // whole wave; a query with nothing visible yet has m = -inf
+        // whole wave, but only for its queries: rows past T hold another prompt's, which would decide how this
+        // one is rounded. A query with nothing visible yet has m = -inf.
+        if (__any(q < T && tmax > m + kPfAttSlack)) {
             const float mn = fmaxf(m, tmax);
             alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
             grown = n != 0u;   // O^T is zero before the first tile
