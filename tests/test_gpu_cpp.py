@@ -35,6 +35,10 @@ def test_cpp_ffn():
     assert "ffn_test ok" in _run("ffn_test")
 
 
+def test_gelu_error():
+    assert "gelu_error_test ok" in _run("gelu_error_test")
+
+
 def test_cpp_gemma3_model(tiny_model):
     prompt = [2, 17, 301, 5]
     got = json.loads(_run("gemma3_test", tiny_model, 10, *prompt).strip().splitlines()[-1])

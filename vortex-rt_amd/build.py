@@ -92,14 +92,19 @@ CPP_TESTS = os.path.join(REPO, "tests", "cpp")
 
 
 def build_cpp_tests(jobs: int = 8) -> list:
-    """The C++ test programs of tests/cpp against libvortexrt.so, into tests/cpp/_build."""
-    srcs = sorted(glob.glob(os.path.join(CPP_TESTS, "*.cpp")))
+    """The test programs of tests/cpp, into tests/cpp/_build: C++ against libvortexrt.so, HIP on the device
+    functions of csrc's headers."""
+    srcs = sorted(glob.glob(os.path.join(CPP_TESTS, "*.cpp")) + glob.glob(os.path.join(CPP_TESTS, "*.hip")))
     out_dir = os.path.join(CPP_TESTS, "_build")
     os.makedirs(out_dir, exist_ok=True)
     rpath = "-Wl,-rpath,$ORIGIN/../../../vortex-rt_amd/_build"
 
     def one(src):
         exe = os.path.join(out_dir, os.path.basename(src)[:-4])
+        if src.endswith(".hip"):
+            _run([HIPCC] + HIP_FLAGS + ["-o", exe + ".tmp", src])
+            os.replace(exe + ".tmp", exe)
+            return exe
         _run(["g++"] + CXX_FLAGS + ["-I" + CPP_TESTS, "-I" + CSRC, "-o", exe + ".tmp", src, "-L" + OUT, "-lvortexrt",
                                     "-lvrt_hip", rpath])
         os.replace(exe + ".tmp", exe)

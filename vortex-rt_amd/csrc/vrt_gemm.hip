@@ -22,14 +22,6 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-// gelu_tanh(gate) * up (shaders/gelu_mul.comp:23-31) with 0.5 x (1 + tanh u) = x / (1 + e^(-2u)): one
-// hardware exponential and one reciprocal (1 ulp each) instead of tanhf, and no cancellation where
-// tanh u is close to -1. Below the exponential's overflow the quotient is 0.
-__device__ __forceinline__ float gm_gelu_mul(float x, float up) {
-    const float t = x * (-2.302208198f - 0.1029432397f * (x * x));   // -2 u log2 e
-    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t)) * up;
-}
-
 // 1.0f / std::sqrt(float(sum_sq / n) + eps) (src/gemma3.cpp:967-983).
 __device__ __forceinline__ float gm_rms_scale(double ss, uint32_t n, float eps) {
 #pragma clang fp contract(off)

@@ -39,6 +39,22 @@ __device__ __forceinline__ void gm_split(float x, _Float16& hi, _Float16& lo) {
     lo = static_cast<_Float16>(x - static_cast<float>(hi));
 }
 
+// gelu_tanh(gate) * up (shaders/gelu_mul.comp:23-31) with 0.5 x (1 + tanh u) = x / (1 + e^(-2u)), which has no
+// cancellation where tanh u is close to -1. The hardware's exponential and reciprocal are approximate to 1 ulp: the
+// exponential's error counts by 1 - s of the quotient's share s, and the quotient is corrected once with the
+// rounding error of 1 + e carried along. Error against 64 bits over gates N(0, 1), 2-norm: 3.7e-8; with tanhf in the
+// reference's order of operations 4.5e-8; without the correction 5.3e-8. Time of the function alone: 0.73 of
+// tanhf's, 1.8 times that without the correction. Past the exponential's range the quotient is 0.
+__device__ __forceinline__ float gm_gelu_mul(float x, float up) {
+#pragma clang fp contract(off)
+    const float t = x * __builtin_fmaf(-0.1029432397f, x * x, -2.302208198f);   // -2 u log2 e
+    const float e = __builtin_amdgcn_exp2f(fminf(t, 126.0f)), d = 1.0f + e;
+    const float lo = e <= 1.0f ? e - (d - 1.0f) : 1.0f - (d - e);   // 1 + e = d + lo
+    const float r = __builtin_amdgcn_rcpf(d), q = x * r;
+    const float y = __builtin_fmaf(__builtin_fmaf(-q, lo, __builtin_fmaf(-d, q, x)), r, q);
+    return (t > 126.0f ? x * 0.0f : y) * up;
+}
+
 // 64 lanes x 16 (or 4) bytes from base + voff straight into LDS at lds + lane * 16 (or 4). In
 // assembly so that the waits are placed by hand: the compiler would wait for every such load in
 // flight before any LDS read.
