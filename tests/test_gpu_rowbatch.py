@@ -1,6 +1,7 @@
 """The row-batch kernels at the row counts where their tiles, K splits and dispatch rules change: a
 prompt prefilled at once against the same positions decoded one by one (other kernels, themselves
 checked against the oracle), at the 270M block shape with a small vocabulary."""
+import ctypes
 import os
 
 import numpy as np
@@ -205,5 +206,30 @@ def test_prefill_repeats_after_other_prompts(ctx, model, tmp_path):
         for hid, logits in runs[1:]:
             np.testing.assert_array_equal(hid, runs[0][0])
             np.testing.assert_array_equal(logits, runs[0][1])
+    finally:
+        g.close()
+
+
+def test_executor_memory_follows_its_context(ctx, tmp_path):
+    """An executor of 512 positions does not hold the attention partials of 8192 (268 MB at 4 heads of 256): its weights
+    twice over (30 MB), the row buffers and K-split partials of 512 rows (45 MB) and 17 MB of partials, rounded up by
+    the allocator."""
+    hip = ctypes.CDLL("libamdhip64.so.7")   # the runtime that libvrt_hip.so is linked to
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+    path = os.path.join(str(tmp_path), "short.gguf")
+    synth.write_gemma3_gguf(path, seed=23, **dict(SHAPE, context=512))
+    vrt.Gemma3(ctx, path).close()   # what the first executor of a process allocates once
+    free = free_bytes()
+    g = vrt.Gemma3(ctx, path)
+    try:
+        took = free - free_bytes()
+        print(f"[rowbatch] 512 positions: {took / 1e6:.0f} MB", flush=True)
+        assert took < 150e6
+        ids = synth.uniform_ids(47, 512, 2, 1000)
+        g.prefill(ids, top_k=1)   # 64 pairs in up to 8 chunks
     finally:
         g.close()

@@ -646,7 +646,8 @@ __global__ void __launch_bounds__(kPfThreads) k_pf_kv_hist(const float* kc, cons
 // and B[k = 8 (l / 32) + j][n = l % 32], j < 8; result r of lane l is C[8 (r / 4) + 4 (l / 32) +
 // r % 4][l % 32].
 constexpr uint32_t kPfAttPairs = 4;        // pairs per workgroup (waves)
-constexpr uint32_t kPfAttParts = 8192;     // partials kept, at least
+constexpr uint32_t kPfAttParts = 8192;     // partials kept, at most, if that is one per pair
+constexpr uint32_t kPfAttMaxChunks = 64;   // chunks of a range, at most (of two key tiles, at least)
 constexpr uint32_t kPfAttFew = 32;         // pairs of a k_pf_attn_few launch, at most
 constexpr float kPfAttSlack = 8.0f;
 struct PfAttn {
@@ -1410,7 +1411,10 @@ int pf_setup(vrt_g3* g, uint32_t max_t) {
     void** kv[] = {&p.khi, &p.klo, &p.vhi, &p.vlo};
     for (void** b : kv)
         if (int rc = take(static_cast<size_t>(hd) * p.tkv * 2u, b)) return rc;
-    p.parts = std::max(kPfAttParts, H * ((max_t + 31u) / 32u));
+    // as many partials as any launch of this executor can cut its ranges into (context 512: 512 of 32 KB
+    // at 4 heads of 256), up to kPfAttParts
+    const uint32_t pairs = H * ((max_t + 31u) / 32u), cut = std::min(kPfAttMaxChunks, (p.tkv + 63u) / 64u);
+    p.parts = std::max(pairs, std::min(kPfAttParts, (pairs + kPfAttPairs - 1u) / kPfAttPairs * kPfAttPairs * cut));
     if (int rc = take(static_cast<size_t>(p.parts) * 32u * hd * 4u, &q)) return rc;
     p.opart = static_cast<float*>(q);
     if (int rc = take(static_cast<size_t>(p.parts) * 32u * 4u, &q)) return rc;
@@ -1483,7 +1487,7 @@ static void pf_att_chunks(PfAttn& A, uint32_t max_parts) {
     uint32_t best_kc = 0;
     for (uint32_t n = 1; n <= longest; ++n) {   // n chunks of the longest range
         const uint32_t tiles = (longest + n - 1u) / n;
-        if (n > 1u && (tiles < 2u || n > 64u || (longest + tiles - 1u) / tiles != n)) continue;
+        if (n > 1u && (tiles < 2u || n > kPfAttMaxChunks || (longest + tiles - 1u) / tiles != n)) continue;
         if (n > 1u && static_cast<uint64_t>(A.groups) * kPfAttPairs * n > max_parts) break;
         uint64_t units = 0;
         for (uint32_t g = 0; g < A.groups; ++g) units += (len[g] + tiles - 1u) / tiles;
