@@ -233,3 +233,68 @@ def test_executor_memory_follows_its_context(ctx, tmp_path):
         g.prefill(ids, top_k=1)   # 64 pairs in up to 8 chunks
     finally:
         g.close()
+
+
+# Batched steps against single-sequence decode. Shapes by what decides their kernels: K blocks of the LM head (20, and 24,
+# 36: two groups of five per wave; 41: past k_gm_lm, the general GEMM and argmax, both of its tile widths), head
+# dimensions without expanded weights (40, and 36, where a run of four straddles the RoPE halves). 26003 rows make
+# 1626 tiles, the last of three rows: three or four in each of 512 chunks, six or seven in each of 256.
+BATCH = dict(
+    k20=dict(vocab=26003),
+    k24=dict(d_model=768, vocab=1003),
+    k36=dict(d_model=1152, vocab=26003),
+    k41=dict(d_model=1312, head_dim=64, ffn=256, vocab=1003),
+    k41w=dict(d_model=1312, head_dim=64, ffn=256, vocab=16384),
+    hd40=dict(d_model=320, head_dim=40, ffn=640, vocab=1003),
+    hd36=dict(d_model=288, n_heads=8, head_dim=36, ffn=576, vocab=1003),
+)
+
+
+@pytest.fixture(scope="module")
+def batch_model(tmp_path_factory):
+    d = str(tmp_path_factory.mktemp("batch"))
+
+    def get(key, **kw):
+        path = os.path.join(d, key + ".gguf")
+        if not os.path.exists(path):
+            synth.write_gemma3_gguf(path, seed=31, **dict(SHAPE, context=400, **BATCH.get(key, {})) | kw)
+        return path
+    return get
+
+
+def _check_row(g, b, row, idx, val, token, pos, where):
+    g.decode(token, pos, top_k=2)
+    want, got = g.logits(), b.logits(row)
+    assert _rel(got, want) <= TOL, where
+    index, value = oracle.argmax(got)   # the row's own greedy token
+    assert idx[row] == index and val[row] == np.float32(value), where
+
+
+@pytest.mark.parametrize("key,n", [("k20", n) for n in (1, 8, 9, 16, 17, 32, 33, 64)] + [("k24", 7), ("k24", 16)] +
+                         [("k36", n) for n in (9, 17, 33, 64)] +
+                         [(k, n) for k in ("k41", "k41w", "hd40", "hd36") for n in (5, 64)])
+def test_batch_rows_match_decode(ctx, batch_model, key, n):
+    """Every row of a step of n sequences, a third of them two positions ahead, against the sequence decoded alone."""
+    path = batch_model(key)
+    vocab = BATCH[key]["vocab"]
+    g = vrt.Gemma3(ctx, path)
+    b = vrt.Gemma3Batch(g, n, 16)
+    try:
+        print(f"[rowbatch] {key}: {n} sequences", flush=True)
+        ids = synth.uniform_ids(60 + n, 4 * n, 2, vocab).reshape(n, 4).astype(int)
+        ahead = [i for i in range(n) if i % 3 == 0]
+        for t in (0, 1):
+            b.step(ahead, [ids[i][t] for i in ahead])
+        order = list(range(n))[::-1]   # rows are not the sequences' numbers
+        at = [2 if i in ahead else 0 for i in range(n)]
+        for _ in range(2):
+            idx, val = b.step(order, [ids[i][at[i]] for i in order])
+            at = [a + 1 for a in at]
+        for row, i in enumerate(order):
+            g.reset()
+            if at[i] > 1:
+                g.forced(ids[i][:at[i] - 1].astype(np.uint32), 0)
+            _check_row(g, b, row, idx, val, int(ids[i][at[i] - 1]), at[i] - 1, f"row {row}")
+    finally:
+        b.close()
+        g.close()

@@ -294,8 +294,10 @@ __global__ void __launch_bounds__(128 * NWN) k_pf_gemm_q8(PfGemm G) {
     const uint32_t nsteps = (kb_hi - kb_lo + 1u) / 2u;
     const uint64_t row_bytes = static_cast<uint64_t>(nkb) * 34u;
 
-    // One K step in registers: A units u = 2t, 2t + 1 of hi and of lo (row u / 8, k 8 (u % 8)
-    // .. + 7 of the step), and the 34-byte W block of thread t < 2 BN (row t / 2, block t % 2).
+    // One K step in registers: A units u = t + NT j of hi and of lo, in the order of the activation buffer (16-row
+    // tile u / 128, block u / 64 % 2, k octet u / 16 % 4, row u % 16), so that a wave's load is one contiguous
+    // 1 KB, and the 34-byte W block of thread t < 2 BN (row t / 2, block t % 2). (Units along a row touch 16
+    // lines per load of eight rows: a step of 8 sequences at head_dim 40, six blocks, 360 us against 313.)
     struct Stage {
         v4u a[2][AU];  // [hi, lo][unit]
         uint32_t d[8]; // dwords at the block start rounded down to 4 bytes
@@ -333,7 +335,7 @@ __global__ void __launch_bounds__(128 * NWN) k_pf_gemm_q8(PfGemm G) {
         const uint32_t kb = kb_lo + 2u * step;
 #pragma unroll
         for (uint32_t j = 0; j < AU; ++j) {
-            const uint32_t u = AU * tid + j, r = u >> 3, c = u & 7u;
+            const uint32_t u = tid + NT * j, r = 16u * (u >> 7) + (u & 15u), c = (u >> 4) & 7u;
             const uint32_t k = 32u * kb + 8u * c;
             const uint32_t rr = min(m0 + r, G.M - 1u), kk = min(k, 32u * kb_hi - 8u);
             const uintptr_t o = reinterpret_cast<uintptr_t>(G.a + gm_off(rr, kk, nkb));
@@ -357,7 +359,7 @@ __global__ void __launch_bounds__(128 * NWN) k_pf_gemm_q8(PfGemm G) {
         const uint32_t kb = kb_lo + 2u * step;
 #pragma unroll
         for (uint32_t j = 0; j < AU; ++j) {
-            const uint32_t u = AU * tid + j, r = u >> 3, c = u & 7u;
+            const uint32_t u = tid + NT * j, r = 16u * (u >> 7) + (u & 15u), c = (u >> 4) & 7u;
             const bool live = m0 + r < G.M && 32u * kb + 8u * c < 32u * kb_hi;
 #pragma unroll
             for (uint32_t p = 0; p < 2; ++p)
