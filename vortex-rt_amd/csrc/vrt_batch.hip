@@ -250,7 +250,7 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn(BdAttn A) {
 // in the sum. The launch is one memory latency, not bandwidth: staged through LDS, with one wave's softmax over
 // shuffles, it took 8.9 us at 8 rows.
 constexpr uint32_t kBdShort = 256;   // four passes; longer histories gain from more workgroups than (heads, rows)
-template <int NU>
+template <int NU, bool WHOLE>   // WHOLE: hd % 8 == 0, no run of four straddles the RoPE halves
 __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
 #pragma clang fp contract(off)
     constexpr uint32_t NW = kBdThreads / 64u;
@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
     const uint32_t n_hist = min(p + 1u, A.slots), t_first = p + 1u - n_hist;
     const uint64_t cache0 = static_cast<uint64_t>(sqn) * A.slots * hd;
     const uint32_t i = min(4u * lane, hd - 4u);   // lanes past hd hold copies and count nothing
-    const bool live = 4u * lane < hd, lower = i < half;
+    const bool live = 4u * lane < hd;
     f4 kr[NU], vr[NU];
     auto load = [&](uint32_t t0) {   // clamped, in-bounds positions
 #pragma unroll
@@ -276,9 +276,31 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
         }
     };
     load(t_first);
-    const uint32_t ri = lower ? i : i - half;
-    const f4 cs = *reinterpret_cast<const f4*>(A.cos_t + static_cast<uint64_t>(p) * half + ri);
-    const f4 sn = *reinterpret_cast<const f4*>(A.sin_t + static_cast<uint64_t>(p) * half + ri);
+    bool lower[4];          // each dim's RoPE half, and the lane that holds its partner (element e, or without
+    uint32_t partner[4];    // WHOLE, where half is 2 mod 4, e + 2 mod 4)
+#pragma unroll
+    for (uint32_t e = 0; e < 4u; ++e) {
+        const uint32_t j = WHOLE ? i : i + e;
+        lower[e] = j < half;
+        partner[e] = ((lower[e] ? j + half : j - half) >> 2) & 63u;
+    }
+    f4 cs, sn;
+    {
+        const float* ct = A.cos_t + static_cast<uint64_t>(p) * half;
+        const float* st = A.sin_t + static_cast<uint64_t>(p) * half;
+        if constexpr (WHOLE) {
+            const uint32_t ri = lower[0] ? i : i - half;
+            cs = *reinterpret_cast<const f4*>(ct + ri);
+            sn = *reinterpret_cast<const f4*>(st + ri);
+        } else {
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) {
+                const uint32_t ri = lower[e] ? i + e : i + e - half;
+                cs[e] = ct[ri];
+                sn[e] = st[ri];
+            }
+        }
+    }
     f4 x[2], v;   // q of the head, k of the row
     {
         const f4 wq = *reinterpret_cast<const f4*>(A.q_norm + i), wk = *reinterpret_cast<const f4*>(A.k_norm + i);
@@ -300,14 +322,16 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
         for (int k = 0; k < 2; ++k)
 #pragma unroll
             for (int e = 0; e < 4; ++e) ss[k] += live ? static_cast<double>(x[k][e]) * static_cast<double>(x[k][e]) : 0.0;
-        const uint32_t partner = (lower ? lane + (hd >> 3) : lane - (hd >> 3)) & 63u;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const float sc = 1.0f / sqrtf(static_cast<float>(wave_red_sum_d(ss[k]) / static_cast<double>(hd)) + A.eps);   // :1087-1093
+            f4 a;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = x[k][e] * (sc * (k ? wk[e] : wq[e]));
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float a = x[k][e] * (sc * (k ? wk[e] : wq[e])), c = __shfl(a, static_cast<int>(partner));
-                x[k][e] = lower ? a * cs[e] - c * sn[e] : a * cs[e] + c * sn[e];
+                const float c = __shfl(a[WHOLE ? e : (e + 2) & 3], static_cast<int>(partner[e]));
+                x[k][e] = lower[e] ? a[e] * cs[e] - c * sn[e] : a[e] * cs[e] + c * sn[e];
             }
         }
     }
@@ -712,9 +736,12 @@ static int bd_enqueue(vrt_g3_batch* B, uint32_t n, hipStream_t s) {
             void* args[] = {&A};
             uint32_t nh_max = 0;   // longest history of the step's rows in this block
             for (uint32_t i = 0; i < n; ++i) nh_max = std::max(nh_max, std::min(B->host_rows.v[1][i] + 1u, BL.slots));
-            if (nh_max <= kBdShort && hd % 8u == 0u) {   // whole runs of four on both sides of a RoPE pair
-                const void* fn = nh_max <= 32u ? reinterpret_cast<const void*>(&k_bd_attn_short<8>)
-                                               : reinterpret_cast<const void*>(&k_bd_attn_short<16>);
+            if (nh_max <= kBdShort) {   // hd is a multiple of four: H hd is one of 32, and H at most 8
+                const void* fn = hd % 8u == 0u
+                                     ? (nh_max <= 32u ? reinterpret_cast<const void*>(&k_bd_attn_short<8, true>)
+                                                      : reinterpret_cast<const void*>(&k_bd_attn_short<16, true>))
+                                     : (nh_max <= 32u ? reinterpret_cast<const void*>(&k_bd_attn_short<8, false>)
+                                                      : reinterpret_cast<const void*>(&k_bd_attn_short<16, false>));
                 VRT_HIP_CHECK(hipLaunchKernel(fn, dim3(H, n), dim3(kBdThreads), args, 0, s));
             } else {
                 const size_t lds = static_cast<size_t>((H + 2u) * hd + H * BL.cmax) * 4u;
