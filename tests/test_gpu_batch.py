@@ -6,7 +6,7 @@ with the oracle's own tokens (teacher forcing) and every greedy token must be id
 oracle's, as on the single-sequence path. (The oracle's smallest top-2 margin over these rows is
 7.1e-4 of the top logit in the tiny-model cases and 2.9e-3 at the full shape; each row's margin
 is printed with the failure.) Sequences join at different steps, so every step mixes rows at
-different positions, local windows and chunk counts."""
+different positions and local windows."""
 import os
 
 import numpy as np
@@ -77,8 +77,7 @@ def _drive(b, runs, starts, check_logits_every=1):
 
 def test_batch_tiny_staggered(ctx, tiny_model):
     """Six sequences of the 6-block model (window 8, one global block): prompts of 1..9 tokens
-    joining at steps 0..11, 14 new tokens each; histories pass the window and a 64-position
-    chunk boundary of the global block."""
+    joining at steps 0..11, 14 new tokens each; histories pass the window."""
     prompts = [synth.uniform_ids(200 + i, 1 + (i * 3) % 9, 2, 1000) for i in range(6)]
     runs = _oracle_runs(tiny_model, prompts, 14)
     g = vrt.Gemma3(ctx, tiny_model)
@@ -92,7 +91,8 @@ def test_batch_tiny_staggered(ctx, tiny_model):
 
 
 def test_batch_tiny_long_history(ctx, tiny_model):
-    """Two sequences past 130 positions: the global block's history spans three chunks."""
+    """Two sequences past 130 positions: the global block's history takes three passes of the short
+    attention. (Past 256 positions, with the chunked kernels: test_gpu_rowbatch.py.)"""
     prompts = [synth.uniform_ids(301, 5, 2, 1000), synth.uniform_ids(302, 70, 2, 1000)]
     runs = _oracle_runs(tiny_model, prompts, 70)
     g = vrt.Gemma3(ctx, tiny_model)

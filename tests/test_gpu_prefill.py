@@ -74,9 +74,9 @@ LONG = dict(n_layers=6, d_model=256, n_heads=2, head_dim=64, ffn=512, vocab=1000
 
 @pytest.mark.parametrize("kv_f16", [False, True])
 def test_prefill_segments(ctx, model_dir, kv_f16):
-    """A prompt longer than the batched workspace (2048 positions) runs as segments of 2048,
-    2048 and 404 positions: a segment's global blocks attend to every earlier position through
-    the KV cache and its local blocks to the window's start rounded down to 32."""
+    """A prompt of 4500 positions, one segment of the batched workspace (8192): the global block's
+    key ranges are cut into chunks, the local blocks see their last 64 positions. (A second segment,
+    past 8192 positions: test_gpu_rowbatch.py.)"""
     path = os.path.join(str(model_dir), "long8k.gguf")
     if not os.path.exists(path):
         synth.write_gemma3_gguf(path, seed=23, **LONG)
@@ -88,12 +88,11 @@ LC_MODEL = dict(synth.GEMMA3_270M, n_layers=6, vocab=4096, context=8448)
 
 def test_prefill_segments_long_context_golden(ctx, model_dir):
     """An 8192-token prompt at the Gemma-3-270M block shape (6 blocks, window 512, block 5
-    global; head_dim 256) prefilled in four segments of 2048, then 16 teacher-forced decode steps
+    global; head_dim 256) prefilled in one full segment, then 16 teacher-forced decode steps
     against the oracle's vectors in tests/golden/long_context_6blk.npz (tests/golden/
     make_long_context.py, the long-context decode test's fixture): greedy ids identical, their
     logits within the tolerance, the last step's logits and hidden state within the tolerances.
-    The segments' global attention reads up to 6144 earlier positions from the cache, the local
-    blocks' their last 512."""
+    The global block's attention runs over up to 8192 keys, the local blocks' over their last 512."""
     gold = np.load(os.path.join(os.path.dirname(__file__), "golden", "long_context_6blk.npz"))
     path = os.path.join(str(model_dir), "lc6.gguf")
     if not os.path.exists(path):
@@ -103,7 +102,7 @@ def test_prefill_segments_long_context_golden(ctx, model_dir):
     scale = np.max(np.abs(gold["last_logits"]))
     g = vrt.Gemma3(ctx, path)
     try:
-        print("[pf] 8192-token prefill in segments at the 270M block shape", flush=True)
+        print("[pf] 8192-token prefill at the 270M block shape", flush=True)
         g.prefill(toks[:8192], top_k=0)
         hid = None
         for j in range(n_check):

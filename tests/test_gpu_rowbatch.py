@@ -298,3 +298,60 @@ def test_batch_rows_match_decode(ctx, batch_model, key, n):
     finally:
         b.close()
         g.close()
+
+
+# Six blocks (the last global), window 64.
+LONG = dict(n_layers=6, window=64, ffn=256, vocab=1003)
+BATCH.update(long64=dict(LONG, d_model=128, n_heads=2, head_dim=64), long36=dict(LONG, d_model=288, n_heads=8, head_dim=36),
+             long256=dict(LONG, d_model=320, n_heads=1, head_dim=256))
+
+
+@pytest.mark.parametrize("key", ("long64", "long36", "long256"))
+def test_batch_passes_256_positions(ctx, batch_model, key):
+    """Three sequences, one of them past 256 positions in the global block, where a step goes from the short
+    attention to the chunked kernels and their merge: every row from position 250 to 262 of the longest, with
+    rows of few positions in the same steps, against the sequences decoded alone; then the long one leaves
+    and the others go back to the short kernel."""
+    path = batch_model(key)
+    g = vrt.Gemma3(ctx, path)
+    b = vrt.Gemma3Batch(g, 3, 300)
+    try:
+        print(f"[rowbatch] {key}: past 256 positions", flush=True)
+        n = (262, 40, 11)
+        ids = [synth.uniform_ids(80 + i, 264, 2, 1003) for i in range(3)]
+        results = {}   # (sequence, position) -> token, value, logits
+        at = [0, 0, 0]
+
+        def step(rows):
+            idx, val = b.step(rows, [int(ids[i][at[i]]) for i in rows])
+            for r, i in enumerate(rows):
+                if i or at[i] >= 250:
+                    results[i, at[i]] = idx[r], val[r], b.logits(r)
+                at[i] += 1
+        while at[0] < n[0]:   # the shorter ones join so that they end with the long one
+            step([i for i in range(3) if at[0] >= n[0] - n[i] or i == 0])
+        for _ in range(2):
+            step([2, 1])
+        for i in range(3):
+            first = min(p for j, p in results if j == i)
+            g.reset()
+            if first:
+                g.forced(ids[i][:first], 0)
+            for p in range(first, at[i]):
+                g.decode(int(ids[i][p]), p, top_k=2)
+                want, (idx, val, got) = g.logits(), results[i, p]
+                assert _rel(got, want) <= TOL, f"sequence {i} position {p}"
+                assert (idx, val) == oracle.argmax(got), f"sequence {i} position {p}"
+    finally:
+        b.close()
+        g.close()
+
+
+@pytest.mark.parametrize("kv,tol", (("f32", 1e-5), ("f16", 4e-4), ("bf16", 2e-3)))
+@pytest.mark.parametrize("rows", (8193, 8700))
+def test_second_segment_with_a_global_block(ctx, batch_model, kv, tol, rows):
+    """Prompts past the 8192 positions of one segment, of six blocks: the second segment's global block attends to all
+    of the first through the cache (a history of 8192 keys, cut into chunks with the segment's own), its local ones
+    to the window's start. Tolerances as above, the fp32 one for three times the blocks."""
+    path = batch_model("segments", **dict(LONG, d_model=256, n_heads=2, head_dim=64, context=8800))
+    _compare(ctx, path, rows, tol, kv)
