@@ -84,6 +84,18 @@ def _span(buf, offset, nbytes):
 def test_codec_runs_and_alignments(ctx, blocks, x_off, q_off):
     """Runs of 128 blocks and what is left of them, on arrays that are 16-byte aligned and not: the bytes and
     values of the oracle, and nothing written past the end."""
+    _codec(ctx, blocks, x_off, q_off)
+
+
+@pytest.mark.parametrize("blocks", (20479, 20480, 20481, 20487, 20607, 20609))
+@pytest.mark.parametrize("x_off,q_off", ((0, 0), (16, 32), (4, 0), (0, 2)))
+def test_codec_many_blocks(ctx, blocks, x_off, q_off):
+    """Both sides of the number of blocks from which aligned arrays pass through LDS, 128 to a workgroup, with last
+    runs of 1, 7, 127 and 128 blocks."""
+    _codec(ctx, blocks, x_off, q_off)
+
+
+def _codec(ctx, blocks, x_off, q_off):
     x = synth.normal_f32(33 + blocks, 32 * blocks + blocks % 2, 0.7)[:32 * blocks]
     x[:32] = 0.0   # an all-zero block
     nq = 34 * blocks
