@@ -249,7 +249,10 @@ __global__ void __launch_bounds__(kBdThreads) k_bd_attn(BdAttn A) {
 // of a slot past it is the row being written, which may still hold a failed step's NaN, and 0 x NaN would be
 // in the sum. The launch is one memory latency, not bandwidth: staged through LDS, with one wave's softmax over
 // shuffles, it took 8.9 us at 8 rows.
-constexpr uint32_t kBdShort = 256;   // four passes; longer histories gain from more workgroups than (heads, rows)
+// Four passes; longer histories gain from more workgroups than (heads, rows). A step of six blocks at 4 heads of 256, all
+// rows in the range: here at 192 to 255 positions, chunked at 257 to 400, 1 row 309 and 311 us, 8 rows 314 and 325, 64
+// rows 446 and 580.
+constexpr uint32_t kBdShort = 256;
 template <int NU, bool WHOLE>   // WHOLE: hd % 8 == 0, no run of four straddles the RoPE halves
 __global__ void __launch_bounds__(kBdThreads) k_bd_attn_short(BdAttn A) {
 #pragma clang fp contract(off)

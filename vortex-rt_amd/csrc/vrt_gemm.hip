@@ -430,13 +430,16 @@ __global__ void __launch_bounds__(256) k_gm_norm_rows(GmArgs G, GmNorm R) {
 // Logits of M rows against Q8_0 rows in their file layout (the tied embedding table), with each
 // workgroup's greedy candidate per row. The table is streamed once per 16 GM rows (178 MB at the 270M shape),
 // so its time is the floor, and what counts is bytes in flight. Tiles of 16 table rows, contiguous in the file,
-// come in whole 1 KB direct-to-LDS loads, R - 1 tiles ahead, two workgroups per CU. The four waves share out the K
-// blocks (wave w: w, w + 4, ...); a wave keeps its blocks' activations of all GM row tiles in registers, takes its
-// blocks of the raw tile (lane l: quants k = 8 (l / 16) .. + 7 of row l % 16) and turns them into the MFMA's
-// second operand in ten instructions (0x6400 | (q ^ 0x80) is the f16 1152 + q), once for all row tiles. The waves'
-// partial tiles are added through LDS one pass later; one barrier per tile. Result r of lane l is logit
-// [m = 4 (l / 16) + r][n = l % 16]; two tiles' logits leave together, 128 bytes per row and store. At 8 / 64
-// rows 45 / 88 us; before: the K loop of a 128-column GEMM and an argmax over its logits 109 + 5 / 130 + 25; operands
+// come in whole 1 KB direct-to-LDS loads, R - 1 tiles ahead (gm_wait counts up to 12 loads per wave: three tiles
+// from 23 K blocks on, two from 31). At 20 K blocks one or four row tiles leave LDS for two workgroups per CU (74 and
+// 76 KB each); two row tiles, with their deeper ring, for one (82 KB), and so do all from 23 K blocks on. The four
+// waves share out the K blocks (wave w: w, w + 4, ...); a wave keeps its blocks' activations of all GM row tiles in
+// registers, takes its blocks of the raw tile (lane l: quants k = 8 (l / 16) .. + 7 of row l % 16) and turns them
+// into the MFMA's second operand in ten instructions (0x6400 | (q ^ 0x80) is the f16 1152 + q), once for all row
+// tiles. The waves' partial tiles are added through LDS one pass later; one barrier per tile. Result r of lane l is
+// logit [m = 4 (l / 16) + r][n = l % 16]; two tiles' logits leave together, 128 bytes per row and store. At 8 / 32 /
+// 64 rows 48 / 92 / 88 us; before: the K loop of a 128-column GEMM and an argmax over its logits 109 + 5 at 8 rows,
+// 130 + 25 at 64. Other forms, at 8 / 64 rows where this one then took 45 / 88: operands
 // from memory straight to registers 68 / 152 (16 rows of addresses per load); one conversion per
 // workgroup shared through LDS 85 (a second dependent LDS pass behind every barrier); row tiles dealt to the
 // waves, each converting every block, 126 at 64. The table bypasses the caches as far as it can, so the blocks'
@@ -732,7 +735,8 @@ int gm_expand(const uint8_t* w0, const uint8_t* w1, const uint8_t* w2, uint32_t 
     return VRT_OK;
 }
 
-// One row tile and up to 24 K blocks (five or six per wave). With more rows a wave norms several in turn and
+// One row tile and up to 24 K blocks (five or six per wave, their weights in registers before the norm; wider models
+// keep the two launches). With more rows a wave norms several in turn and
 // the launch that is saved costs more than it took (32 rows per workgroup: 13.8 us against 4.5 + 4.5).
 bool gm_norm_fits(uint32_t M, uint32_t nkb) { return M <= 16u && nkb <= 24u; }
 
@@ -781,7 +785,8 @@ bool gm_lm_fits(const uint8_t* table, uint64_t readable, uint32_t V, uint32_t nk
            nkb <= 40u;
 }
 
-// Two workgroups per CU in all: 512 chunks of one row group, 256 of two.
+// 512 workgroups in all, two for each CU: 512 chunks of one row group, 256 of two. Where LDS holds one per CU (k_gm_lm)
+// they run as two rounds.
 uint32_t gm_lm_chunks(uint32_t M, uint32_t nkb) { return M <= 16u * gm_lm_tiles(M, nkb) ? kGmLmMaxChunks : kGmLmMaxChunks / 2u; }
 
 int gm_lm(const uint8_t* table, uint32_t V, uint32_t nkb, const _Float16* x, uint32_t M, float* logits, GmBest* best,

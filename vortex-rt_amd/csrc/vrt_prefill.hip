@@ -31,7 +31,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kPfThreads = 256;
-constexpr uint32_t kPfMaxSplits = 4;   // K splits of the O and down projections (pf_splits)
+constexpr uint32_t kPfMaxSplits = 4;   // K splits of a projection, at most (gm_splits, pf_splits_q8)
 constexpr uint64_t kPfExpandBudget = 16ull << 30;   // device bytes for the prefill's expanded weights
 constexpr uint32_t kPfTile = 64;     // attention score rows are padded to a multiple of this
 
@@ -688,10 +688,15 @@ __host__ __device__ __forceinline__ void pf_att_group(const PfAttn& A, uint32_t 
 }
 
 // O^T tiles times alpha, in the accumulation registers they live in: as plain code the multiplication
-// would move all of them to VGPRs and back in every tile, taken or not. The leading waits cover an
-// MFMA's last write, the trailing one the next MFMA's read.
+// would move all of them to VGPRs and back in every tile, taken or not. The compiler does not see the
+// accesses inside the assembly, so the waits are here: the leading ones cover an MFMA's last write, the trailing
+// one the next MFMA's read. The empty statements on every tile tie them down: volatile statements keep
+// their order, no product that writes a tile can follow the first row of them, and none that reads one can
+// precede the last.
 template <uint32_t DT>
 __device__ __forceinline__ void att_rescale(float16v (&o)[DT], float alpha) {
+#pragma unroll
+    for (uint32_t j = 0; j < DT; ++j) asm volatile("" : "+a"(o[j]));
     asm volatile("s_nop 15\n\ts_nop 7");
 #pragma unroll
     for (uint32_t j = 0; j < DT; ++j)
@@ -704,6 +709,8 @@ __device__ __forceinline__ void att_rescale(float16v (&o)[DT], float alpha) {
             o[j][r] = x;
         }
     asm volatile("s_nop 7");
+#pragma unroll
+    for (uint32_t j = 0; j < DT; ++j) asm volatile("" : "+a"(o[j]));
 }
 
 template <uint32_t HD, bool LO>
@@ -997,7 +1004,9 @@ __global__ void __launch_bounds__(256, 1) k_pf_attn(PfAttn A) {
 // w + 4, ... of S^T and the d tiles w, w + 4, ... of O^T). The operands come straight to registers, the
 // next tile's during the current one; each wave's partial S^T goes through LDS and every wave adds the
 // four in wave order (the same scores in every wave), one barrier per tile. Softmax, results and
-// partials as in k_pf_attn. 37 rows: 11.5 -> 8.3 us.
+// partials as in k_pf_attn. 37 rows: 11.5 -> 8.3 us. Up to kPfAttFew pairs; a prefill
+// of six blocks, 4 heads of 256, with this kernel and with k_pf_attn: 8 pairs 318 and 333 us, 16 pairs 361 and 381,
+// 24 pairs 409 and 404, 32 pairs 422 and 417 (processes differ by 1%), 64 pairs 497 and 490.
 template <uint32_t HD, bool LO>
 __global__ void __launch_bounds__(256) k_pf_attn_few(PfAttn A) {
 #pragma clang fp contract(off)

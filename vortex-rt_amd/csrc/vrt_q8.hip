@@ -200,7 +200,8 @@ int launch_matvec(hipStream_t stream, const uint8_t* const* bases, const uint32_
     const uint64_t row_bytes = static_cast<uint64_t>(K / 32u) * 34u;
     // Many rows of 17 to 20 blocks: slots of 4 lanes x 5 blocks keep 85 to 100% of the lanes on a block, where one
     // block on each of 32 lanes keeps 53 to 62% (262144 x 640: 50 -> 38 us). Fewer rows than fill the chip
-    // that way are better spread thin.
+    // that way are better spread thin. Other block counts between powers of two idle as many lanes and keep the
+    // plain slots; no such variant was measured.
     if (sh.S == 32 && K / 32u <= 20u && total >= 32768u && even) return launch_mv_t<4, 5, 1>(stream, rs, row_bytes, K, w_end, x, y);
     switch (sh.S * 16 + sh.NB) {
     case 1 * 16 + 1: return launch_mv_t<1, 1, 2>(stream, rs, row_bytes, K, w_end, x, y);
