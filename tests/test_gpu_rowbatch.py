@@ -367,3 +367,40 @@ def test_second_segment_with_a_global_block(ctx, batch_model, kv, tol, rows):
     to the window's start. Tolerances as above, the fp32 one for three times the blocks."""
     path = batch_model("segments", **dict(LONG, d_model=256, n_heads=2, head_dim=64, context=8800))
     _compare(ctx, path, rows, tol, kv)
+
+
+def test_batch_table_not_on_16_bytes(ctx, batch_model, monkeypatch):
+    """A tensor section that starts four bytes past a 16-byte unit: k_gm_lm's direct loads do not fit, so the LM head is
+    the general GEMM and argmax, and the tokens are those of the aligned section."""
+    path, n = batch_model("k20"), 5
+    ids = synth.uniform_ids(90, 3 * n, 2, 26003).reshape(3, n)
+
+    def run():
+        g = vrt.Gemma3(ctx, path)
+        b = vrt.Gemma3Batch(g, n, 16)
+        try:
+            out = [b.step(range(n), t) for t in ids]
+            return g.arena.ptr, out, [b.logits(r) for r in range(n)]
+        finally:
+            b.close()
+            g.close()
+    at, want, logits = run()
+    assert at % 16 == 0
+
+    class Shifted(vrt.DeviceBuffer):
+        def __init__(self, ctx, nbytes):
+            super().__init__(ctx, nbytes + 64)
+            self.ptr += 4
+
+        def free(self):
+            if getattr(self, "ptr", None):
+                self.ptr -= 4
+            super().free()
+    monkeypatch.setattr(vrt, "DeviceBuffer", Shifted)
+    at, got, logits4 = run()
+    assert at % 16 == 4
+    for (i, v), (j, w), in zip(got, want):
+        np.testing.assert_array_equal(i, j)
+        assert np.max(np.abs(v - w)) <= TOL * np.max(np.abs(w))
+    for a, b in zip(logits4, logits):
+        assert _rel(a, b) <= TOL

@@ -667,7 +667,7 @@ static bool gm_use_rows(uint32_t M, uint32_t N, uint32_t nkb) {
 // Tile of k_gm_tile. 64 x 128 from two workgroups per CU on (below, 64 x 64: q|k|v at 2048 rows 15.7 against
 // 16.7 us, gate/up at 512 rows 11.2 against 12.9, O at 4096 rows 20.9 against 22.8; above, O at 8192 rows 35.0
 // against 31.3); 128 x 128 with the GELU epilogue, which it amortises (gate/up at 2048 rows 29.9 -> 27.6;
-// q|k|v at 8192 rows 43.9 -> 47.1, not taken). Few 64 x 64 tiles split K in up to four (down at 512 rows
+// q|k|v at 8192 rows 43.9 -> 47.1 on that card, not taken). Few 64 x 64 tiles split K in up to four (down at 512 rows
 // 21.4 -> 9.6).
 struct GmTile {
     uint32_t mt, nt, splits;
